@@ -64,8 +64,13 @@ enum Mode : int32_t {
     MODE_COUNT = 4
 };
 
-constexpr int RB_DEFAULT[MODE_COUNT] = {128, 16, 16, 128};
-constexpr int64_t SMALL_BATCH_ITEMS = 512;  // rect items aimed at when rows are not tuned
+// Rows per work item when not tuned.  rect_fast: 192 (1024 templates of 250 to
+// 2000 rows and columns: maps 1880 us; 128 rows 1955, 256 rows 1915).
+constexpr int RB_DEFAULT[MODE_COUNT] = {192, 16, 16, 128};
+// Rect items aimed at when rows are not tuned: eight a CU, since five fit a CU
+// at a time (256 templates of 48 x 48 to 240 x 240: maps 22 us, 26 at 1024
+// items, 29 at 512; 1024 templates of 125 x 125: 35 us, 37 at 1024, 38 at 4096).
+constexpr int64_t SMALL_BATCH_ITEMS = 2048;
 constexpr int EXP_SMALL_BATCH_ROWS = 64;    // exp rows when untuned and under 256 column blocks
 
 struct TmplDev {
@@ -90,6 +95,13 @@ struct TmplDev {
     int64_t etab_off;            // MODE_EXP_FAST: doubles, [n_seg + INIT_PARTS][7][N_tau]
     uint32_t o_t0, o_t0Band, o_tau, o_tauBand;  // caller's window (posterior modes)
 };
+
+// Per-template flags: set by the stage kernels, FLAG_SINGLE_ATOM raised by the
+// strict map kernels.
+constexpr int FLAG_SINGLE_ATOM = 1;  // a window spans a single atom
+// a merged bin has a negative or NaN a^2 or b^2, or a non-finite ab: window
+// traces need not grow with the window, nor determinants be numbers
+constexpr int FLAG_NO_BOUND = 2;
 
 struct SegDev {
     int64_t begin, end;
@@ -142,10 +154,13 @@ __global__ __launch_bounds__(SR_WG) void stage_kernel(
     const TmplDev *__restrict__ tds, const SegDev *__restrict__ segs,
     const uint32_t *__restrict__ ts, const float *__restrict__ cols, int64_t cstride,
     double *__restrict__ prefix, int *__restrict__ flags) {
-    // one block per template, before any map kernel: clear its single-atom flag
-    if (threadIdx.x == 0) flags[blockIdx.x] = 0;
+    // one block per template, before any map kernel: set its flags (exp
+    // templates: none)
     const TmplDev td = tds[blockIdx.x];
-    if (td.mode != MODE_RECT_FAST && td.mode != MODE_RECT_GENERIC) return;  // block-uniform
+    if (td.mode != MODE_RECT_FAST && td.mode != MODE_RECT_GENERIC) {  // block-uniform
+        if (threadIdx.x == 0) flags[blockIdx.x] = 0;
+        return;
+    }
     // staging: ts [SR_CHUNK] uint32, then NC float planes [SR_CHUNK];
     // output: per wave SR_PASS_BINS x NC doubles
     __shared__ double s_buf[SR_CHUNK * (NC + 1) / 2];
@@ -155,6 +170,8 @@ __global__ __launch_bounds__(SR_WG) void stage_kernel(
     __shared__ double s_off[NC][SR_WG / 64];  // wave totals, then wave offsets
     __shared__ double s_carry[NC];            // sum of all earlier rounds
     __shared__ int64_t s_ka;
+    __shared__ int s_flag;
+    if (threadIdx.x == 0) s_flag = 0;  // a barrier follows in the first round
 
     const uint32_t N = td.N;
     const uint64_t TA = td.TAtom;
@@ -228,6 +245,11 @@ __global__ __launch_bounds__(SR_WG) void stage_kernel(
             }
             if (tid == X) cur = next;
         }
+        bool odd = false;  // what FLAG_NO_BOUND is for (NaN compares false)
+#pragma unroll
+        for (int j = 0; j < SR_BINS; j++)
+            odd |= !(v[j][0] >= 0.0f) | !(v[j][1] >= 0.0f) | !(fabsf(v[j][2]) < INFINITY);
+        if (odd) s_flag = FLAG_NO_BOUND;
         // inclusive scan of the thread totals within the wave (bins >= N hold 0)
         double x[NC];
 #pragma unroll
@@ -290,6 +312,7 @@ __global__ __launch_bounds__(SR_WG) void stage_kernel(
         }
     }
     if (tid < NC) P[(int64_t)N * NC + tid] = s_carry[tid];
+    if (tid == 0) flags[blockIdx.x] = s_flag;
 }
 
 // Bins of a template's atom table: the recurrence path reads none at or
@@ -451,23 +474,37 @@ __global__ __launch_bounds__(256) void stage_exp_kernel(
 // F from window sums: determinant, numerator and condition guard in FP64
 // (rect.cu:98-118 / exp.cu:109-129; F = 2 when the guard fails); the final
 // quotient in float32 (the stored map is float32).
-__device__ __forceinline__ float cell_F(double A, double B, double C, double far,
-                                        double fai, double fbr, double fbi) {
-    const double D = fma(A, B, -(C * C));
-    const double T = A + B;
+__device__ __forceinline__ double cell_D(double A, double B, double C) {
+    return fma(A, B, -(C * C));
+}
+
+// The quotient, whatever the condition number; Df is the determinant as float.
+// The map is float32: the quotient of the FP64 numerator and determinant
+// (each rounded to float) through v_rcp_f32 is within ~3e-7 relative, and
+// v_rcp_f64 issues at ~1/3.5 the rate of an FP64 FMA.
+__device__ __forceinline__ float cell_quot(double A, double B, double C, double far, double fai,
+                                           double fbr, double fbi, float &Df) {
     const double p = fma(far, far, fai * fai);
     const double q = fma(fbr, fbr, fbi * fbi);
     const double r = fma(far, fbr, fai * fbi);
     const double num = fma(B, p, fma(A, q, (-2.0 * C) * r));
-    // the map is float32: the quotient of the FP64 numerator and determinant
-    // (each rounded to float) through v_rcp_f32 is within ~3e-7 relative, and
-    // v_rcp_f64 issues at ~1/3.5 the rate of an FP64 FMA.  The condition test
-    // is FP64 (two multiplies and a compare: one conversion fewer than on
-    // float T and D).  A, B >= 0 (sums of squares), so T <= 0 only for an
-    // empty window, where D = 0 and the test fails as well.
-    const bool ok = T * T < QCOND * D;
-    const float F = (float)num * __builtin_amdgcn_rcpf((float)D);
-    return ok ? F : 2.0f;
+    Df = (float)cell_D(A, B, C);
+    return (float)num * __builtin_amdgcn_rcpf(Df);
+}
+
+// The condition test is FP64 (two multiplies and a compare: one conversion
+// fewer than on float T and D).  A, B >= 0 (sums of squares), so T <= 0 only
+// for an empty window, where D = 0 and the test fails as well.
+__device__ __forceinline__ bool cell_ok(double A, double B, double C) {
+    const double T = A + B;
+    return T * T < QCOND * cell_D(A, B, C);
+}
+
+__device__ __forceinline__ float cell_F(double A, double B, double C, double far,
+                                        double fai, double fbr, double fbi) {
+    float Df;
+    const float F = cell_quot(A, B, C, far, fai, fbr, fbi, Df);
+    return cell_ok(A, B, C) ? F : 2.0f;
 }
 
 // uint32 index maths of rect.cu:21-31 (start) and rect.cu:59-69 (end).
@@ -557,13 +594,26 @@ __device__ __forceinline__ void argmax_merge(float &bv, int &bi, float v, int i)
     }
 }
 
+// wave minimum of non-negative integers, the same on every lane
+__device__ __forceinline__ int wave_min_idx(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, DPP_QUAD_XOR1, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, DPP_QUAD_XOR2, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_ROR4, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_ROR8, 0xf, 0xf, false));
+    const auto p = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    v = min((int)p[0], (int)p[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return min((int)q[0], (int)q[1]);
+}
+
+// Wave argmax, the first index on ties: the maximum first, then the smallest
+// index among the lanes that hold it, both by DPP (~30 instructions; pairwise
+// exchanges of value and index through LDS take ~130).  No lane's value is
+// NaN (a running maximum starts from -inf and drops NaN).
 __device__ __forceinline__ void wave_argmax(float &bv, int &bi) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        float ov = __shfl_xor(bv, o);
-        int oi = __shfl_xor(bi, o);
-        argmax_merge(bv, bi, ov, oi);
-    }
+    const float m = wave_max(bv);
+    bi = wave_min_idx(bv == m ? bi : 0x7fffffff);
+    bv = m;
 }
 
 constexpr int MAX_RB = 512;
@@ -599,10 +649,10 @@ __device__ __forceinline__ float rows_sum<4>(const float (&v)[4], int lane, int 
     return rows16_sum(quads_sum(z));
 }
 
-// Per-work-item reduction state.  A lane owns 4 columns; every sub-tile brings
-// R wave-uniform rows x those 4 columns, with invalid cells set to -inf.
-//  - argmax: lane maximum of the sub-tile; only when it beats the lane's best
-//    is the first (row-major) position searched;
+// Per-work-item reduction state.  A lane owns NCOLS columns; every sub-tile
+// brings R wave-uniform rows x those columns, with invalid cells set to -inf.
+//  - argmax (add): lane maximum of the sub-tile; only when it beats the lane's
+//    best is the first (row-major) position searched;
 //  - BtSG: sum of 2^(F*LOG2E - ML), ML = Mw*LOG2E rounded to float, Mw the
 //    wave's running maximum (accumulators rescaled when it grows) -- one FMA
 //    and one exp2 per cell; each sum is relative to its reference in log2
@@ -613,10 +663,6 @@ template <bool BTSG, int NCOLS = 4>
 struct Reducer {
     float best;
     int bidx;
-    // a lower bound of the wave's largest value so far (the wave maximum of
-    // best at the last search): a lane whose block maximum is below it holds
-    // no candidate for the item's first maximum and skips the search
-    float wbest;
     float Mw;
     float ML;
     float Scol[NCOLS];
@@ -624,7 +670,6 @@ struct Reducer {
     __device__ void init() {
         best = -INFINITY;
         bidx = 0x7fffffff;
-        wbest = -INFINITY;
         Mw = -INFINITY;
         ML = -INFINITY;
 #pragma unroll
@@ -639,24 +684,23 @@ struct Reducer {
         return s;
     }
 
-    // F[r][c]: cell values (-inf when invalid); row index m0 + r; colidx[c]
-    // column index of the lane's c-th column; rl0: item-local row of r = 0.
-    template <int R>
-    __device__ void add(const float (&F)[R][NCOLS], int m0, const int (&colidx)[NCOLS], int N_tau,
-                        int lane, int rl0, float *sh_rowM, float *sh_rowS) {
+    template <int R, typename Row>
+    __device__ static float block_max(const Row (&F)[R]) {
         float lm = -INFINITY;
 #pragma unroll
         for (int r = 0; r < R; r++)
 #pragma unroll
             for (int c = 0; c < NCOLS; c++) lm = fmaxf(lm, F[r][c]);
-        // a block holding the item's largest value V always searches (V >=
-        // wbest, V >= best); a block below wbest has a larger value in
-        // another lane of the wave.  Only for 16-cell blocks: for 4 cells the
-        // wave maximum that updates wbest costs more than the search
-        constexpr bool FILTER = R * NCOLS >= 16;
-        const bool search = (!FILTER || lm >= wbest) &&
-                            (lm > best || (lm == best && lm != -INFINITY));
-        if (search) {
+        return lm;
+    }
+
+    // F[r][c]: cell values (-inf when invalid); row index m0 + r; colidx[c]
+    // column index of the lane's c-th column; rl0: item-local row of r = 0.
+    template <int R, typename Row>
+    __device__ void add(const Row (&F)[R], int m0, const int (&colidx)[NCOLS], int N_tau,
+                        int lane, int rl0, float *sh_rowM, float *sh_rowS) {
+        const float lm = block_max(F);
+        if (lm > best || (lm == best && lm != -INFINITY)) {
             // the first cell (row-major) equal to lm: selects from the last
             // cell to the first, no branches (a search with an early exit
             // compiles to a chain of masked branches, one per cell)
@@ -664,13 +708,19 @@ struct Reducer {
 #pragma unroll
             for (int q = R * NCOLS - 1; q >= 0; q--) pos = F[q / NCOLS][q % NCOLS] == lm ? q : pos;
             const int rr = pos / NCOLS, cc = pos % NCOLS;
-            // a lane's columns are evenly spaced (1 or 64 apart): arithmetic,
-            // not a selection the compiler would turn into a private array
+            // a lane's columns are evenly spaced (64 apart): arithmetic, not a
+            // selection the compiler would turn into a private array
             int col = colidx[0];
             if constexpr (NCOLS > 1) col += cc * (colidx[1] - colidx[0]);
             argmax_merge(best, bidx, lm, (m0 + rr) * N_tau + col);
         }
-        if (FILTER && __any(search)) wbest = wave_max(best);
+        sums(F, lm, lane, rl0, sh_rowM, sh_rowS);
+    }
+
+    // the BtSG sums of a sub-tile whose lane maximum is lm
+    template <int R, typename Row>
+    __device__ void sums(const Row (&F)[R], float lm, int lane, int rl0, float *sh_rowM,
+                         float *sh_rowS) {
         if (!BTSG) return;
         // exp(F - Mw) only has to stay finite, so the wave reference Mw is
         // raised (wave maximum, accumulators rescaled) only when some lane
@@ -685,13 +735,17 @@ struct Reducer {
             ML = wmL;
         }
         if (Mw == -INFINITY) return;  // wave-uniform: no valid cell yet
+        // (-ML in a register of its own: a multiply-add of two registers and a
+        // literal issues in ~2.7 cycles, of three registers in 4)
+        float nML = -ML;
+        asm("" : "+v"(nML));
         float sr[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
             sr[r] = 0.0f;
 #pragma unroll
             for (int c = 0; c < NCOLS; c++) {
-                const float e = __builtin_amdgcn_exp2f(fmaf(F[r][c], LOG2E, -ML));
+                const float e = __builtin_amdgcn_exp2f(fmaf(F[r][c], LOG2E, nML));
                 sr[r] = c == 0 ? e : sr[r] + e;
                 Scol[c] += e;
             }
@@ -705,22 +759,29 @@ struct Reducer {
     }
 };
 
-// End of a work item: combine the 4 waves, then write the item partial
+// End of a work item (red.best, red.bidx already the wave's): combine the 4 waves, then write the item partial
 // {max, argmax, M, S} and, for BtSG, the row and column partial sums rescaled
 // to the item reference M (so each is a single float).  M is in log2 units:
 // the partial sums are relative to exp(M / LOG2E).
+struct FinShared {
+    float best[4];
+    int bidx[4];
+    float M[4], S[4];
+    float col[4][TILE_COLS];
+};
+
 template <bool BTSG, int NCOLS, typename ColMap>
 __device__ void finish_item(Reducer<BTSG, NCOLS> &red, int wave, int lane, const TmplDev &td,
                             const ItemDev &it, int64_t item_id, int nrows_item,
                             ItemPart *ipart, float *rowpart, float *colpart,
-                            const float *sh_rowM, const float *sh_rowS, ColMap colmap) {
-    __shared__ float sh_best[4];
-    __shared__ int sh_bidx[4];
-    __shared__ float sh_M[4];
-    __shared__ float sh_S[4];
-    __shared__ float sh_col[4][TILE_COLS];
+                            const float *sh_rowM, const float *sh_rowS, FinShared &fs,
+                            ColMap colmap) {
+    float(&sh_best)[4] = fs.best;
+    int(&sh_bidx)[4] = fs.bidx;
+    float(&sh_M)[4] = fs.M;
+    float(&sh_S)[4] = fs.S;
+    float(&sh_col)[4][TILE_COLS] = fs.col;
 
-    wave_argmax(red.best, red.bidx);
     float stot = 0.0f;
     if (BTSG) stot = wave_sum(red.total());
     if (lane == 0) {
@@ -775,20 +836,93 @@ __device__ void finish_item(Reducer<BTSG, NCOLS> &red, int wave, int lane, const
 //   i(m)   = min(q0 + a*m, N-1)                      (rect.cu:21-31)
 //   j(D)   = min(max(q00 + a*D - 1, 0), N-1) + 1     (rect.cu:54-69), D = m+n,
 // and j >= i always, so the incremental sum of rect.cu:75-91 equals
-// P[j] - P[i].  The item's j(D) range is staged in LDS in groups of 4
-// diagonals, each group's 7 components x 4 diagonals contiguous plus one pad
-// double (LDS_GS doubles: a lane's 4-group stride of 58 words spreads its
-// 8-byte reads over all banks); each lane computes a 4x4 block whose 16
-// cells touch 7 diagonals -- its own group and 3 entries of the next, all at
-// constant offsets from one address -- loading 4 entries for the first row
-// and one more per following row.
-constexpr int LDS_GS = 4 * NC + 1;
+// P[j] - P[i].  A lane computes a 4 x C block of cells (4 rows, C columns),
+// whose cells touch 3 + C diagonals; the item's j(D) range is staged in LDS in
+// groups of C diagonals, each group's 7 components x C diagonals contiguous
+// (padded to an odd number of doubles: the lanes' 8-byte reads then spread
+// over all banks), so that all of a lane's reads are at constant offsets from
+// one address.
+//
+// C is 4 where the item's columns need it (a wave spans 64 C columns), 2 or 1
+// in the last column block of a template and for maps of at most 128 or 64
+// columns: the lanes of a 256-column wave past N_tau would idle (half of them
+// on a 125-column map; 1024 such maps of 125 rows: 59 us with C = 4, 37 us
+// with C = 2).
+//
+// Bound: VALU issue (every SIMD cycle is taken).  A 16-cell step issues ~490
+// instructions, 306 of them FP64 -- 7 differences, 2 for the determinant and
+// 10 for the numerator per cell, which is what the formula takes -- at ~4.4
+// cycles each, and 32 transcendentals at ~8.3.  The FP64 matrix instructions
+// do not run beside vector work on this chip (measured), so the differences
+// stay on the VALU.  1024 templates of 1000 to 8000 bins, 1.57e9 cells, BtSG:
+// maps 2150 -> 1880 us (0.83e12 cells/s, 3.3 TB/s of map written) with the
+// shared condition test, the diagonal order, the narrow last blocks, the
+// position of the maximum found once per item, and 192 rows an item.
+template <int C>
+constexpr int LDS_GS = C * NC + 1 - (C * NC) % 2;
 // entry (diagonal d, component k) of the staged range
+template <int C>
 __host__ __device__ __forceinline__ int lds_at(int d, int k) {
-    return (d >> 2) * LDS_GS + k * 4 + (d & 3);
+    return d / C * LDS_GS<C> + k * C + d % C;
 }
 // doubles of LDS for nd diagonals
-__host__ __device__ __forceinline__ int lds_doubles(int nd) { return (nd + 3) / 4 * LDS_GS; }
+template <int C>
+constexpr int lds_doubles(int nd) {
+    return (nd + C - 1) / C * LDS_GS<C>;
+}
+// columns per lane of the column block that starts `rem` columns before N_tau
+__host__ __device__ __forceinline__ int rect_lane_cols(int rem) {
+    return rem > 128 ? 4 : rem > 64 ? 2 : 1;
+}
+// dynamic LDS of an item of rb rows: the rows' references and sums, then the
+// staged range, which the item's final reduction reuses
+constexpr int rect_item_lds(int rb, int C) {
+    const int nd = rb + 64 * C - 1;
+    return rb * 2 * (int)sizeof(float) +
+           (C == 4 ? lds_doubles<4>(nd) : C == 2 ? lds_doubles<2>(nd) : lds_doubles<1>(nd)) *
+               (int)sizeof(double);
+}
+static_assert(rect_item_lds(16, 1) - 16 * 2 * sizeof(float) >= sizeof(FinShared) &&
+                  rect_item_lds(16, 2) - 16 * 2 * sizeof(float) >= sizeof(FinShared),
+              "the staged range holds the final reduction");
+
+// The condition test of a lane's cells at once.  With a^2, b^2 >= 0 in every
+// bin (the stage kernel flags templates where that fails) the trace T of a
+// window is at most that of the window from the block's first start to its
+// last end, so T_all^2 < Q min(D) implies T^2 < Q D for every cell, and the
+// quotients stand as they are; otherwise the wave repeats the test cell by
+// cell.  The slack covers the determinants' rounding to float (6e-8) and that
+// of the prefix sums (1e-11 of the window on 8000 bins).  Windows fail the
+// shared test only when they are a few bins long, i.e. in a template's first
+// column block, whose items test cell by cell from the start.  Per 16 cells: 8
+// minima and ~8 FP64 operations in place of 80.
+constexpr double GUARD_SLACK = 1.0 + 1e-5;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// A lane's cells of one row, in one register tuple as their store needs them;
+// rows of a map start at any 4-byte boundary.
+template <int C>
+struct RowCells;
+template <>
+struct RowCells<4> {
+    typedef f32x4 type;
+    typedef f32x4 store __attribute__((aligned(4)));
+};
+template <>
+struct RowCells<2> {
+    typedef f32x2 type;
+    typedef f32x2 store __attribute__((aligned(4)));
+};
+template <>
+struct RowCells<1> {
+    struct type {
+        float v;
+        __device__ float &operator[](int) { return v; }
+        __device__ float operator[](int) const { return v; }
+    };
+    typedef type store;
+};
 
 // Word 3 of a raw buffer resource: 32-bit data format, as gfx9 raw buffer
 // accesses require.
@@ -811,131 +945,246 @@ __device__ __forceinline__ int64_t block_slot() {
 #endif
 }
 
-#ifndef TCW_FAST_MIN_WAVES
-#define TCW_FAST_MIN_WAVES 4
-#endif
+// The wave's maximum (into `best`, on every lane) and the first cell
+// (row-major) that holds it, from each lane's maximum and the step that
+// brought it.  The cells of that step are evaluated again, by the same
+// operations: the 4 C cells of the one lane that holds the maximum on as many
+// lanes, or row by row where several lanes hold it.  This runs once a wave and
+// item; keeping the position as the steps go by costs a 71-instruction search
+// whenever any lane of the wave sees a new maximum (about three of eight
+// steps).
+template <int C>
+__device__ __forceinline__ int rect_first_max(float &best, int bstep, const TmplDev &td,
+                                              const double *__restrict__ P,
+                                              const double *__restrict__ lds, int row0, int col0,
+                                              int wave, int lane) {
+    const float wm = wave_max(best);
+    const int s = wave_min_idx(best == wm ? bstep : 0x7fffffff);
+    uint64_t held = __ballot(best == wm && bstep == s);
+    best = wm;
+    if (wm == -INFINITY) return 0x7fffffff;
+    const int N_t0 = (int)td.N_t0, N_tau = (int)td.N_tau;
+    const int rl0 = s * 16 + wave * 4;
+    auto value = [&](int r, int col) {  // cell (row0 + rl0 + r, col0 + col)
+        const double *__restrict__ pi =
+            P + (int64_t)min(td.q0 + td.a * (row0 + rl0 + r), (int)td.N - 1) * NC;
+        double S[NC];
+#pragma unroll
+        for (int k = 0; k < NC; k++) S[k] = lds[lds_at<C>(rl0 + r + col, k)] - pi[k];
+        return cell_F(S[0], S[1], S[2], S[3], S[4], S[5], S[6]);
+    };
+    if (__popcll(held) == 1) {
+        const int r = lane / C & 3;
+        const int col = __builtin_ctzll(held) * C + lane % C;
+        const bool in = lane < 4 * C && row0 + rl0 + r < N_t0 && col0 + col < N_tau;
+        const uint64_t at = __ballot(in && value(r, col) == wm);
+        if (at) {
+            const int q = __builtin_ctzll(at);
+            return (row0 + rl0 + q / C) * N_tau + col0 + __builtin_ctzll(held) * C + q % C;
+        }
+    }
+    for (int r = 0; r < 4 && row0 + rl0 + r < N_t0; r++) {
+        int first = C;  // the lane's first column of row r that holds the maximum
+#pragma unroll
+        for (int c = C - 1; c >= 0; c--)
+            if (col0 + lane * C + c < N_tau && value(r, lane * C + c) == wm) first = c;
+        const uint64_t at = __ballot(first < C);
+        if (at) {
+            const int l = __builtin_ctzll(at);
+            return (row0 + rl0 + r) * N_tau + col0 + l * C + __builtin_amdgcn_readlane(first, l);
+        }
+    }
+    return 0x7fffffff;
+}
 
-template <bool BTSG, bool STRICT>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(TCW_FAST_MIN_WAVES, 8)))
-void rect_fast_kernel(
-    const TmplDev *__restrict__ tds, const ItemDev *__restrict__ items, int64_t item0,
-    const double *__restrict__ prefix, float *__restrict__ Fout,
-    ItemPart *__restrict__ ipart, float *__restrict__ rowpart,
-    float *__restrict__ colpart, int *__restrict__ flags) {
-    extern __shared__ double lds[];
-    __shared__ float sh_rowM[MAX_RB];
-    __shared__ float sh_rowS[MAX_RB];
-    const int64_t item_id = item0 + block_slot();
-    const ItemDev it = items[item_id];
-    const TmplDev td = tds[it.t];
+// One work item.  FIRST: the template's first column block (cell-by-cell
+// condition test).
+template <bool BTSG, bool STRICT, int C, bool FIRST>
+__device__ __forceinline__ void rect_fast_item(const TmplDev &td, const ItemDev &it,
+                                               int64_t item_id, const double *__restrict__ P,
+                                               float *__restrict__ Ft, ItemPart *ipart,
+                                               float *rowpart, float *colpart, int *flags,
+                                               double *lds) {
     const int RB = td.rb_rows;
     const int row0 = it.rb * RB;
     const int col0 = it.cb * TILE_COLS;
     const int N_t0 = (int)td.N_t0, N_tau = (int)td.N_tau;
-    const int nd = RB + TILE_COLS - 1;
+    const int nd = RB + 64 * C - 1;
     const int D0 = row0 + col0;
-    const double *__restrict__ P = prefix + td.prefix_off;
     const int Nm1 = (int)td.N - 1;
+    float *sh_rowM = reinterpret_cast<float *>(lds);
+    float *sh_rowS = sh_rowM + RB;
+    lds += RB;
 
     for (int d = threadIdx.x; d < nd; d += WG) {
         int64_t q = (int64_t)td.q00 + (int64_t)td.a * (D0 + d) - 1;
         q = min(max(q, (int64_t)0), (int64_t)Nm1);
         const double *__restrict__ src = P + (q + 1) * NC;
 #pragma unroll
-        for (int c = 0; c < NC; c++) lds[lds_at(d, c)] = src[c];
+        for (int c = 0; c < NC; c++) lds[lds_at<C>(d, c)] = src[c];
     }
     __syncthreads();
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    Reducer<BTSG> red;
+    Reducer<BTSG, C> red;
     red.init();
+    int bstep = 0;  // the step that brought the lane's maximum
     bool single = false;
-    float *__restrict__ Ft = Fout + td.F_off;
-    const int c0 = col0 + lane * 4;  // the lane's first column
-    const int nvc = min(max(N_tau - c0, 0), 4);
-    int colidx[4];
+    const int c0 = col0 + lane * C;  // the lane's first column
+    int colidx[C];
 #pragma unroll
-    for (int c = 0; c < 4; c++) colidx[c] = c0 + c;
-    const bool cols_full = col0 + TILE_COLS <= N_tau;
-    // partial sub-tiles store through a buffer resource over their rows
-    // inside the map: the lane's column c at byte voff[c] of a row, or far
-    // outside the resource for a column past N_tau (the hardware drops the
-    // store; rows past the map lie beyond the resource as well), so no
-    // branch per cell
+    for (int c = 0; c < C; c++) colidx[c] = c0 + c;
+    const bool cols_full = col0 + 64 * C <= N_tau;
+    const bool no_bound = !FIRST && (flags[it.t] & FLAG_NO_BOUND);
     const uint32_t rowb = (uint32_t)N_tau * (uint32_t)sizeof(float);
-    uint32_t voff[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) voff[c] = c < nvc ? (uint32_t)(c0 + c) * 4u : 0x80000000u;
 
     for (int s = 0; s < RB / 16; s++) {
         const int rl0 = s * 16 + wave * 4;
         const int m0 = row0 + rl0;
         if (m0 >= N_t0) break;
         const int nvr = min(N_t0 - m0, 4);
-        // lane's diagonals d = rl0 + 4*lane + x, x = 0..6; rl0 + 4*lane is a
-        // multiple of 4, so lds_at(d, k) = lb + lds_at(x, k)
-        const double *__restrict__ lb = lds + lds_at(rl0 + lane * 4, 0);
-        double w[4][NC];
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int k = 0; k < NC; k++) w[c][k] = lb[lds_at(c, k)];
-        float F[4][4];
+        // lane's diagonals d = rl0 + C*lane + x, x = 0 .. C + 2; rl0 + C*lane
+        // is a multiple of C, so lds_at(d, k) = lb + lds_at(x, k)
+        const double *__restrict__ lb = lds + lds_at<C>(rl0 + lane * C, 0);
+        // window starts: wave-uniform, read through the scalar cache
+        int i0[4];
+        double Pi[4][NC];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            if (r > 0) {
+            i0[r] = min(td.q0 + td.a * (m0 + r), Nm1);
 #pragma unroll
-                for (int c = 0; c < 3; c++)
+            for (int k = 0; k < NC; k++) Pi[r][k] = P[(int64_t)i0[r] * NC + k];
+        }
+        typename RowCells<C>::type F[4];
+        float Dmin = INFINITY;
+        double Tall = 0.0;
+        // Diagonal by diagonal: its entry meets the starts of up to four rows.
+        // The starts sit in scalar registers, so a lane holds one diagonal's 7
+        // sums at a time (79 VGPRs, six waves a SIMD; row by row it holds C of
+        // them: 96-104, four or five waves).
 #pragma unroll
-                    for (int k = 0; k < NC; k++) w[c][k] = w[c + 1][k];
-                const int x = r + 3;
+        for (int x = 0; x < C + 3; x++) {
+            double w[NC];
 #pragma unroll
-                for (int k = 0; k < NC; k++) w[3][k] = lb[lds_at(x, k)];
-            }
-            // window start: wave-uniform, read through the scalar cache
-            const int i = min(td.q0 + td.a * (m0 + r), Nm1);
-            double Pi[NC];
+            for (int k = 0; k < NC; k++) w[k] = lb[lds_at<C>(x, k)];
+            // the window from the block's first start to its last end
+            if (!FIRST && x == C + 2) Tall = (w[0] - Pi[0][0]) + (w[1] - Pi[0][1]);
 #pragma unroll
-            for (int k = 0; k < NC; k++) Pi[k] = P[(int64_t)i * NC + k];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                F[r][c] = cell_F(w[c][0] - Pi[0], w[c][1] - Pi[1], w[c][2] - Pi[2],
-                                 w[c][3] - Pi[3], w[c][4] - Pi[4], w[c][5] - Pi[5],
-                                 w[c][6] - Pi[6]);
-                if (STRICT) {
-                    const int m = m0 + r;
-                    int64_t q = (int64_t)td.q00 + (int64_t)td.a * (m + colidx[c]) - 1;
-                    q = min(max(q, (int64_t)0), (int64_t)Nm1);
-                    single |= (q == i) && (r < nvr) && (c < nvc);
+            for (int r = 0; r < 4; r++) {
+                const int c = x - r;
+                if (c < 0 || c >= C) continue;
+                float f;
+                if constexpr (FIRST) {
+                    f = cell_F(w[0] - Pi[r][0], w[1] - Pi[r][1], w[2] - Pi[r][2], w[3] - Pi[r][3],
+                               w[4] - Pi[r][4], w[5] - Pi[r][5], w[6] - Pi[r][6]);
+                } else {
+                    float Df;
+                    f = cell_quot(w[0] - Pi[r][0], w[1] - Pi[r][1], w[2] - Pi[r][2],
+                                  w[3] - Pi[r][3], w[4] - Pi[r][4], w[5] - Pi[r][5],
+                                  w[6] - Pi[r][6], Df);
+                    Dmin = fminf(Dmin, Df);
                 }
+                // (finished here: not after the shared test, nor together with
+                // the other diagonals' cells)
+                asm volatile("" : "+v"(f));
+                F[r][c] = f;
+                if (STRICT) {
+                    int64_t q = (int64_t)td.q00 + (int64_t)td.a * (m0 + r + colidx[c]) - 1;
+                    q = min(max(q, (int64_t)0), (int64_t)Nm1);
+                    single |= (q == i0[r]) && (r < nvr) && (colidx[c] < N_tau);
+                }
+            }
+        }
+        if constexpr (!FIRST) {
+            const bool ok_all = Tall * Tall * GUARD_SLACK < QCOND * (double)Dmin;
+            if (no_bound || !__all(ok_all)) {  // wave-uniform: cell by cell
+                // (an address the compiler cannot match with the one above: it
+                // would keep the differences of all cells alive, and spill)
+                int at = rl0 + lane * C;
+                asm volatile("" : "+v"(at));
+                const double *__restrict__ lb = lds + lds_at<C>(at, 0);
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        const int x = r + c;
+                        if (!cell_ok(lb[lds_at<C>(x, 0)] - Pi[r][0], lb[lds_at<C>(x, 1)] - Pi[r][1],
+                                     lb[lds_at<C>(x, 2)] - Pi[r][2]))
+                            F[r][c] = 2.0f;
+                    }
             }
         }
         if (cols_full && nvr == 4) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                float *Frow = Ft + (int64_t)(m0 + r) * N_tau + c0;
-#pragma unroll
-                for (int c = 0; c < 4; c++) Frow[c] = F[r][c];
-            }
+            for (int r = 0; r < 4; r++)
+                *(typename RowCells<C>::store *)(Ft + (int64_t)(m0 + r) * N_tau + c0) = F[r];
         } else {
+            // partial sub-tiles store through a buffer resource over their rows
+            // inside the map: the lane's column c at byte voff of a row, or far
+            // outside the resource for a column past N_tau (the hardware drops
+            // the store; rows past the map lie beyond the resource as well), so
+            // no branch per cell (the offsets are formed here: held over the
+            // loop, they cost registers)
+            int first = c0, nvc = N_tau - c0;
+            asm volatile("" : "+v"(first), "+v"(nvc));
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
                 Ft + (int64_t)m0 * N_tau, (short)0, (int)((uint32_t)nvr * rowb), BUF_RSRC_WORD3);
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
+                for (int c = 0; c < C; c++) {
+                    const uint32_t voff = c < nvc ? (uint32_t)(first + c) * 4u : 0x80000000u;
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F[r][c]), rs,
-                                                          (int)voff[c], (int)(r * rowb), 0);
+                                                          (int)voff, (int)(r * rowb), 0);
                     F[r][c] = (r < nvr) && (c < nvc) ? F[r][c] : -INFINITY;
                 }
         }
-        red.template add<4>(F, m0, colidx, N_tau, lane, rl0, sh_rowM, sh_rowS);
+        const float lm = red.block_max(F);
+        bstep = lm > red.best ? s : bstep;
+        red.best = fmaxf(red.best, lm);
+        red.sums(F, lm, lane, rl0, sh_rowM, sh_rowS);
     }
-    if (STRICT && single) atomicOr(flags + it.t, 1);
-    __syncthreads();
-    finish_item(red, wave, lane, td, it, item_id, min(RB, N_t0 - row0), ipart, rowpart,
-                      colpart, sh_rowM, sh_rowS, [](int ln, int c) { return ln * 4 + c; });
+    if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
+    red.bidx = rect_first_max<C>(red.best, bstep, td, P, lds, row0, col0, wave, lane);
+    __syncthreads();  // the staged range is consumed: the final reduction reuses it
+    finish_item(red, wave, lane, td, it, item_id, min(RB, N_t0 - row0), ipart, rowpart, colpart,
+                sh_rowM, sh_rowS, *reinterpret_cast<FinShared *>(lds),
+                [](int ln, int c) { return ln * C + c; });
+}
+
+template <bool BTSG, bool STRICT>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void rect_fast_kernel(
+    const TmplDev *__restrict__ tds, const ItemDev *__restrict__ items, int64_t item0,
+    const double *__restrict__ prefix, float *__restrict__ Fout,
+    ItemPart *__restrict__ ipart, float *__restrict__ rowpart,
+    float *__restrict__ colpart, int *__restrict__ flags) {
+    extern __shared__ double lds[];
+    const int64_t item_id = item0 + block_slot();
+    const ItemDev it = items[item_id];
+    const TmplDev td = tds[it.t];
+    const double *P = prefix + td.prefix_off;
+    float *Ft = Fout + td.F_off;
+    const int C = rect_lane_cols((int)td.N_tau - it.cb * TILE_COLS);
+#define RECT_ITEM(cols, first)                                                              \
+    rect_fast_item<BTSG, STRICT, cols, first>(td, it, item_id, P, Ft, ipart, rowpart, colpart, \
+                                              flags, lds)
+    if (it.cb == 0) {  // block-uniform
+        if (C == 4)
+            RECT_ITEM(4, true);
+        else if (C == 2)
+            RECT_ITEM(2, true);
+        else
+            RECT_ITEM(1, true);
+    } else {
+        if (C == 4)
+            RECT_ITEM(4, false);
+        else if (C == 2)
+            RECT_ITEM(2, false);
+        else
+            RECT_ITEM(1, false);
+    }
+#undef RECT_ITEM
 }
 
 // ----------------------------------------------------------------------------
@@ -976,6 +1225,7 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
     float *__restrict__ colpart, int *__restrict__ flags) {
     __shared__ float sh_rowM[MAX_RB];
     __shared__ float sh_rowS[MAX_RB];
+    __shared__ FinShared sh_fin;
     const int64_t item_id = item0 + block_slot();
     const ItemDev it = items[item_id];
     const TmplDev td = tds[it.t];
@@ -1018,12 +1268,13 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
             if (valid) Ft[(int64_t)m * N_tau + colidx[c]] = f;
             F[0][c] = valid ? f : -INFINITY;
         }
-        red.template add<1>(F, m, colidx, N_tau, lane, rl, sh_rowM, sh_rowS);
+        red.add(F, m, colidx, N_tau, lane, rl, sh_rowM, sh_rowS);
     }
-    if (STRICT && single) atomicOr(flags + it.t, 1);
+    if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
     __syncthreads();
+    wave_argmax(red.best, red.bidx);
     finish_item(red, wave, lane, td, it, item_id, min(RB, N_t0 - row0), ipart, rowpart,
-                      colpart, sh_rowM, sh_rowS, [](int ln, int c) { return c * 64 + ln; });
+                colpart, sh_rowM, sh_rowS, sh_fin, [](int ln, int c) { return c * 64 + ln; });
 }
 
 // Exponential window, direct weighted sum over the truncated support
@@ -1041,6 +1292,7 @@ __global__ __launch_bounds__(WG) void exp_direct_kernel(
     float *__restrict__ colpart, int *__restrict__ flags) {
     __shared__ float sh_rowM[MAX_RB];
     __shared__ float sh_rowS[MAX_RB];
+    __shared__ FinShared sh_fin;
     const int64_t item_id = item0 + block_slot();
     const ItemDev it = items[item_id];
     const TmplDev td = tds[it.t];
@@ -1109,12 +1361,13 @@ __global__ __launch_bounds__(WG) void exp_direct_kernel(
             if (valid) Ft[(int64_t)m * N_tau + colidx[c]] = f;
             F[0][c] = valid ? f : -INFINITY;
         }
-        red.template add<1>(F, m, colidx, N_tau, lane, rl, sh_rowM, sh_rowS);
+        red.add(F, m, colidx, N_tau, lane, rl, sh_rowM, sh_rowS);
     }
-    if (STRICT && single) atomicOr(flags + it.t, 1);
+    if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
     __syncthreads();
+    wave_argmax(red.best, red.bidx);
     finish_item(red, wave, lane, td, it, item_id, min(RB, N_t0 - row0), ipart, rowpart,
-                      colpart, sh_rowM, sh_rowS, [](int ln, int c) { return c * 64 + ln; });
+                colpart, sh_rowM, sh_rowS, sh_fin, [](int ln, int c) { return c * 64 + ln; });
 }
 
 // ----------------------------------------------------------------------------
@@ -1713,7 +1966,7 @@ __device__ __forceinline__ void expw_rows(const TmplDev &td, const ExpWalk &wk, 
         }
         vo -= 4 * rowb;
         if (g - 3 <= m_hi)
-            red.template add<4>(F4, g - 3, colidx, N_tau, lane, g - 3 - sb, sh_rowM, sh_rowS);
+            red.add(F4, g - 3, colidx, N_tau, lane, g - 3 - sb, sh_rowM, sh_rowS);
     }
 }
 
@@ -1807,7 +2060,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         }
         __syncthreads();  // staging, row sums and sh_M are rewritten by the next pass
     }
-    if (STRICT && single) atomicOr(flags + it.t, 1);
+    if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
     // combine: each column belongs to one lane; each row to all 4 waves
     wave_argmax(red.best, red.bidx);
     float stot = 0.0f;
@@ -2040,7 +2293,7 @@ __global__ __launch_bounds__(NT) void finalize_kernel(
     if (threadIdx.x == 0) {
         tcw_stats st;
         st.maxF = maxF;
-        st.single_atom = flags[t];
+        st.single_atom = flags[t] & FLAG_SINGLE_ATOM;
         st.m_ML = m_ML;
         st.n_ML = n_ML;
         st.N_t0 = td.N_t0;
@@ -2492,9 +2745,10 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         for (uint32_t cbk = 0; cbk < td.n_colblk; cbk++)
             items_by_mode[mode].push_back(ItemDev{(int32_t)t, (int32_t)rbk, (int32_t)cbk, 0});
     if (mode == MODE_RECT_FAST) {
-        const int nd = rb + TILE_COLS - 1;
-        const int bytes = (int)sizeof(double) * lds_doubles(nd);
-        p.max_lds_bytes = std::max(p.max_lds_bytes, bytes);
+        // the widest column block (the first) and the last one
+        const int last = (int)N_tau - (int)(td.n_colblk - 1) * TILE_COLS;
+        for (int rem : {(int)std::min<int64_t>(N_tau, TILE_COLS), last})
+            p.max_lds_bytes = std::max(p.max_lds_bytes, rect_item_lds(rb, rect_lane_cols(rem)));
     }
     p.tmpl.push_back(td);
     return TCW_OK;
