@@ -50,7 +50,10 @@ namespace {
 constexpr int NC = TCW_NCOL;
 constexpr int WG = 256;           // threads per workgroup (4 wave64)
 constexpr int TILE_COLS = 256;    // tau columns per work item
-constexpr int MERGED_STRIDE = 8;  // floats per atom in the atom table (7 columns + pad)
+constexpr int MERGED_STRIDE = 8;  // floats per atom in the atom table (7 columns + kind)
+// the kind column: 0 for a bin of zeros, 1 for one with data, BIN_ODD for one
+// with an infinity or NaN (more than any count of bins with data)
+constexpr float BIN_ODD = 2147483648.0f;
 constexpr double COND_MAX = 1e4;  // rect.cu:104
 // cond < K  <=>  T^2 < Q*D  with T = A+B, D = AB-C^2 > 0, Q = (K+1)^2/K, because
 // cond = (T+s)/(T-s), s^2 = T^2-4D, and (1+cond)^2/cond = T^2/D grows with cond.
@@ -71,6 +74,13 @@ constexpr int RB_DEFAULT[MODE_COUNT] = {192, 16, 16, 128};
 // at a time (256 templates of 48 x 48 to 240 x 240: maps 22 us, 26 at 1024
 // items, 29 at 512; 1024 templates of 125 x 125: 35 us, 37 at 1024, 38 at 4096).
 constexpr int64_t SMALL_BATCH_ITEMS = 2048;
+// exp_walk_kernel items aimed at when rows are not tuned: two a CU, which is
+// how many fit at a time; fewer rows repeat the direct sum, more leave CUs idle
+// (256 templates of 125 x 125 cells: 130 us at 64 rows, 165 at 32, 152 at 128;
+// 64 of 500 x 500: 575 us at 128 rows, 739 at 64, 604 at 256; 4 of 500 x 500:
+// 200 us at 16 rows, 228 at 32).
+constexpr int64_t WALK_ITEMS = 512;
+constexpr int WALK_MAX_ROWS = 256;
 constexpr int EXP_SMALL_BATCH_ROWS = 64;    // exp rows when untuned and under 256 column blocks
 
 struct TmplDev {
@@ -92,6 +102,7 @@ struct TmplDev {
                                  // L(n) = L0 + Ls*n atoms, atoms [0, H) reachable
     int32_t n_seg;               // MODE_EXP_FAST: row chunks (>= n_rowblk)
     int32_t init_empty;          // MODE_EXP_FAST: the top chunk's direct sum is empty
+    int32_t walk;                // MODE_EXP_DIRECT: exp_walk_item applies
     int64_t etab_off;            // MODE_EXP_FAST: doubles, [n_seg + INIT_PARTS][7][N_tau]
     uint32_t o_t0, o_t0Band, o_tau, o_tauBand;  // caller's window (posterior modes)
 };
@@ -454,9 +465,14 @@ __global__ __launch_bounds__(256) void stage_exp_kernel(
 #pragma unroll
         for (int j = 0; j < SX_BINS; j++) {
             float *r = s_raw + (tid * SX_BINS + j) * SX_ROW;
+            bool some = false, odd = false;
 #pragma unroll
-            for (int c = 0; c < NC; c++) r[c] = v[j][c];
-            r[NC] = 0.0f;
+            for (int c = 0; c < NC; c++) {
+                r[c] = v[j][c];
+                some |= v[j][c] != 0.0f;
+                odd |= !(fabsf(v[j][c]) < INFINITY);
+            }
+            r[NC] = odd ? BIN_ODD : some ? 1.0f : 0.0f;
         }
         __syncthreads();
         float *base = merged + td.merged_off + (int64_t)B0 * MERGED_STRIDE;
@@ -1159,7 +1175,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     const double *__restrict__ prefix, float *__restrict__ Fout,
     ItemPart *__restrict__ ipart, float *__restrict__ rowpart,
     float *__restrict__ colpart, int *__restrict__ flags) {
-    extern __shared__ double lds[];
+    extern __shared__ double lds_raw[];  // one dynamic LDS symbol per file
     const int64_t item_id = item0 + block_slot();
     const ItemDev it = items[item_id];
     const TmplDev td = tds[it.t];
@@ -1168,7 +1184,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     const int C = rect_lane_cols((int)td.N_tau - it.cb * TILE_COLS);
 #define RECT_ITEM(cols, first)                                                              \
     rect_fast_item<BTSG, STRICT, cols, first>(td, it, item_id, P, Ft, ipart, rowpart, colpart, \
-                                              flags, lds)
+                                              flags, lds_raw)
     if (it.cb == 0) {  // block-uniform
         if (C == 4)
             RECT_ITEM(4, true);
@@ -1277,6 +1293,405 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
                 colpart, sh_rowM, sh_rowS, sh_fin, [](int ln, int c) { return c * 64 + ln; });
 }
 
+// Exponential window off the atom grid: the window sum slides with any steps.
+//
+// Row m starts at T = t0 + m dt0 - t_min = TAtom q + phi, column n lasts 3 tau =
+// TAtom Q + R.  The cell's atoms (exp.cu:39-102) are lo(m) .. hi(m, n),
+//   lo = q + [phi > 0],   hi = q + Q - 1 + [s >= h] + [s >= TAtom + h],
+// s = phi + R, h = TAtom - TAtom / 2 (atoms at or past N count as zero), with
+// weights w rho^(i - lo), rho = e^(-TAtom/tau).  F does not change with a
+// common factor of the weights, so w is left out, and
+//   E(m) = sum_{i = lo}^{hi} rho^(i - lo) x_i   (rho^2 for a^2, b^2, ab)
+// goes from row to row by the atoms that enter (the same on every lane) and
+// those that leave (dt0 / TAtom or one more, by lane):
+//   E(m-1) = rho^(lo - lo') E(m) + sum_{i = lo'}^{lo-1} rho^(i-lo') x_i
+//            - sum_{i = hi'+1}^{hi} rho^(i-lo') x_i;
+// rho^(hi' + 1 - lo') is one of four values per lane, as that exponent is
+// Q - 1 .. Q + 2.  A cell costs O(dt0 / TAtom) instead of O(3 tau / TAtom).
+//
+// An item of RB rows x 256 columns starts with the direct sum at its top row
+// and walks down.  A group of 64 columns has two waves, or four or eight in
+// items of at most 128 or 64 columns: they share the direct sum's atoms (staged
+// in LDS chunk by chunk), then all walk and take turns at evaluating four rows.
+// Entering and leaving atoms come from LDS where the item's ranges of them fit.
+//
+// What the direct sum gives exactly and a sliding sum would not: a window
+// whose bins are all zero has E = 0 (the kind column counts bins with data),
+// and from the first infinite or NaN atom on, the item's rows are summed
+// directly, as are all rows where the steps are longer than the windows.
+//
+// Bound: latency -- the direct sum at the top (16 to 21 instructions and 16 LDS
+// cycles an atom and wave, two waves a SIMD) and ~0.9 us a row step.  32
+// templates of 125 x 125 cells and 1000 bins: 700 us with a direct sum for
+// every cell, 52 us so (four waves a workgroup instead of eight: 74; the atoms
+// through scalar loads instead of LDS: 172).
+constexpr int WALK_WAVES = 8;
+constexpr int WALK_WG = 64 * WALK_WAVES;
+constexpr int WALK_TAIL_CAP = 1024;  // leaving atoms staged in LDS (32 KB)
+constexpr int WALK_HEAD_CAP = 256;   // entering atoms staged in LDS (8 KB)
+constexpr int WALK_CHUNK = 512;      // atoms of the direct sum staged at a time (16 KB)
+static_assert(WALK_WAVES * MERGED_STRIDE * 64 * 2 <= WALK_TAIL_CAP * MERGED_STRIDE &&
+                  WALK_CHUNK <= WALK_TAIL_CAP,
+              "the direct sum's chunk and parts share the leaving atoms' LDS");
+constexpr int walk_lds(int rb) {
+    return ((WALK_TAIL_CAP + WALK_HEAD_CAP) * MERGED_STRIDE + 4 * rb * 2) * (int)sizeof(float);
+}
+
+struct WalkCol {  // a lane's column, 3 tau = TAtom Q + R
+    double rho[2];   // rho^2, rho
+    double lead[4];  // rho^(Q - 1 + k)
+    double ratau;    // TAtom / tau
+    int Q;
+    uint32_t R;
+};
+
+struct WalkRow {  // a row's start, T = TAtom q + phi
+    int q;
+    uint32_t phi;
+    __device__ int lo() const { return q + (phi > 0); }
+    // hi - (q + Q - 1) of the lane's column
+    __device__ int end(const WalkCol &wc, uint32_t TA) const {
+        const uint32_t s = phi + wc.R, h = TA - TA / 2;
+        return (s >= h) + (s >= TA + h);
+    }
+    __device__ int hi(const WalkCol &wc, uint32_t TA) const { return q + wc.Q - 1 + end(wc, TA); }
+};
+
+// Copy `count` atoms (at most CAP) of the table to LDS, all loads of a thread
+// in flight together; true if one of this thread's atoms is not finite.
+template <int CAP>
+__device__ __forceinline__ bool walk_stage(float *dst, const float *__restrict__ src, int count) {
+    static_assert(MERGED_STRIDE == 8, "two 16-byte words an atom, the kind in the second");
+    constexpr int PER = (CAP * 2 + WALK_WG - 1) / WALK_WG;
+    f32x4 v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const int k = i * WALK_WG + (int)threadIdx.x;
+        if (k < count * 2) v[i] = reinterpret_cast<const f32x4 *>(src)[k];
+    }
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const int k = i * WALK_WG + (int)threadIdx.x;
+        if (k < count * 2) {
+            reinterpret_cast<f32x4 *>(dst)[k] = v[i];
+            odd |= (k & 1) && v[i][3] == BIN_ODD;
+        }
+    }
+    return odd;
+}
+
+// E = sum over atoms x[0 .. count) of rho^l x_l, and the sum of their kinds, by
+// Horner from the far end.  MASK: atoms l >= L are left out on this lane: the
+// sum starts anew at l = L - 1 (the weight of what came before is 0 there,
+// which is why every atom has to be finite).
+template <bool MASK>
+__device__ __forceinline__ void walk_horner(const float *x, int count, int L, const WalkCol &wc,
+                                            double (&E)[NC], float &kinds) {
+#pragma unroll 4
+    for (int l = count - 1; l >= 0; l--) {
+        const float *v = x + l * MERGED_STRIDE;
+        double r0 = wc.rho[0], r1 = wc.rho[1];
+        if (MASK) {
+            r0 = l == L - 1 ? 0.0 : r0;
+            r1 = l == L - 1 ? 0.0 : r1;
+            kinds = l == L - 1 ? 0.0f : kinds;
+        }
+#pragma unroll
+        for (int c = 0; c < NC; c++) E[c] = fma(c < 3 ? r0 : r1, E[c], (double)v[c]);
+        kinds += v[NC];
+    }
+}
+
+// The direct sum of a row, for any atoms: lo + l for l below the lane's L (at
+// most Lmax on any lane; uniform), read from the table X below atom N.
+__device__ __forceinline__ void walk_row_sum(const float *__restrict__ X, int N, const WalkCol &wc,
+                                             int lo, int L, int Lmax, double (&E)[NC],
+                                             float &kinds) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) E[c] = 0.0;
+    kinds = 0.0f;
+#pragma unroll 1
+    for (int l = min(Lmax, N - lo) - 1; l >= 0; l--) {
+        const float *v = X + (int64_t)(lo + l) * MERGED_STRIDE;  // uniform: scalar loads
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+            E[c] = fma(wc.rho[c < 3 ? 0 : 1], E[c], l < L ? (double)v[c] : 0.0);
+        kinds += l < L ? v[NC] : 0.0f;
+    }
+}
+
+template <bool BTSG, bool STRICT>
+__global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
+    const TmplDev *__restrict__ tds, const ItemDev *__restrict__ items, int64_t item0,
+    const float *__restrict__ merged, float *__restrict__ Fout, ItemPart *__restrict__ ipart,
+    float *__restrict__ rowpart, float *__restrict__ colpart, int *__restrict__ flags) {
+    extern __shared__ double lds_raw[];  // one dynamic LDS symbol per file
+    __shared__ float sh_best[WALK_WAVES], sh_M[WALK_WAVES], sh_S[WALK_WAVES];
+    __shared__ int sh_bidx[WALK_WAVES];
+    __shared__ float sh_col[WALK_WAVES][64];
+    const int64_t item_id = item0 + block_slot();
+    const ItemDev it = items[item_id];
+    const TmplDev td = tds[it.t];
+    if (!td.walk) return;  // block-uniform: an exp_direct_kernel item
+    float *lds = reinterpret_cast<float *>(lds_raw);
+    const float *__restrict__ X = merged + td.merged_off;
+    float *__restrict__ Ft = Fout + td.F_off;
+    const int RB = td.rb_rows;
+    const int row0 = it.rb * RB, col0 = it.cb * TILE_COLS;
+    const int N_tau = (int)td.N_tau;
+    const int nrows = min(RB, (int)td.N_t0 - row0);
+    const int N = (int)td.N;
+    const uint32_t TA = td.TAtom;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int groups = (min(TILE_COLS, N_tau - col0) + 63) / 64;
+    const int W = WALK_WAVES / (groups == 3 ? 4 : groups);  // waves of a group
+    const int g = wave / W, w = wave % W;
+    const bool active = g < groups;  // (three groups: the others only keep the barriers)
+    const int n = col0 + g * 64 + lane;
+    const bool valid = active && n < N_tau;
+    float *tail = lds;
+    double *comb = reinterpret_cast<double *>(lds);
+    float *head = tail + WALK_TAIL_CAP * MERGED_STRIDE;
+    float *sh_rowM = head + WALK_HEAD_CAP * MERGED_STRIDE;  // [4][RB]
+    float *sh_rowS = sh_rowM + 4 * RB;
+    for (int k = threadIdx.x; k < 4 * RB; k += WALK_WG) {
+        sh_rowM[k] = -INFINITY;
+        sh_rowS[k] = 0.0f;
+    }
+
+    auto column = [&](int nn) {
+        WalkCol wc;
+        const uint32_t tau = td.tau + (uint32_t)nn * td.dtau;
+        wc.ratau = (double)TA / (double)tau;
+        wc.Q = (int)(3u * tau / TA);
+        wc.R = 3u * tau % TA;
+        return wc;
+    };
+    WalkCol wc = column(min(n, N_tau - 1));
+    wc.rho[1] = exp(-wc.ratau);
+    wc.rho[0] = wc.rho[1] * wc.rho[1];
+    wc.lead[0] = exp(-(double)(wc.Q - 1) * wc.ratau);
+#pragma unroll
+    for (int k = 1; k < 4; k++) wc.lead[k] = wc.lead[k - 1] * wc.rho[1];
+    const WalkCol wfirst = column(col0), wlast = column(min(col0 + TILE_COLS, N_tau) - 1);
+
+    const int dq = (int)(td.dt0 / TA);
+    const uint32_t dphi = td.dt0 % TA;
+    auto row_at = [&](int m) {
+        const uint32_t T = td.t0 - td.t_min + (uint32_t)m * td.dt0;
+        return WalkRow{(int)(T / TA), T % TA};
+    };
+    WalkRow row = row_at(row0 + nrows - 1);
+    const WalkRow bottom = row_at(row0);
+    int hi = row.hi(wc, TA);
+    // the last lane's window is the longest, the first one's the shortest
+    const int Q63 = __builtin_amdgcn_readlane(wc.Q, 63);
+    double E[NC];
+    float kinds = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; c++) E[c] = 0.0;
+    bool odd = false;  // an infinity or NaN in reach of the block (block-uniform)
+    {   // the direct sum at the top row, chunk by chunk over the block's longest
+        // window: the waves of a group take equal shares of each chunk
+        const int lo = row.lo();
+        const int L = active ? hi - lo + 1 : 0;
+        const int Lmin = __builtin_amdgcn_readlane(L, 0), Lmax = __builtin_amdgcn_readlane(L, 63);
+        const int Lblk = min(row.hi(wlast, TA) - lo + 1, N - lo);
+        for (int c0 = 0; c0 < Lblk; c0 += WALK_CHUNK) {  // block-uniform
+            const int nc = min(WALK_CHUNK, Lblk - c0);
+            odd |= __syncthreads_or(walk_stage<WALK_CHUNK>(
+                tail, X + (int64_t)(lo + c0) * MERGED_STRIDE, nc));
+            const int share = (nc + W - 1) / W;
+            const int s0 = w * share, cnt = min(min(share, nc - s0), Lmax - c0 - s0);
+            if (cnt > 0 && !odd) {  // uniform
+                double H[NC];
+                float kh = 0.0f;
+#pragma unroll
+                for (int c = 0; c < NC; c++) H[c] = 0.0;
+                if (c0 + s0 + cnt <= Lmin) {
+                    walk_horner<false>(tail + s0 * MERGED_STRIDE, cnt, 0, wc, H, kh);
+                } else {
+                    walk_horner<true>(tail + s0 * MERGED_STRIDE, cnt, L - c0 - s0, wc, H, kh);
+                    if (L <= c0 + s0) {  // the lane's window ends before the share
+                        kh = 0.0f;
+#pragma unroll
+                        for (int c = 0; c < NC; c++) H[c] = 0.0;
+                    }
+                }
+                const double w1 = exp(-(double)(c0 + s0) * wc.ratau);
+#pragma unroll
+                for (int c = 0; c < NC; c++) E[c] = fma(c < 3 ? w1 * w1 : w1, H[c], E[c]);
+                kinds += kh;
+            }
+            __syncthreads();
+        }
+    }
+    if (W > 1) {  // add the group's parts, in one order on all of its waves
+        double *mine = comb + wave * MERGED_STRIDE * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < NC; c++) mine[c * 64] = E[c];
+        mine[NC * 64] = (double)kinds;
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NC; c++) E[c] = 0.0;
+        kinds = 0.0f;
+        for (int k = 0; k < W; k++) {
+            const double *part = comb + (g * W + k) * MERGED_STRIDE * 64 + lane;
+#pragma unroll
+            for (int c = 0; c < NC; c++) E[c] += part[c * 64];
+            kinds += (float)part[NC * 64];
+        }
+        __syncthreads();  // comb is staged over
+    }
+    // atoms that leave and enter in the item's row steps: block-uniform ranges below N
+    const int tail_lo = bottom.q + wfirst.Q;  // hi' + 1 at least
+    const int tail_n = min(N, row.q + wlast.Q + 2) - tail_lo;
+    const int head_lo = bottom.lo();
+    const int head_n = min(N, row.lo()) - head_lo;
+    const bool in_lds = tail_n < WALK_TAIL_CAP && head_n <= WALK_HEAD_CAP;
+    if (in_lds) {
+        // slot 0 holds zeros, for the lanes with no atom to take out
+        if (threadIdx.x < MERGED_STRIDE) tail[threadIdx.x] = 0.0f;
+        walk_stage<WALK_TAIL_CAP>(tail + MERGED_STRIDE, X + (int64_t)tail_lo * MERGED_STRIDE,
+                                  tail_n);
+        walk_stage<WALK_HEAD_CAP>(head, X + (int64_t)head_lo * MERGED_STRIDE, head_n);
+    }
+    __syncthreads();
+    auto load = [&](float (&x)[MERGED_STRIDE], const float *sh, int64_t at, bool some) {
+        if (in_lds) {
+#pragma unroll
+            for (int c = 0; c < MERGED_STRIDE; c++) x[c] = sh[c];
+        } else {
+#pragma unroll
+            for (int c = 0; c < MERGED_STRIDE; c++) x[c] = some ? X[at * MERGED_STRIDE + c] : 0.0f;
+        }
+    };
+
+    Reducer<BTSG, 1> red;
+    red.init();
+    bool single = false;
+    // sum every row directly: where an atom is not finite, or the steps are
+    // longer than the windows
+    bool direct = odd || dq >= Q63;
+    if (odd && active)
+        walk_row_sum(X, N, wc, row.lo(), hi - row.lo() + 1, row.q + Q63 + 2 - row.lo(), E, kinds);
+    const int colidx[1] = {n};
+    for (int k4 = active ? (nrows - 1) / 4 : -1; k4 >= 0; k4--) {
+        const bool mine = k4 % W == w;  // uniform
+        float F4[4][1];
+#pragma unroll
+        for (int j = 3; j >= 0; j--) {
+            const int m = row0 + 4 * k4 + j;
+            F4[j][0] = -INFINITY;
+            if (4 * k4 + j >= nrows) continue;  // uniform
+            if (mine) {
+                const float f = cell_F(E[0], E[1], E[2], E[3], E[4], E[5], E[6]);
+                if (valid) {
+                    Ft[(int64_t)m * N_tau + n] = f;
+                    F4[j][0] = f;
+                }
+                if (STRICT) {
+                    const int i0 = min(row.q + (row.phi + TA / 2 >= TA), N - 1);
+                    single |= valid && min(hi, N - 1) == i0;
+                }
+            }
+            if (m == row0) continue;
+            // to row m - 1
+            const int lo = row.lo();
+            row.q -= dq;
+            if (row.phi < dphi) {
+                row.phi += TA;
+                row.q--;
+            }
+            row.phi -= dphi;
+            const int lo2 = row.lo(), hi2 = row.hi(wc, TA);
+            if (!direct) {
+                for (int l = min(lo, N) - 1; l >= lo2; l--) {
+                    float x[MERGED_STRIDE];
+                    load(x, head + (l - head_lo) * MERGED_STRIDE, l, true);
+                    direct |= __any(x[NC] == BIN_ODD);  // (the same on every lane)
+                    kinds += x[NC];
+#pragma unroll
+                    for (int c = 0; c < NC; c++)
+                        E[c] = fma(wc.rho[c < 3 ? 0 : 1], E[c], (double)x[c]);
+                }
+            }
+            if (direct) {  // uniform
+                walk_row_sum(X, N, wc, lo2, hi2 - lo2 + 1, row.q + Q63 + 2 - lo2, E, kinds);
+            } else {
+                const int lead = row.end(wc, TA) + (row.phi == 0);
+                const double wa = lead & 1 ? wc.lead[1] : wc.lead[0];
+                const double wb = lead & 1 ? wc.lead[3] : wc.lead[2];
+                double w1 = lead & 2 ? wb : wa;
+                double w2 = w1 * w1;
+                const int last = min(hi, N - 1);
+                for (int i = hi2 + 1, d = 0; d <= dq; d++, i++) {
+                    const bool out = i <= last;
+                    float x[MERGED_STRIDE];
+                    load(x, tail + (out ? i - tail_lo + 1 : 0) * MERGED_STRIDE, i, out);
+#pragma unroll
+                    for (int c = 0; c < NC; c++)
+                        E[c] = fma(c < 3 ? -w2 : -w1, (double)x[c], E[c]);
+                    kinds -= x[NC];
+                    w1 *= wc.rho[1];
+                    w2 *= wc.rho[0];
+                }
+                if (kinds == 0.0f) {
+#pragma unroll
+                    for (int c = 0; c < NC; c++) E[c] = 0.0;
+                }
+            }
+            hi = hi2;
+        }
+        if (mine)
+            red.add(F4, row0 + 4 * k4, colidx, N_tau, lane, 4 * k4, sh_rowM + g * RB,
+                    sh_rowS + g * RB);
+    }
+    if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
+    // combine: a column belongs to the waves of its group, a row to one wave of each group
+    wave_argmax(red.best, red.bidx);
+    float stot = 0.0f;
+    if (BTSG) stot = wave_sum(red.total());
+    if (lane == 0) {
+        sh_best[wave] = red.best;
+        sh_bidx[wave] = red.bidx;
+        sh_M[wave] = red.ML;
+        sh_S[wave] = stot;
+    }
+    if (BTSG) sh_col[wave][lane] = red.Scol[0];
+    __syncthreads();
+    float M = sh_M[0];
+    for (int k = 1; k < WALK_WAVES; k++) M = fmaxf(M, sh_M[k]);
+    if (BTSG) {
+        if (valid && w == 0) {
+            float S = 0.0f;
+            for (int k = 0; k < W; k++)
+                if (sh_M[wave + k] != -INFINITY)
+                    S += sh_col[wave + k][lane] * exp2_diff(sh_M[wave + k], M);
+            colpart[td.colpart_off + (int64_t)it.rb * N_tau + n] = S;
+        }
+        for (int rl = threadIdx.x; rl < nrows; rl += WALK_WG) {
+            float S = 0.0f;
+            for (int k = 0; k < groups; k++)
+                if (sh_rowM[k * RB + rl] != -INFINITY)
+                    S += sh_rowS[k * RB + rl] * exp2_diff(sh_rowM[k * RB + rl], M);
+            rowpart[td.rowpart_off + (int64_t)it.cb * td.N_t0 + row0 + rl] = S;
+        }
+    }
+    if (threadIdx.x == 0) {
+        float bv = sh_best[0];
+        int bi = sh_bidx[0];
+        float S = 0.0f;
+        for (int k = 0; k < WALK_WAVES; k++) {
+            argmax_merge(bv, bi, sh_best[k], sh_bidx[k]);
+            if (BTSG && sh_M[k] != -INFINITY) S += sh_S[k] * exp2_diff(sh_M[k], M);
+        }
+        ipart[item_id] = ItemPart{bv, bi, M, S};
+    }
+}
+
 // Exponential window, direct weighted sum over the truncated support
 // (exp.cu:39-102): atoms i in [i_t0, i_t1] with t0 <= t_i <= t1 = t0 + 3 tau,
 // weight w_i = exp(-(t_i - t0)/tau), A/B/C weighted by w^2, Fa/Fb by w.  All
@@ -1296,6 +1711,7 @@ __global__ __launch_bounds__(WG) void exp_direct_kernel(
     const int64_t item_id = item0 + block_slot();
     const ItemDev it = items[item_id];
     const TmplDev td = tds[it.t];
+    if (td.walk) return;  // block-uniform: an exp_walk_kernel item
     const int RB = td.rb_rows;
     const int row0 = it.rb * RB;
     const int col0 = it.cb * TILE_COLS;
@@ -2419,6 +2835,8 @@ struct tcw_plan {
     int64_t F_total = 0;
     int max_lds_bytes = 0;  // rect_fast_kernel dynamic LDS
     int max_lds_expf = 0;   // exp_fast_kernel dynamic LDS
+    int max_lds_walk = 0;   // exp_walk_kernel dynamic LDS
+    int64_t walk_tmpls = 0, direct_tmpls = 0;  // MODE_EXP_DIRECT templates of either kernel
     DevBuf d_tmpl, d_segs, d_items, d_prefix, d_merged, d_ipart, d_rowpart, d_colpart,
         d_flags, d_seg_items, d_col_items, d_etab, d_exp_tmpls, d_init_items;
     hipGraphExec_t graph = nullptr;
@@ -2448,6 +2866,8 @@ struct tcw_plan {
         etab_doubles = 0;
         max_lds_bytes = 0;
         max_lds_expf = 0;
+        max_lds_walk = 0;
+        walk_tmpls = direct_tmpls = 0;
         if (graph) (void)hipGraphExecDestroy(graph);
         graph = nullptr;
     }
@@ -2628,6 +3048,9 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
                              w.dtau % TAtom == 0 && w.tau >= TAtom;
         // (rows of at most 2^20 cells: the map kernel's row stores address a
         // pass of rows by 32-bit byte offsets)
+        // off the grid: the sliding sum with any steps
+        td.walk = !(p.flags & TCW_FLAG_GENERIC) && w.t0 >= t_min && end < (1ull << 32) &&
+                  w.tau >= TAtom;
         if (!(p.flags & TCW_FLAG_GENERIC) && on_grid && end < (1ull << 32) &&
             N_tau <= (int64_t)1 << 20) {
             mode = MODE_EXP_FAST;
@@ -2666,6 +3089,13 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         const double want = (double)N_t0 * ncb * (double)p.T / (double)SMALL_BATCH_ITEMS;
         rb = want >= RB_DEFAULT[mode] ? RB_DEFAULT[mode]
                                       : std::max(16, ((int)std::ceil(want) + 15) / 16 * 16);
+    }
+    if (mode == MODE_EXP_DIRECT && td.walk && req <= 0) {
+        // enough items for the chip, and otherwise long ones: each starts with
+        // a direct sum
+        const double ncb = (double)((N_tau + TILE_COLS - 1) / TILE_COLS);
+        const double want = (double)N_t0 * ncb * (double)p.T / (double)WALK_ITEMS;
+        rb = std::min(WALK_MAX_ROWS, std::max(16, ((int)std::min(want, 1e6) + 15) / 16 * 16));
     }
     if (mode == MODE_EXP_FAST && req <= 0) {
         const int64_t pairs = p.T * ((N_tau + TILE_COLS - 1) / TILE_COLS);
@@ -2730,6 +3160,12 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         p.merged_floats += nbins * MERGED_STRIDE;
         p.exp_tmpls.push_back((int32_t)t);
         p.exp_max_N = std::max<int64_t>(p.exp_max_N, nbins);
+        if (mode == MODE_EXP_DIRECT && td.walk) {
+            p.max_lds_walk = std::max(p.max_lds_walk, walk_lds(rb));
+            p.walk_tmpls++;
+        } else if (mode == MODE_EXP_DIRECT) {
+            p.direct_tmpls++;
+        }
     } else {
         td.prefix_off = p.prefix_doubles;
         p.prefix_doubles += ((int64_t)N + 1) * NC;
@@ -2908,10 +3344,18 @@ void launch_maps(tcw_plan &p, float *F, hipStream_t st) {
                            p.max_lds_expf, st, tds, items, p.mode_begin[MODE_EXP_FAST], merged,
                            (const double *)p.d_etab.p, F, ipart, rowpart, colpart, flags,
                            p.max_lds_expf > 0 ? 1 : 0);
-    if ((n = p.mode_begin[MODE_EXP_DIRECT + 1] - p.mode_begin[MODE_EXP_DIRECT]) > 0)
-        hipLaunchKernelGGL((exp_direct_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG), 0,
-                           st, tds, items, p.mode_begin[MODE_EXP_DIRECT], merged, F, ipart,
-                           rowpart, colpart, flags);
+    // the items of a mode lie template by template: each kernel leaves the
+    // other's at once
+    if ((n = p.mode_begin[MODE_EXP_DIRECT + 1] - p.mode_begin[MODE_EXP_DIRECT]) > 0) {
+        if (p.walk_tmpls > 0)
+            hipLaunchKernelGGL((exp_walk_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WALK_WG),
+                               p.max_lds_walk, st, tds, items, p.mode_begin[MODE_EXP_DIRECT],
+                               merged, F, ipart, rowpart, colpart, flags);
+        if (p.direct_tmpls > 0)
+            hipLaunchKernelGGL((exp_direct_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG), 0,
+                               st, tds, items, p.mode_begin[MODE_EXP_DIRECT], merged, F, ipart,
+                               rowpart, colpart, flags);
+    }
 }
 
 // Optional per-stage event marks: ev[0] before the stage kernel, ev[1] after
