@@ -49,7 +49,7 @@ namespace {
 
 constexpr int NC = TCW_NCOL;
 constexpr int WG = 256;           // threads per workgroup (4 wave64)
-constexpr int TILE_COLS = 256;    // tau columns per work item
+constexpr int TILE_COLS = 256;    // tau columns per work item (rect_step_kernel: 256, 128 or 64)
 constexpr int MERGED_STRIDE = 8;  // floats per atom in the atom table (7 columns + kind)
 // the kind column: 0 for a bin of zeros, 1 for one with data, BIN_ODD for one
 // with an infinity or NaN (more than any count of bins with data)
@@ -92,17 +92,20 @@ struct TmplDev {
     int64_t rowpart_off;         // float, [n_colblk][N_t0], relative to the item max
     int64_t colpart_off;         // float, [n_rowblk][N_tau], relative to the item max
     uint32_t N, TAtom, t_min;    // binned atoms, atom length, t0_data
+    uint32_t TA_rcp;             // floor((2^32 - 1) / TAtom), for div_TA
     uint32_t type, t0, dt0, tau, dtau;  // effective window (after NONE -> RECT)
     uint32_t N_t0, N_tau;
     uint32_t n_rowblk, n_colblk;
     int32_t mode;
     int32_t rb_rows;             // rows per work item
+    int32_t tile;                // columns per work item
     int32_t q0, q00, a;          // MODE_RECT_FAST index maths; a also MODE_EXP_FAST
     int32_t k00, L0, Ls, H;      // MODE_EXP_FAST: first start atom, window lengths
                                  // L(n) = L0 + Ls*n atoms, atoms [0, H) reachable
     int32_t n_seg;               // MODE_EXP_FAST: row chunks (>= n_rowblk)
     int32_t init_empty;          // MODE_EXP_FAST: the top chunk's direct sum is empty
-    int32_t walk;                // MODE_EXP_DIRECT: exp_walk_item applies
+    int32_t walk;                // MODE_EXP_DIRECT, MODE_RECT_GENERIC: exp_walk_kernel's or
+                                 // rect_step_kernel's, not the generic kernel's
     int64_t etab_off;            // MODE_EXP_FAST: doubles, [n_seg + INIT_PARTS][7][N_tau]
     uint32_t o_t0, o_t0Band, o_tau, o_tauBand;  // caller's window (posterior modes)
 };
@@ -814,8 +817,8 @@ __device__ void finish_item(Reducer<BTSG, NCOLS> &red, int wave, int lane, const
     const int tid = threadIdx.x;
     const float M = fmaxf(fmaxf(sh_M[0], sh_M[1]), fmaxf(sh_M[2], sh_M[3]));
     if (BTSG) {
-        const int n = it.cb * TILE_COLS + tid;
-        if (n < (int)td.N_tau) {
+        const int n = it.cb * td.tile + tid;
+        if (tid < td.tile && n < (int)td.N_tau) {
             float S = 0.0f;
 #pragma unroll
             for (int w = 0; w < 4; w++)
@@ -1204,6 +1207,230 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 }
 
 // ----------------------------------------------------------------------------
+// rectangular window, any steps without wrap-around
+// ----------------------------------------------------------------------------
+//
+// Row m starts at t0 + m dt0 + TAtom/2 - t_min = TAtom q + phi, column n lasts
+// tau + n dtau = TAtom Q + R, and (rect.cu:21-31, 54-69; nothing wraps, so the
+// ends grow with n and no running maximum is needed)
+//   i = min(q, N-1),   j = min(max(q + Q + [phi + R >= TAtom], 1), N) >= i,
+// a compare and an add with carry per cell.  The item's range of prefix entries
+// is staged in LDS where it fits: entry e at e*7 + (e >> pad) doubles, pad the
+// lanes' stride of entries if that is even, rounded down to a power of two, so
+// that the lanes' reads spread over the banks; wider steps read the table in
+// place.  A lane owns the columns lane, + 64, + 128, + 192 of the block (as many
+// as the block has groups of 64) and a wave 4 rows at a time, whose starts are read through the scalar cache.
+//
+// Bound: VALU issue and latency together (63 instructions a cell, 24 of them
+// FP64; 69% of the cycles issue, at ~3 waves a SIMD).  128 templates of 1000 to
+// 4000 bins, steps of 2 and 3 bins, 37e6 cells: maps 192 us with the generic
+// kernel (an integer division and an uncoalesced 56-byte read a cell), 90 us
+// so, 210 us with these indices but the table read in place.
+// rows per item at most and items aimed at, untuned
+// Rows per item at most and items aimed at, untuned (the maps below: 64 rows
+// 100 us, 32 rows 110, 96 rows 115, all with 256 columns an item).
+constexpr int STEP_RB = 64;
+constexpr int64_t STEP_ITEMS = 1024;
+// Bytes of staged range per item.  The widest of 256, 128 and 64 columns whose
+// range stays below the first figure (four workgroups a CU or more), else 64
+// columns if that stays below the second, else 256 read from the table (the
+// maps below at 20, 28, 36 and 52 KB: 112, 95, 94 and 100 us).
+constexpr int STEP_LDS_AIM = 36 << 10;
+constexpr int STEP_LDS_MOST = 76 << 10;
+
+// x / TAtom and x % TAtom: the product with the reciprocal is at most one short
+__device__ __forceinline__ uint32_t div_TA(uint32_t x, const TmplDev &td, uint32_t &rem) {
+    uint32_t q = __umulhi(x, td.TA_rcp);
+    rem = x - q * td.TAtom;
+    const bool more = rem >= td.TAtom;
+    rem -= more ? td.TAtom : 0;
+    return q + more;
+}
+
+struct StepShape {
+    int entries;  // staged prefix entries of an item at most
+    int pad;
+};
+__host__ __device__ __forceinline__ StepShape step_shape(int rb, int tile, uint32_t N_tau,
+                                                         uint32_t dt0, uint32_t dtau,
+                                                         uint32_t TA) {
+    const uint32_t nc = N_tau < (uint32_t)tile ? N_tau : (uint32_t)tile;
+    const uint64_t span = ((uint64_t)(rb - 1) * dt0 + (uint64_t)(nc - 1) * dtau) / TA + 3;
+    StepShape sh;
+    sh.entries = span < (1u << 20) ? (int)span : 1 << 20;
+    const uint32_t b = dtau / TA;
+    sh.pad = 31;
+    if (b > 0 && b % 2 == 0 && dtau % TA == 0)
+        for (sh.pad = 0; 2u << sh.pad <= b; sh.pad++) {
+        }
+    return sh;
+}
+__host__ __device__ __forceinline__ int step_bytes(const StepShape &sh) {
+    return (sh.entries * NC + (sh.entries >> sh.pad) + 1) * (int)sizeof(double);
+}
+__host__ __device__ __forceinline__ bool step_in_lds(const StepShape &sh) {
+    return step_bytes(sh) <= STEP_LDS_MOST;
+}
+// dynamic LDS of an item: the rows' references and sums, and the staged range
+// (none if it does not fit) or the final reduction in its place
+__host__ __device__ __forceinline__ int step_lds(int rb, const StepShape &sh) {
+    const int range = step_in_lds(sh) ? step_bytes(sh) : 0;
+    return rb * 2 * (int)sizeof(float) + (range < (int)sizeof(FinShared) ? (int)sizeof(FinShared) : range);
+}
+
+template <bool BTSG, bool STRICT, bool LDS, int C>
+__device__ __forceinline__ void rect_step_item(const TmplDev &td, const ItemDev &it,
+                                               int64_t item_id, const double *__restrict__ P,
+                                               float *__restrict__ Ft, ItemPart *ipart,
+                                               float *rowpart, float *colpart, int *flags,
+                                               double *lds) {
+    const int RB = td.rb_rows;
+    const int row0 = it.rb * RB;
+    const int col0 = it.cb * td.tile;
+    const int N_t0 = (int)td.N_t0, N_tau = (int)td.N_tau;
+    const int N = (int)td.N;
+    const uint32_t TA = td.TAtom, dt0 = td.dt0, dtau = td.dtau;
+    const StepShape sh = step_shape(RB, td.tile, td.N_tau, dt0, dtau, TA);
+    float *sh_rowM = reinterpret_cast<float *>(lds);
+    float *sh_rowS = sh_rowM + RB;
+    lds += RB;
+    const uint32_t T0 = td.t0 + TA / 2 - td.t_min;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    auto clamp_j = [&](int j) { return min(max(j, 1), N); };
+    int jb = 0;  // entry in LDS slot 0
+    if (LDS) {
+        const uint32_t Tr = T0 + (uint32_t)row0 * dt0;
+        const uint32_t Tl = T0 + (uint32_t)min(row0 + RB - 1, N_t0 - 1) * dt0;
+        const uint32_t xf = td.tau + (uint32_t)col0 * dtau;
+        const uint32_t xl = td.tau + (uint32_t)min(col0 + td.tile - 1, N_tau - 1) * dtau;
+        uint32_t rem;
+        jb = clamp_j((int)(div_TA(Tr, td, rem) + div_TA(xf, td, rem)));
+        const int nw = (clamp_j((int)(div_TA(Tl, td, rem) + div_TA(xl, td, rem) + 1)) - jb + 1) * NC;
+        const double *__restrict__ src = P + (int64_t)jb * NC;
+        for (int k0 = threadIdx.x; k0 < nw; k0 += 8 * WG) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (k0 + u * WG < nw) v[u] = src[k0 + u * WG];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int k = k0 + u * WG;
+                if (k < nw) lds[k + ((k / NC) >> sh.pad)] = v[u];
+            }
+        }
+    }
+    int colidx[C], Q[C];
+    uint32_t R[C], voff[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        colidx[c] = col0 + c * 64 + lane;
+        const bool valid = colidx[c] < N_tau;
+        const uint32_t x = td.tau + (uint32_t)(valid ? colidx[c] : col0) * dtau;
+        Q[c] = (int)div_TA(x, td, R[c]) - jb;
+        voff[c] = valid ? (uint32_t)colidx[c] * 4u : 0x80000000u;
+    }
+    const bool cols_full = col0 + 64 * C <= N_tau;
+    const uint32_t rowb = (uint32_t)N_tau * (uint32_t)sizeof(float);
+    const uint32_t dq = dt0 / TA, dphi = dt0 % TA;
+    Reducer<BTSG, C> red;
+    red.init();
+    bool single = false;
+    __syncthreads();
+    for (int s = 0; s < RB / 16; s++) {
+        const int rl0 = s * 16 + wave * 4;
+        const int m0 = row0 + rl0;
+        if (m0 >= N_t0) break;
+        const int nvr = min(N_t0 - m0, 4);
+        uint32_t phi;
+        uint32_t q = div_TA(T0 + (uint32_t)m0 * dt0, td, phi);
+        float F[4][C];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            // (rows past the map repeat the last one: their entries are staged)
+            if (r > 0 && r < nvr) {
+                phi += dphi;
+                q += dq + (phi >= TA);
+                phi -= phi >= TA ? TA : 0;
+            }
+            const int i = min((int)q, N - 1);
+            double Pi[NC];
+#pragma unroll
+            for (int k = 0; k < NC; k++) Pi[k] = P[(int64_t)i * NC + k];
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                const int j = min(max((int)q + Q[c] + (R[c] >= TA - phi), 1 - jb), N - jb);
+                double w[NC];
+                if (LDS) {
+                    const double *e = lds + (__umul24(j, NC) + (j >> sh.pad));
+#pragma unroll
+                    for (int k = 0; k < NC; k++) w[k] = e[k];
+                } else {
+                    const double *e = P + (int64_t)j * NC;
+#pragma unroll
+                    for (int k = 0; k < NC; k++) w[k] = e[k];
+                }
+                F[r][c] = cell_F(w[0] - Pi[0], w[1] - Pi[1], w[2] - Pi[2], w[3] - Pi[3],
+                                 w[4] - Pi[4], w[5] - Pi[5], w[6] - Pi[6]);
+                // i_t1 == i_t0 (i_t1 = j - 1)
+                if (STRICT) single |= j + jb - 1 == i && r < nvr && colidx[c] < N_tau;
+            }
+        }
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            Ft + (int64_t)m0 * N_tau, (short)0, (int)((uint32_t)nvr * rowb), BUF_RSRC_WORD3);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int c = 0; c < C; c++)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F[r][c]), rs, (int)voff[c],
+                                                      (int)(r * rowb), 0);
+        if (!cols_full || nvr < 4) {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int c = 0; c < C; c++)
+                    F[r][c] = r < nvr && colidx[c] < N_tau ? F[r][c] : -INFINITY;
+        }
+        red.add(F, m0, colidx, N_tau, lane, rl0, sh_rowM, sh_rowS);
+    }
+    if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
+    wave_argmax(red.best, red.bidx);
+    __syncthreads();  // the staged range is consumed: the final reduction reuses it
+    finish_item(red, wave, lane, td, it, item_id, min(RB, N_t0 - row0), ipart, rowpart, colpart,
+                sh_rowM, sh_rowS, *reinterpret_cast<FinShared *>(lds),
+                [](int ln, int c) { return c * 64 + ln; });
+}
+
+template <bool BTSG, bool STRICT>
+__global__ __launch_bounds__(WG) void rect_step_kernel(
+    const TmplDev *__restrict__ tds, const ItemDev *__restrict__ items, int64_t item0,
+    const double *__restrict__ prefix, float *__restrict__ Fout,
+    ItemPart *__restrict__ ipart, float *__restrict__ rowpart,
+    float *__restrict__ colpart, int *__restrict__ flags) {
+    extern __shared__ double lds_raw[];  // one dynamic LDS symbol per file
+    const int64_t item_id = item0 + block_slot();
+    const ItemDev it = items[item_id];
+    const TmplDev td = tds[it.t];
+    if (!td.walk) return;  // block-uniform: a rect_generic_kernel item
+    const int groups = (min((int)td.tile, (int)td.N_tau - it.cb * td.tile) + 63) / 64;
+#define STEP_ITEM(lds, cols)                                                                  \
+    rect_step_item<BTSG, STRICT, lds, cols>(td, it, item_id, prefix + td.prefix_off,           \
+                                            Fout + td.F_off, ipart, rowpart, colpart, flags, \
+                                            lds_raw)
+    if (!step_in_lds(step_shape(td.rb_rows, td.tile, td.N_tau, td.dt0, td.dtau, td.TAtom)))
+        STEP_ITEM(false, 4);
+    else if (groups == 4)
+        STEP_ITEM(true, 4);
+    else if (groups == 3)
+        STEP_ITEM(true, 3);
+    else if (groups == 2)
+        STEP_ITEM(true, 2);
+    else
+        STEP_ITEM(true, 1);
+#undef STEP_ITEM
+}
+
+// ----------------------------------------------------------------------------
 // generic per-cell kernels (rect with exact wrap-around semantics; exp)
 // ----------------------------------------------------------------------------
 //
@@ -1245,6 +1472,7 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
     const int64_t item_id = item0 + block_slot();
     const ItemDev it = items[item_id];
     const TmplDev td = tds[it.t];
+    if (td.walk) return;  // block-uniform: a rect_step_kernel item
     const int RB = td.rb_rows;
     const int row0 = it.rb * RB;
     const int col0 = it.cb * TILE_COLS;
@@ -2677,7 +2905,7 @@ __global__ __launch_bounds__(NT) void finalize_kernel(
                 }
             }
             if (i < (int)td.N_tau) {  // column i: [rowblk][N_tau]
-                const int cb = i / TILE_COLS;
+                const int cb = i / td.tile;
                 const float *cp = colpart + td.colpart_off + i;
                 auto term = [&](uint32_t rb) {
                     return (double)(cp[(int64_t)rb * td.N_tau] *
@@ -2836,7 +3064,9 @@ struct tcw_plan {
     int max_lds_bytes = 0;  // rect_fast_kernel dynamic LDS
     int max_lds_expf = 0;   // exp_fast_kernel dynamic LDS
     int max_lds_walk = 0;   // exp_walk_kernel dynamic LDS
-    int64_t walk_tmpls = 0, direct_tmpls = 0;  // MODE_EXP_DIRECT templates of either kernel
+    int max_lds_step = 0;   // rect_step_kernel dynamic LDS
+    int64_t walk_tmpls = 0, direct_tmpls = 0;   // MODE_EXP_DIRECT templates of either kernel
+    int64_t step_tmpls = 0, generic_tmpls = 0;  // MODE_RECT_GENERIC templates of either kernel
     DevBuf d_tmpl, d_segs, d_items, d_prefix, d_merged, d_ipart, d_rowpart, d_colpart,
         d_flags, d_seg_items, d_col_items, d_etab, d_exp_tmpls, d_init_items;
     hipGraphExec_t graph = nullptr;
@@ -2867,7 +3097,8 @@ struct tcw_plan {
         max_lds_bytes = 0;
         max_lds_expf = 0;
         max_lds_walk = 0;
-        walk_tmpls = direct_tmpls = 0;
+        max_lds_step = 0;
+        walk_tmpls = direct_tmpls = step_tmpls = generic_tmpls = 0;
         if (graph) (void)hipGraphExecDestroy(graph);
         graph = nullptr;
     }
@@ -3024,6 +3255,7 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     td.seg_end = seg_end;
     td.N = N;
     td.TAtom = TAtom;
+    td.TA_rcp = 0xffffffffu / TAtom;
     td.t_min = t_min;
     td.type = w.type;
     td.t0 = w.t0;
@@ -3070,8 +3302,9 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         const uint64_t x_hi = (uint64_t)w.t0 + w.t0Band + w.tau + w.tauBand + half;
         // (rows of at most 2^20 cells: partial sub-tiles store by 32-bit byte
         // offsets within their four rows)
-        if (!(p.flags & TCW_FLAG_GENERIC) && regular && x_lo >= t_min && x_hi < (1ull << 32) &&
-            N_tau <= (int64_t)1 << 20) {
+        td.walk = !(p.flags & TCW_FLAG_GENERIC) && x_lo >= t_min && x_hi < (1ull << 32) &&
+                  N_tau <= (int64_t)1 << 20;
+        if (td.walk && regular) {
             mode = MODE_RECT_FAST;
             td.a = (int32_t)(w.dt0 / TAtom);
             td.q0 = (int32_t)(((uint64_t)w.t0 - t_min + half) / TAtom);
@@ -3081,14 +3314,15 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     td.mode = mode;
     const int req = p.rows_req[mode];  // the plan's tuned rows, 0 = built-in choice
     int rb = req > 0 ? req : RB_DEFAULT[mode];
-    if (mode == MODE_RECT_FAST && req <= 0) {
+    if ((mode == MODE_RECT_FAST || (mode == MODE_RECT_GENERIC && td.walk)) && req <= 0) {
         // few or small maps (the single-map call): fewer rows per item, so
         // that the batch's items cover the CUs (about SMALL_BATCH_ITEMS of them
         // if the templates are alike)
+        const int most = mode == MODE_RECT_FAST ? RB_DEFAULT[mode] : STEP_RB;
         const double ncb = (double)((N_tau + TILE_COLS - 1) / TILE_COLS);
-        const double want = (double)N_t0 * ncb * (double)p.T / (double)SMALL_BATCH_ITEMS;
-        rb = want >= RB_DEFAULT[mode] ? RB_DEFAULT[mode]
-                                      : std::max(16, ((int)std::ceil(want) + 15) / 16 * 16);
+        const double want = (double)N_t0 * ncb * (double)p.T /
+                            (double)(mode == MODE_RECT_FAST ? SMALL_BATCH_ITEMS : STEP_ITEMS);
+        rb = want >= most ? most : std::max(16, ((int)std::ceil(want) + 15) / 16 * 16);
     }
     if (mode == MODE_EXP_DIRECT && td.walk && req <= 0) {
         // enough items for the chip, and otherwise long ones: each starts with
@@ -3113,7 +3347,15 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         rb = (int)std::min<int64_t>(rb, (N_t0 + 15) / 16 * 16);
     td.rb_rows = rb;
     td.n_rowblk = (uint32_t)((N_t0 + rb - 1) / rb);
-    td.n_colblk = (uint32_t)((N_tau + TILE_COLS - 1) / TILE_COLS);
+    td.tile = TILE_COLS;
+    if (mode == MODE_RECT_GENERIC && td.walk) {
+        auto bytes = [&](int tile) {
+            return step_bytes(step_shape(rb, tile, td.N_tau, td.dt0, td.dtau, TAtom));
+        };
+        while (td.tile > 64 && bytes(td.tile) > STEP_LDS_AIM) td.tile /= 2;
+        if (bytes(td.tile) > STEP_LDS_MOST) td.tile = TILE_COLS;
+    }
+    td.n_colblk = (uint32_t)((N_tau + td.tile - 1) / td.tile);
     if (mode == MODE_EXP_DIRECT || mode == MODE_EXP_FAST) {
         td.mode = mode;  // exp_table_bins reads it
         if (mode == MODE_EXP_FAST) {
@@ -3180,6 +3422,14 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     for (uint32_t rbk = 0; rbk < td.n_rowblk; rbk++)
         for (uint32_t cbk = 0; cbk < td.n_colblk; cbk++)
             items_by_mode[mode].push_back(ItemDev{(int32_t)t, (int32_t)rbk, (int32_t)cbk, 0});
+    if (mode == MODE_RECT_GENERIC && td.walk) {
+        p.max_lds_step = std::max(
+            p.max_lds_step,
+            step_lds(rb, step_shape(rb, td.tile, td.N_tau, td.dt0, td.dtau, TAtom)));
+        p.step_tmpls++;
+    } else if (mode == MODE_RECT_GENERIC) {
+        p.generic_tmpls++;
+    }
     if (mode == MODE_RECT_FAST) {
         // the widest column block (the first) and the last one
         const int last = (int)N_tau - (int)(td.n_colblk - 1) * TILE_COLS;
@@ -3335,17 +3585,23 @@ void launch_maps(tcw_plan &p, float *F, hipStream_t st) {
         hipLaunchKernelGGL((rect_fast_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG),
                            p.max_lds_bytes, st, tds, items, p.mode_begin[MODE_RECT_FAST],
                            prefix, F, ipart, rowpart, colpart, flags);
-    if ((n = p.mode_begin[MODE_RECT_GENERIC + 1] - p.mode_begin[MODE_RECT_GENERIC]) > 0)
-        hipLaunchKernelGGL((rect_generic_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG), 0,
-                           st, tds, items, p.mode_begin[MODE_RECT_GENERIC], prefix, F, ipart,
-                           rowpart, colpart, flags);
+    // the items of a mode lie template by template: where two kernels share a
+    // mode, each leaves the other's items at once
+    if ((n = p.mode_begin[MODE_RECT_GENERIC + 1] - p.mode_begin[MODE_RECT_GENERIC]) > 0) {
+        if (p.step_tmpls > 0)
+            hipLaunchKernelGGL((rect_step_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG),
+                               p.max_lds_step, st, tds, items, p.mode_begin[MODE_RECT_GENERIC],
+                               prefix, F, ipart, rowpart, colpart, flags);
+        if (p.generic_tmpls > 0)
+            hipLaunchKernelGGL((rect_generic_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG), 0,
+                               st, tds, items, p.mode_begin[MODE_RECT_GENERIC], prefix, F, ipart,
+                               rowpart, colpart, flags);
+    }
     if ((n = p.mode_begin[MODE_EXP_FAST + 1] - p.mode_begin[MODE_EXP_FAST]) > 0)
         hipLaunchKernelGGL((exp_fast_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG),
                            p.max_lds_expf, st, tds, items, p.mode_begin[MODE_EXP_FAST], merged,
                            (const double *)p.d_etab.p, F, ipart, rowpart, colpart, flags,
                            p.max_lds_expf > 0 ? 1 : 0);
-    // the items of a mode lie template by template: each kernel leaves the
-    // other's at once
     if ((n = p.mode_begin[MODE_EXP_DIRECT + 1] - p.mode_begin[MODE_EXP_DIRECT]) > 0) {
         if (p.walk_tmpls > 0)
             hipLaunchKernelGGL((exp_walk_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WALK_WG),
