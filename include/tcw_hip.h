@@ -122,6 +122,15 @@ int tcw_map(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win,
  * copy per device, held from library load until the process ends). */
 #define TCW_NOALLOC_SCRATCH_BYTES (32u << 20)
 
+/* tcw_map from host atoms: atoms->ts and atoms->cols are HOST arrays (cols
+ * [7][col_stride] with col_stride = the atom count det_off[numDet]), sent with
+ * the map's descriptors in one copy.  F_mn_host (host, may be NULL) receives the
+ * map as well.  The pinned staging memory belongs to the handle (at most 20 MiB;
+ * more data than that goes unstaged).  Returns when everything is done. */
+int tcw_map_host(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win,
+                 float *F_mn_dev, float *F_mn_host, tcw_stats *stats, uint32_t flags,
+                 void *stream);
+
 /* tcw_map without any device or pinned-memory allocation.  No counterpart in
  * the reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The same

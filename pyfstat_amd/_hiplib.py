@@ -42,6 +42,7 @@ EXPORTED_SYMBOLS = (
     "tcw_create",
     "tcw_destroy",
     "tcw_map",
+    "tcw_map_host",
     "tcw_map_noalloc",
     "tcw_batch_plan",
     "tcw_batch_plan_rows",
@@ -193,6 +194,8 @@ def load():
     lib.tcw_destroy.argtypes = [vp]
     lib.tcw_map.restype = ctypes.c_int
     lib.tcw_map.argtypes = [vp, P(Atoms), P(Window), vp, P(Stats), ctypes.c_uint32, vp]
+    lib.tcw_map_host.restype = ctypes.c_int
+    lib.tcw_map_host.argtypes = [vp, P(Atoms), P(Window), vp, vp, P(Stats), ctypes.c_uint32, vp]
     lib.tcw_map_noalloc.restype = ctypes.c_int
     lib.tcw_map_noalloc.argtypes = [vp, P(Atoms), P(Window), vp, vp, ctypes.c_uint32, vp]
     lib.tcw_batch_plan.restype = ctypes.c_int

@@ -215,8 +215,9 @@ class BatchedTransientMaps:
 
     def stats(self):
         """Per-template statistics as a numpy structured array (synchronises)."""
-        raw = self.stats_d.cpu().numpy()
-        st = raw.view(STATS_DTYPE).copy()
+        # (a copy of its own already: a copy of the structured view would go
+        # field by field)
+        st = self.stats_d.cpu().numpy().view(STATS_DTYPE)
         if self.lal_strict and np.any(st["single_atom"]):
             bad = int(np.nonzero(st["single_atom"])[0][0])
             raise _hiplib.SingleAtomError(

@@ -3043,6 +3043,39 @@ using tcwc::set_device;
 
 }  // namespace
 
+// Host data on its way to the device for one call: gathered in pinned memory and
+// sent by one copy into one device buffer, of which the destinations are
+// views.  Grow-only up to HOST_STAGE_MAX; the caller waits for the stream
+// before the next use.
+constexpr size_t HOST_STAGE_MAX = 16u << 20;
+struct HostStage {
+    char *pin = nullptr;
+    size_t cap = 0;
+    DevBuf dev;
+    int ensure(size_t bytes) {
+        const int rc = ensure_pin(bytes);
+        return rc ? rc : dev.ensure(bytes);
+    }
+    int ensure_pin(size_t bytes) {
+        if (bytes > cap) {
+            if (pin) (void)hipHostFree(pin);
+            pin = nullptr;
+            cap = 0;
+            if (hipHostMalloc((void **)&pin, bytes, hipHostMallocDefault) != hipSuccess) {
+                pin = nullptr;
+                return fail(TCW_ERR_NOMEM, "hipHostMalloc of " + std::to_string(bytes) + " bytes failed");
+            }
+            cap = bytes;
+        }
+        return TCW_OK;
+    }
+    ~HostStage() {
+        if (pin) (void)hipHostFree(pin);
+        dev.release();
+    }
+};
+constexpr size_t stage_align(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
 struct tcw_plan {
     int device = 0;
     uint32_t flags = 0;
@@ -3078,6 +3111,12 @@ struct tcw_plan {
     int64_t g_cstride = -1;
     // rows per work item requested for each kernel mode (0: built-in choice)
     int32_t rows_req[MODE_COUNT] = {0, 0, 0, 0};
+    // when set, the descriptors (and ts / cols, if host_ts) go through it in one copy
+    HostStage *stage = nullptr;
+    const uint32_t *host_ts = nullptr;  // n_host_atoms timestamps
+    const float *host_cols = nullptr;   // [7][n_host_atoms]
+    int64_t n_host_atoms = 0;
+    DevBuf d_ts, d_cols;                // views of the stage's device buffer
     // when set, device buffers are views into this memory (tcw_map_noalloc)
     char *arena = nullptr;
     size_t arena_bytes = 0;
@@ -3122,6 +3161,8 @@ struct tcw_plan {
         d_init_items.release();
         d_etab.release();
         d_exp_tmpls.release();
+        d_ts.release();
+        d_cols.release();
     }
 };
 
@@ -3130,12 +3171,13 @@ struct tcw_plan {
 struct tcw_handle {
     int device = 0;
     tcw_plan single;
+    HostStage single_in;   // the single plan's descriptors and host atoms
+    HostStage single_out;  // a small map on its way to the caller (pin only)
     tcw_plan noalloc;  // tcw_map_noalloc: buffers are views into the static scratch
-    tcw_stats *d_stats = nullptr;
-    tcw_stats *h_stats = nullptr;  // pinned
+    tcw_stats *h_stats = nullptr;  // pinned, written by the last kernel
+    tcw_stats *d_stats = nullptr;  // its device address
     DevBuf d_mtab, d_mseg, d_msegs;  // tcw_merge_batch tables
     ~tcw_handle() {
-        if (d_stats) (void)hipFree(d_stats);
         if (h_stats) (void)hipHostFree(h_stats);
         d_mtab.release();
         d_mseg.release();
@@ -3480,7 +3522,44 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
         }
     }
     p.mode_begin[MODE_COUNT] = (int64_t)p.items.size();
+    struct Up {
+        DevBuf *buf;
+        const void *src;
+        size_t bytes;
+    };
+    std::vector<Up> ups = {
+        {&p.d_tmpl, p.tmpl.data(), sizeof(TmplDev) * p.tmpl.size()},
+        {&p.d_segs, p.segs.data(), sizeof(SegDev) * p.segs.size()},
+        {&p.d_items, p.items.data(), sizeof(ItemDev) * p.items.size()},
+        {&p.d_seg_items, p.seg_items.data(), sizeof(ItemDev) * p.seg_items.size()},
+        {&p.d_col_items, p.col_items.data(), sizeof(ItemDev) * p.col_items.size()},
+        {&p.d_init_items, p.init_items.data(), sizeof(ItemDev) * p.init_items.size()},
+        {&p.d_exp_tmpls, p.exp_tmpls.data(), sizeof(int32_t) * p.exp_tmpls.size()},
+    };
+    if (p.host_ts) {
+        ups.push_back({&p.d_ts, p.host_ts, sizeof(uint32_t) * (size_t)p.n_host_atoms});
+        ups.push_back({&p.d_cols, p.host_cols, sizeof(float) * NC * (size_t)p.n_host_atoms});
+    }
+    // one copy instead of one per table (each costs ~4 us of launch and, from
+    // pageable memory, ~4 us of a staging kernel on the stream)
+    size_t staged = 0;
+    for (const Up &u : ups) staged += stage_align(std::max<size_t>(u.bytes, 1));
+    const bool one_copy = p.stage && async && staged <= HOST_STAGE_MAX;
     int rc = TCW_OK;
+    if (one_copy) {
+        if ((rc = p.stage->ensure(staged))) return rc;
+        size_t off = 0;
+        for (const Up &u : ups) {
+            const size_t a = stage_align(std::max<size_t>(u.bytes, 1));
+            if (u.bytes) std::memcpy(p.stage->pin + off, u.src, u.bytes);
+            u.buf->set_view((char *)p.stage->dev.p + off, a);
+            off += a;
+        }
+        TCW_HIP_TRY(hipMemcpyAsync(p.stage->dev.p, p.stage->pin, staged, hipMemcpyHostToDevice, st));
+    } else {
+        for (const Up &u : ups)  // views of an earlier call
+            if (u.buf->view) u.buf->release();
+    }
     if (p.arena) {
         // carve every buffer out of the caller-provided arena (no allocation)
         size_t off = 0;
@@ -3499,18 +3578,13 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
         });
         if (rc) return rc;
     }
-    auto up = [&](void *dst, const void *src, size_t bytes) -> hipError_t {
-        if (bytes == 0) return hipSuccess;
-        return async ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st)
-                     : hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
-    };
-    TCW_HIP_TRY(up(p.d_tmpl.p, p.tmpl.data(), sizeof(TmplDev) * p.tmpl.size()));
-    TCW_HIP_TRY(up(p.d_segs.p, p.segs.data(), sizeof(SegDev) * p.segs.size()));
-    TCW_HIP_TRY(up(p.d_items.p, p.items.data(), sizeof(ItemDev) * p.items.size()));
-    TCW_HIP_TRY(up(p.d_seg_items.p, p.seg_items.data(), sizeof(ItemDev) * p.seg_items.size()));
-    TCW_HIP_TRY(up(p.d_col_items.p, p.col_items.data(), sizeof(ItemDev) * p.col_items.size()));
-    TCW_HIP_TRY(up(p.d_init_items.p, p.init_items.data(), sizeof(ItemDev) * p.init_items.size()));
-    TCW_HIP_TRY(up(p.d_exp_tmpls.p, p.exp_tmpls.data(), sizeof(int32_t) * p.exp_tmpls.size()));
+    if (one_copy) return TCW_OK;
+    for (const Up &u : ups) {
+        if (u.bytes == 0) continue;
+        if ((rc = u.buf->ensure(u.bytes))) return rc;
+        TCW_HIP_TRY(async ? hipMemcpyAsync(u.buf->p, u.src, u.bytes, hipMemcpyHostToDevice, st)
+                          : hipMemcpy(u.buf->p, u.src, u.bytes, hipMemcpyHostToDevice));
+    }
     return TCW_OK;
 }
 
@@ -3780,8 +3854,9 @@ int tcw_create(int device, tcw_handle **out) {
     auto *h = new tcw_handle;
     h->device = device;
     noalloc_scratch_setup(device);  // with `device` current
-    if (hipMalloc(&h->d_stats, sizeof(tcw_stats)) != hipSuccess ||
-        hipHostMalloc(&h->h_stats, sizeof(tcw_stats), hipHostMallocDefault) != hipSuccess) {
+    h->single.stage = &h->single_in;
+    if (hipHostMalloc(&h->h_stats, sizeof(tcw_stats), hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&h->d_stats, h->h_stats, 0) != hipSuccess) {
         delete h;
         return fail(TCW_ERR_NOMEM, "tcw_create: stats slot allocation failed");
     }
@@ -3946,6 +4021,56 @@ int plan_single(tcw_handle *h, tcw_plan &p, const tcw_atoms *atoms, const tcw_wi
     return plan_build(p, h->device, &d, flags, nullptr, st, true);
 }
 
+// A map on its way to the host goes through pinned memory up to this size (the
+// map's copy then shares the call's one wait); larger ones are copied
+// afterwards, straight to the caller's memory.
+constexpr size_t HOST_OUT_MAX = 4u << 20;
+
+// tcw_map (host = false) and tcw_map_host (the atoms' ts and cols, and F_host
+// if given, in host memory); returns with the stream drained.
+int map_single(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win, float *F_dev,
+               float *F_host, tcw_stats *stats, uint32_t flags, hipStream_t st, bool host,
+               const char *who) {
+    tcw_plan &p = h->single;
+    p.host_ts = nullptr;
+    if (host && atoms->numDet >= 1 && atoms->numDet <= TCW_MAX_DETECTORS && atoms->ts && atoms->cols) {
+        const int64_t n = atoms->det_off[atoms->numDet];
+        if (n < 1 || atoms->col_stride != n)
+            return fail(TCW_ERR_INVALID, std::string(who) + ": host columns must be [7][atoms]");
+        p.host_ts = atoms->ts;
+        p.host_cols = atoms->cols;
+        p.n_host_atoms = n;
+    }
+    int rc = plan_single(h, p, atoms, win, flags, st, who);
+    if (!rc)
+        rc = launch_all(p, host ? (const uint32_t *)p.d_ts.p : atoms->ts,
+                        host ? (const float *)p.d_cols.p : atoms->cols, atoms->col_stride, F_dev,
+                        h->d_stats, st);
+    size_t out = 0;
+    if (!rc && F_host) {
+        out = sizeof(float) * (size_t)p.F_total;
+        if (out > HOST_OUT_MAX) out = 0;
+        if (out && !(rc = h->single_out.ensure_pin(out)) &&
+            hipMemcpyAsync(h->single_out.pin, F_dev, out, hipMemcpyDeviceToHost, st) != hipSuccess)
+            rc = fail(TCW_ERR_DEVICE, std::string(who) + ": copying the map failed");
+    }
+    // (also after a failure: the staged copy may still be reading)
+    const hipError_t e = hipStreamSynchronize(st);
+    if (rc) return rc;
+    TCW_HIP_TRY(e);
+    *stats = *h->h_stats;
+    if (out)
+        std::memcpy(F_host, h->single_out.pin, out);
+    else if (F_host)
+        TCW_HIP_TRY(hipMemcpy(F_host, F_dev, sizeof(float) * (size_t)p.F_total,
+                              hipMemcpyDeviceToHost));
+    if ((flags & TCW_FLAG_LAL_STRICT) && stats->single_atom)
+        return fail(TCW_ERR_SINGLE_ATOM,
+                    "encountered a single-atom Fstat-calculation. This is degenerate and cannot "
+                    "be computed! t0 must stay away *at least* 2*TAtom from the end of the data.");
+    return TCW_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -3954,21 +4079,16 @@ int tcw_map(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win, float 
             tcw_stats *stats, uint32_t flags, void *stream) {
     if (!h || !atoms || !win || !F_mn_dev || !stats)
         return fail(TCW_ERR_INVALID, "tcw_map: null argument");
-    hipStream_t st = (hipStream_t)stream;
-    int rc = plan_single(h, h->single, atoms, win, flags, st, "tcw_map");
-    if (rc) return rc;
-    rc = launch_all(h->single, atoms->ts, atoms->cols, atoms->col_stride, F_mn_dev,
-                    h->d_stats, st);
-    if (rc) return rc;
-    TCW_HIP_TRY(hipMemcpyAsync(h->h_stats, h->d_stats, sizeof(tcw_stats),
-                               hipMemcpyDeviceToHost, st));
-    TCW_HIP_TRY(hipStreamSynchronize(st));
-    *stats = *h->h_stats;
-    if ((flags & TCW_FLAG_LAL_STRICT) && stats->single_atom)
-        return fail(TCW_ERR_SINGLE_ATOM,
-                    "encountered a single-atom Fstat-calculation. This is degenerate and cannot "
-                    "be computed! t0 must stay away *at least* 2*TAtom from the end of the data.");
-    return TCW_OK;
+    return map_single(h, atoms, win, F_mn_dev, nullptr, stats, flags, (hipStream_t)stream, false,
+                      "tcw_map");
+}
+
+int tcw_map_host(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win, float *F_mn_dev,
+                 float *F_mn_host, tcw_stats *stats, uint32_t flags, void *stream) {
+    if (!h || !atoms || !win || !F_mn_dev || !stats)
+        return fail(TCW_ERR_INVALID, "tcw_map_host: null argument");
+    return map_single(h, atoms, win, F_mn_dev, F_mn_host, stats, flags, (hipStream_t)stream, true,
+                      "tcw_map_host");
 }
 
 int tcw_map_noalloc(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win,

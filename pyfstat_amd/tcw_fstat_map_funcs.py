@@ -352,13 +352,6 @@ def _check_window_type(windowRange):
         )
 
 
-def _upload_packed(packed, dev):
-    torch = _torch()
-    ts = torch.from_numpy(packed.ts.view(np.int32)).to(dev, non_blocking=False)
-    cols = torch.from_numpy(packed.cols).to(dev, non_blocking=False)
-    return ts, cols
-
-
 def _map_from_stats(F_mn, st, BtSG):
     FstatMap = pyTransientFstatMap.__new__(pyTransientFstatMap)
     FstatMap.F_mn = F_mn
@@ -395,13 +388,13 @@ def hip_compute_transient_fstat_map(multiFstatAtoms, windowRange, BtSG=False,
     _hiplib.check(lib.tcw_map_shape(packed.num_binned, packed.TAtom, packed.t_min,
                                     ctypes.byref(win), ctypes.byref(nt0), ctypes.byref(ntau)),
                   "tcw_map_shape")
-    ts_d, cols_d = _upload_packed(packed, dev)
     F_d = torch.empty((nt0.value, ntau.value), dtype=torch.float32, device=dev)
+    F_h = None if return_device else np.empty((nt0.value, ntau.value), dtype=np.float32)
     at = _hiplib.Atoms()
     at.numDet = packed.numDet
     at.TAtom = packed.TAtom
-    at.ts = ts_d.data_ptr()
-    at.cols = cols_d.data_ptr()
+    at.ts = packed.ts.ctypes.data
+    at.cols = packed.cols.ctypes.data
     at.col_stride = packed.cols.shape[1]
     for X in range(packed.numDet + 1):
         at.det_off[X] = int(packed.det_off[X])
@@ -416,10 +409,12 @@ def hip_compute_transient_fstat_map(multiFstatAtoms, windowRange, BtSG=False,
         flags |= _hiplib.TCW_FLAG_GENERIC
     st = _hiplib.Stats()
     stream = torch.cuda.current_stream(dev).cuda_stream
-    _hiplib.check(lib.tcw_map(handle, ctypes.byref(at), ctypes.byref(win),
-                              ctypes.c_void_p(F_d.data_ptr()), ctypes.byref(st), flags,
-                              ctypes.c_void_p(stream)), "tcw_map")
-    F_mn = F_d if return_device else F_d.cpu().numpy()
+    _hiplib.check(lib.tcw_map_host(handle, ctypes.byref(at), ctypes.byref(win),
+                                   ctypes.c_void_p(F_d.data_ptr()),
+                                   None if F_h is None else ctypes.c_void_p(F_h.ctypes.data),
+                                   ctypes.byref(st), flags, ctypes.c_void_p(stream)),
+                  "tcw_map_host")
+    F_mn = F_d if return_device else F_h
     FstatMap = _map_from_stats(F_mn, st, BtSG)
     logger.debug(
         "Done computing transient F-stat map. maxF={:.4f}, t0_ML={}, tau_ML={}".format(
