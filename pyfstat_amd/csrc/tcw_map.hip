@@ -2753,115 +2753,130 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // finalize: per-template stats from the partials
 // ----------------------------------------------------------------------------
 
-template <int NT>
-__device__ double block_sum_d(double v) {
-    __shared__ double sd[NT / 64];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) sd[wave] = v;
-    __syncthreads();
-    double s = 0.0;
-    for (int w = 0; w < NT / 64; w++) s += sd[w];
-    __syncthreads();
-    return s;
-}
-
 constexpr int FIN_SCALE_CAP = 4096;        // per-item scale factors kept in LDS
-constexpr int64_t FIN_WIDE_MAX_T = 256;  // batches smaller than this finalize with 1024 threads
+// Batches smaller than this finalize with 1024 threads (1024 templates with
+// 1024 threads each: 125 x 125 cells 17 us, 250-2000 rows and columns 40-46 us;
+// with 256 threads 9.5 and 39).
+constexpr int64_t FIN_WIDE_MAX_T = 256;
+// Partials of a row or column loaded together (1024 templates of 250 to 2000
+// rows and columns: 66 us one by one, 50 by 4, 43 by 8, 39 by 12).
+constexpr int FIN_AHEAD = 12;
 
-// Block-wide: argmax (first index on ties) of (bv, bi) and maximum of mm.
-template <int NT>
-__device__ void block_argmax_max(float &bv, int &bi, float &mm) {
-    __shared__ float sv[NT / 64], sm[NT / 64];
-    __shared__ int si[NT / 64];
-    wave_argmax(bv, bi);
-    mm = wave_max(mm);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) {
-        sv[wave] = bv;
-        si[wave] = bi;
-        sm[wave] = mm;
-    }
-    __syncthreads();
-    bv = sv[0];
-    bi = si[0];
-    mm = sm[0];
-    for (int w = 1; w < NT / 64; w++) {
-        argmax_merge(bv, bi, sv[w], si[w]);
-        mm = fmaxf(mm, sm[w]);
-    }
-    __syncthreads();
+// FP64 values across the wave without LDS, as wave_sum and wave_max do for
+// floats: every lane ends with the same bits.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// Block-wide argmax over doubles (first index on ties) of two pairs at once.
-template <int NT>
-__device__ void block_argmax2_d(double &av, int &ai, double &bv, int &bi) {
-    __shared__ double sav[NT / 64], sbv[NT / 64];
-    __shared__ int sai[NT / 64], sbi[NT / 64];
-    auto merge = [](double &v, int &i, double ov, int oi) {
-        if (ov > v || (ov == v && oi < i)) {
-            v = ov;
-            i = oi;
-        }
+template <typename Op>
+__device__ __forceinline__ double wave_reduce_d(double v, Op op) {
+    v = op(v, dpp_d<DPP_QUAD_XOR1>(v));
+    v = op(v, dpp_d<DPP_QUAD_XOR2>(v));
+    v = op(v, dpp_d<DPP_ROW_ROR4>(v));
+    v = op(v, dpp_d<DPP_ROW_ROR8>(v));
+    auto both = [](unsigned lo, unsigned hi) {
+        return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
     };
+    {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+        const auto l = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32),
+                                                        false, false);
+        v = op(both(l[0], h[0]), both(l[1], h[1]));
+    }
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const auto l = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false,
+                                                    false);
+    return op(both(l[0], h[0]), both(l[1], h[1]));
+}
+
+__device__ __forceinline__ double wave_sum_d(double v) {
+    return wave_reduce_d(v, [](double a, double b) { return a + b; });
+}
+
+// Wave argmax of doubles (none NaN), the first index on ties.
+__device__ __forceinline__ void wave_argmax_d(double &v, int &i) {
+    const double m = wave_reduce_d(v, [](double a, double b) { return a > b ? a : b; });
+    i = wave_min_idx(v == m ? i : 0x7fffffff);
+    v = m;
+}
+
+// The sum, in order, of the partials p[0], p[stride], ... (count of them), each
+// times its item's scale, of a row or column; FIN_AHEAD loads in flight.
+template <typename Scale>
+__device__ __forceinline__ double partial_sum(const float *__restrict__ p, uint32_t count,
+                                              uint32_t stride, Scale scale) {
+    double sum = 0.0;
+    for (uint32_t b = 0; b < count; b += FIN_AHEAD) {
+        float x[FIN_AHEAD];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const double oa = __shfl_xor(av, o), ob = __shfl_xor(bv, o);
-        const int oai = __shfl_xor(ai, o), obi = __shfl_xor(bi, o);
-        merge(av, ai, oa, oai);
-        merge(bv, bi, ob, obi);
+        for (uint32_t u = 0; u < FIN_AHEAD; u++)  // (a repeated load past the end, not added)
+            x[u] = p[(int64_t)min(b + u, count - 1) * stride];
+#pragma unroll
+        for (uint32_t u = 0; u < FIN_AHEAD; u++)
+            if (b + u < count) sum += (double)(x[u] * scale(b + u));
     }
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) {
-        sav[wave] = av;
-        sai[wave] = ai;
-        sbv[wave] = bv;
-        sbi[wave] = bi;
-    }
-    __syncthreads();
-    av = sav[0];
-    ai = sai[0];
-    bv = sbv[0];
-    bi = sbi[0];
-    for (int w = 1; w < NT / 64; w++) {
-        merge(av, ai, sav[w], sai[w]);
-        merge(bv, bi, sbv[w], sbi[w]);
-    }
-    __syncthreads();
+    return sum;
 }
 
 // One workgroup of NT threads per template (NT = 1024 for small batches, whose
-// maps are large, 256 otherwise).  Three block reductions: the argmax of F
-// with the largest item reference Mref (log2 units), the lnBtSG sum, and the
-// two posterior argmaxes together.  Item k's partials are relative to
-// 2^(M_k) (M_k = -inf: no valid cell, partials 0), rescaled here by
-// exp((M_k - Mref) / LOG2E) <= 1, so no item reference needs maxF; the row
-// and column partials of a thread are read in one pass.
+// maps are large, 256 otherwise): the argmax of F with the largest item
+// reference Mref (log2 units), then the lnBtSG sum and the two posterior
+// argmaxes.  Item k's partials are relative to 2^(M_k) (M_k = -inf: no valid
+// cell, partials 0), rescaled here by exp((M_k - Mref) / LOG2E) <= 1, so no
+// item reference needs maxF; the row and column partials of a thread are read
+// in one pass.
+//
+// Bound: latency -- the descriptor, the items, three barriers, and each
+// thread's partials (2000 x 2000 cells at 192 rows an item are 8 passes of 8 +
+// 11 loads).  The reductions go through DPP; with pairwise exchanges through
+// LDS and partials read one by one: 128 maps of 250 to 1000 rows 16 us, now
+// 10; one map of 47 x 46 cells 10, now 5; 1024 maps of 250 to 2000 rows 66, now
+// 39.
 template <bool BTSG, int NT>
 __global__ __launch_bounds__(NT) void finalize_kernel(
     const TmplDev *__restrict__ tds, const ItemPart *__restrict__ ipart,
     const float *__restrict__ rowpart, const float *__restrict__ colpart,
     const int *__restrict__ flags, tcw_stats *__restrict__ stats) {
+    constexpr int NW = NT / 64;
     __shared__ float sh_scale[FIN_SCALE_CAP];
-    // the wide variant (few, large maps: many partials per row and column)
-    // unrolls the partial sums by 8 so their independent loads issue
-    // together; the narrow one (many templates) is faster as the compiler
-    // schedules it by itself
-    constexpr bool FIN_UNROLL = NT >= 1024;
+    __shared__ float sh_max[NW], sh_M[NW];
+    __shared__ int sh_idx[NW];
+    __shared__ double sh_sum[NW], sh_row[NW], sh_colv[NW];
+    __shared__ int sh_ri[NW], sh_ci[NW];
     constexpr double INV_LOG2E = 1.0 / (double)LOG2E;
     const int t = blockIdx.x;
     const TmplDev td = tds[t];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     const int64_t nitems = (int64_t)td.n_rowblk * td.n_colblk;
     const ItemPart *ip = ipart + td.item_begin;
     float bv = -INFINITY, Mref = -INFINITY;
     int bi = 0x7fffffff;
+    ItemPart first{-INFINITY, 0x7fffffff, -INFINITY, 0.0f};
     for (int64_t k = threadIdx.x; k < nitems; k += NT) {
         const ItemPart q = ip[k];
+        if (k < NT) first = q;  // the only one unless the template has over NT items
         argmax_merge(bv, bi, q.maxF, q.idx);
         Mref = fmaxf(Mref, q.M);
     }
-    block_argmax_max<NT>(bv, bi, Mref);
+    wave_argmax(bv, bi);
+    Mref = wave_max(Mref);
+    if (lane == 0) {
+        sh_max[wave] = bv;
+        sh_idx[wave] = bi;
+        sh_M[wave] = Mref;
+    }
+    __syncthreads();
+    bv = lane < NW ? sh_max[lane] : -INFINITY;
+    bi = lane < NW ? sh_idx[lane] : 0x7fffffff;
+    Mref = wave_max(lane < NW ? sh_M[lane] : -INFINITY);
+    wave_argmax(bv, bi);
     const float maxF = bv;
     const int64_t m_ML = bi / (int)td.N_tau;
     const int64_t n_ML = bi - m_ML * (int64_t)td.N_tau;
@@ -2869,20 +2884,21 @@ __global__ __launch_bounds__(NT) void finalize_kernel(
     double lnB = NAN, t0_MP = NAN, tau_MP = NAN;
     int64_t m_MP = -1, n_MP = -1;
     if (BTSG) {
-        auto item_scale = [&](int64_t k) -> float {
-            const float Mk = ip[k].M;
+        auto item_scale = [&](float Mk) -> float {
             return Mk == -INFINITY ? 0.0f : __expf((float)((double)(Mk - Mref) * INV_LOG2E));
         };
         double s = 0.0;
         for (int64_t k = threadIdx.x; k < nitems; k += NT) {
-            const float sc = item_scale(k);
+            const float Mk = k < NT ? first.M : ip[k].M, Sk = k < NT ? first.S : ip[k].S;
+            const float sc = item_scale(Mk);
             if (k < FIN_SCALE_CAP) sh_scale[k] = sc;
-            s += (double)ip[k].S * (double)sc;
+            s += (double)Sk * (double)sc;
         }
-        s = block_sum_d<NT>(s);  // contains a barrier: sh_scale is complete
-        lnB = log(70.0 / ((double)td.N_t0 * (double)td.N_tau)) + (double)Mref * INV_LOG2E + log(s);
-        auto scale = [&](int64_t k) -> float {
-            return k < FIN_SCALE_CAP ? sh_scale[k] : item_scale(k);
+        s = wave_sum_d(s);
+        if (lane == 0) sh_sum[wave] = s;
+        __syncthreads();  // sh_scale and sh_sum are complete
+        auto scale = [&](uint32_t k) -> float {
+            return k < FIN_SCALE_CAP ? sh_scale[k] : item_scale(ip[k].M);
         };
         double rv = -1.0, cv = -1.0;
         int ri = 0x7fffffff, ci = 0x7fffffff;
@@ -2890,34 +2906,14 @@ __global__ __launch_bounds__(NT) void finalize_kernel(
         for (int i = threadIdx.x; i < nmax; i += NT) {
             double R = -1.0, Cs = -1.0;
             if (i < (int)td.N_t0) {  // row i: [colblk][N_t0]
-                const int rb = i / td.rb_rows;
-                const float *rp = rowpart + td.rowpart_off + i;
-                auto term = [&](uint32_t cb) {
-                    return (double)(rp[(int64_t)cb * td.N_t0] *
-                                    scale((int64_t)rb * td.n_colblk + cb));
-                };
-                R = 0.0;
-                if constexpr (FIN_UNROLL) {
-#pragma unroll 8
-                    for (uint32_t cb = 0; cb < td.n_colblk; cb++) R += term(cb);
-                } else {
-                    for (uint32_t cb = 0; cb < td.n_colblk; cb++) R += term(cb);
-                }
+                const uint32_t k0 = (uint32_t)(i / td.rb_rows) * td.n_colblk;
+                R = partial_sum(rowpart + td.rowpart_off + i, td.n_colblk, td.N_t0,
+                                [&](uint32_t cb) { return scale(k0 + cb); });
             }
             if (i < (int)td.N_tau) {  // column i: [rowblk][N_tau]
-                const int cb = i / td.tile;
-                const float *cp = colpart + td.colpart_off + i;
-                auto term = [&](uint32_t rb) {
-                    return (double)(cp[(int64_t)rb * td.N_tau] *
-                                    scale((int64_t)rb * td.n_colblk + cb));
-                };
-                Cs = 0.0;
-                if constexpr (FIN_UNROLL) {
-#pragma unroll 8
-                    for (uint32_t rb = 0; rb < td.n_rowblk; rb++) Cs += term(rb);
-                } else {
-                    for (uint32_t rb = 0; rb < td.n_rowblk; rb++) Cs += term(rb);
-                }
+                const uint32_t cb = (uint32_t)(i / td.tile);
+                Cs = partial_sum(colpart + td.colpart_off + i, td.n_rowblk, td.N_tau,
+                                 [&](uint32_t rb) { return scale(rb * td.n_colblk + cb); });
             }
             if (R > rv) {  // i grows within a thread: the first maximum stays
                 rv = R;
@@ -2928,7 +2924,24 @@ __global__ __launch_bounds__(NT) void finalize_kernel(
                 ci = i;
             }
         }
-        block_argmax2_d<NT>(rv, ri, cv, ci);
+        wave_argmax_d(rv, ri);
+        wave_argmax_d(cv, ci);
+        if (lane == 0) {
+            sh_row[wave] = rv;
+            sh_ri[wave] = ri;
+            sh_colv[wave] = cv;
+            sh_ci[wave] = ci;
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        rv = lane < NW ? sh_row[lane] : -1.0;
+        ri = lane < NW ? sh_ri[lane] : 0x7fffffff;
+        cv = lane < NW ? sh_colv[lane] : -1.0;
+        ci = lane < NW ? sh_ci[lane] : 0x7fffffff;
+        wave_argmax_d(rv, ri);
+        wave_argmax_d(cv, ci);
+        s = wave_sum_d(lane < NW ? sh_sum[lane] : 0.0);
+        lnB = log(70.0 / ((double)td.N_t0 * (double)td.N_tau)) + (double)Mref * INV_LOG2E + log(s);
         m_MP = ri;
         n_MP = ci;
         t0_MP = (double)td.o_t0 + ((double)m_MP + 0.5) * ((double)td.o_t0Band / (double)td.N_t0);
