@@ -233,6 +233,15 @@ int tcw_merge_batch(tcw_handle *h, const tcw_batch_desc *desc, const uint32_t *t
                     int64_t merged_stride, int64_t *m_off, uint32_t *t_data,
                     int64_t *atom_bin, void *stream);
 
+/* The same merge for repeated runs: the plan holds the tables (shapes to m_off
+ * and t_data as above), a run only launches, asynchronously on `stream`. */
+typedef struct tcw_merge_plan tcw_merge_plan;
+int tcw_merge_plan_create(tcw_handle *h, const tcw_batch_desc *desc, tcw_merge_plan **out,
+                          int64_t *m_off, uint32_t *t_data);
+int tcw_merge_plan_destroy(tcw_merge_plan *p);
+int tcw_merge_run(tcw_merge_plan *p, const uint32_t *ts, const float *cols, int64_t col_stride,
+                  float *merged, int64_t merged_stride, int64_t *atom_bin, void *stream);
+
 /* out[c*out_stride + j] = in[c*in_stride + atom_bin[j]] for the 7 columns and
  * j < n_atoms: the adjoint of the merge (each atom's gradient is that of its
  * bin).  Asynchronous on `stream`. */

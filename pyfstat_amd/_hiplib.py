@@ -52,6 +52,9 @@ EXPORTED_SYMBOLS = (
     "tcw_batch_run_timed",
     "tcw_plan_destroy",
     "tcw_merge_batch",
+    "tcw_merge_plan_create",
+    "tcw_merge_plan_destroy",
+    "tcw_merge_run",
     "tcw_gather_bins",
     "tcw_refine_plan_create",
     "tcw_refine_plan_destroy",
@@ -215,6 +218,12 @@ def load():
     i64 = ctypes.c_int64
     lib.tcw_merge_batch.restype = ctypes.c_int
     lib.tcw_merge_batch.argtypes = [vp, P(BatchDesc), vp, vp, i64, vp, i64, vp, vp, vp, vp]
+    lib.tcw_merge_plan_create.restype = ctypes.c_int
+    lib.tcw_merge_plan_create.argtypes = [vp, P(BatchDesc), P(vp), vp, vp]
+    lib.tcw_merge_plan_destroy.restype = ctypes.c_int
+    lib.tcw_merge_plan_destroy.argtypes = [vp]
+    lib.tcw_merge_run.restype = ctypes.c_int
+    lib.tcw_merge_run.argtypes = [vp, vp, vp, i64, vp, i64, vp, vp]
     lib.tcw_gather_bins.restype = ctypes.c_int
     lib.tcw_gather_bins.argtypes = [vp, i64, vp, i64, vp, i64, vp]
     lib.tcw_refine_plan_create.restype = ctypes.c_int

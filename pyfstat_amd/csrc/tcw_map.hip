@@ -2978,57 +2978,103 @@ struct MergeTmpl {
     uint32_t N, t_min;
 };
 
-// One thread per merged bin: per detector segment a binary search for the
-// bin's first atom, then float32 sums over the bin's atoms, detectors in
-// order -- the accumulation order of mergeMultiFstatAtomsBinned, so the
-// result is bit-identical to the stage kernel's merge.
-__global__ __launch_bounds__(256) void merge_kernel(
+// A workgroup owns MERGE_BINS consecutive bins of one template.  Per detector a
+// block-wide search bounds the block's atoms; chunk by chunk their bins are
+// formed, the first atom of every bin is marked where the bin changes, and each
+// thread sums the atoms of its bins, MERGE_WG apart, so that the lanes' reads of
+// the columns and the stores are nearly and exactly consecutive.  Float32 sums,
+// detectors in order, atoms in order -- the accumulation order of
+// mergeMultiFstatAtomsBinned, so the result is bit-identical to the stage
+// kernel's merge.  atom_bin[k] = out_off + (ts[k] - t_min) / TA of every atom is
+// written by the blocks in equal shares of the atoms.
+// Bound: HBM bytes -- 32 an atom in, 28 a bin and 8 an atom out.  512 templates
+// of 2 x 1844 atoms: 33 us with a binary search of the timestamps per bin and
+// 7 for the atoms' bins in a kernel of its own, 25 together so (4.2 TB/s).
+constexpr int MERGE_WG = 256;
+constexpr int MERGE_PER = 4;                      // bins and atoms of a thread
+constexpr int MERGE_BINS = MERGE_WG * MERGE_PER;  // bins per block, atoms per chunk
+
+__global__ __launch_bounds__(MERGE_WG) void merge_kernel(
     const MergeTmpl *__restrict__ mt, const SegDev *__restrict__ segs, int64_t T,
     const uint32_t *__restrict__ ts, const float *__restrict__ cols, int64_t cstride,
-    uint32_t TA, float *__restrict__ out, int64_t ostride) {
+    uint32_t TA, float *__restrict__ out, int64_t ostride, int64_t *__restrict__ atom_bin) {
+    __shared__ int s_bin[MERGE_BINS], s_first[MERGE_BINS];
+    __shared__ int64_t s_rng[2][2];
+    __shared__ int s_cnt[4];
+    const int tid = threadIdx.x;
     for (int64_t t = blockIdx.y; t < T; t += gridDim.y) {
         const MergeTmpl m = mt[t];
-        const uint32_t b = blockIdx.x * 256u + threadIdx.x;
-        if (b >= m.N) continue;
-        float v[NC];
+        const uint32_t B0 = blockIdx.x * (uint32_t)MERGE_BINS;
+        if (B0 >= m.N) continue;  // block-uniform
+        const int nb = (int)min(m.N - B0, (uint32_t)MERGE_BINS);
+        const int64_t blocks = ((int64_t)m.N + MERGE_BINS - 1) / MERGE_BINS;  // of the template
+        const uint64_t t_lo = (uint64_t)m.t_min + (uint64_t)B0 * TA;
+        const uint64_t t_hi = t_lo + (uint64_t)nb * TA;
+        float v[MERGE_PER][NC];
 #pragma unroll
-        for (int c = 0; c < NC; c++) v[c] = 0.0f;
-        const uint64_t t_lo = (uint64_t)m.t_min + (uint64_t)b * TA, t_hi = t_lo + TA;
+        for (int j = 0; j < MERGE_PER; j++)
+#pragma unroll
+            for (int c = 0; c < NC; c++) v[j][c] = 0.0f;
         for (int64_t s = m.seg_begin; s < m.seg_end; s++) {
             const SegDev sg = segs[s];
-            int64_t lo = sg.begin, hi = sg.end;
-            while (lo < hi) {
-                const int64_t mid = (lo + hi) >> 1;
-                if ((uint64_t)ts[mid] < t_lo)
-                    lo = mid + 1;
-                else
-                    hi = mid;
-            }
-            for (int64_t k = lo; k < sg.end && (uint64_t)ts[k] < t_hi; k++) {
+            block_lower_bound2(ts, sg.begin, sg.end, t_lo, t_hi, s_rng, s_cnt);
+            const int64_t ka = s_rng[0][0], kb = s_rng[1][0];
+            for (int64_t c0 = ka; c0 < kb; c0 += MERGE_BINS) {  // block-uniform
+                const int na = (int)min((int64_t)MERGE_BINS, kb - c0);
+                int bin[MERGE_PER];
 #pragma unroll
-                for (int c = 0; c < NC; c++) v[c] += cols[c * cstride + k];
+                for (int j = 0; j < MERGE_PER; j++) {
+                    const int i = j * MERGE_WG + tid;
+                    bin[j] = i < na ? (int)((ts[c0 + i] - (uint32_t)t_lo) / TA) : MERGE_BINS;
+                    s_bin[i] = bin[j];
+                    s_first[i] = -1;
+                }
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < MERGE_PER; j++) {
+                    const int i = j * MERGE_WG + tid;
+                    if ((unsigned)bin[j] < (unsigned)MERGE_BINS && (i == 0 || s_bin[i - 1] != bin[j]))
+                        s_first[bin[j]] = i;
+                }
+                __syncthreads();
+                const float *__restrict__ col = cols + c0;
+                int k[MERGE_PER];
+                float x[MERGE_PER][NC];  // the bins' first atoms, all loads in flight
+#pragma unroll
+                for (int j = 0; j < MERGE_PER; j++) {
+                    k[j] = s_first[j * MERGE_WG + tid];
+#pragma unroll
+                    for (int c = 0; c < NC; c++) x[j][c] = col[c * cstride + max(k[j], 0)];
+                }
+#pragma unroll
+                for (int j = 0; j < MERGE_PER; j++) {
+                    if (k[j] < 0) continue;
+#pragma unroll
+                    for (int c = 0; c < NC; c++) v[j][c] += x[j][c];
+                    for (int q = k[j] + 1; q < na && s_bin[q] == j * MERGE_WG + tid; q++) {
+#pragma unroll
+                        for (int c = 0; c < NC; c++) v[j][c] += col[c * cstride + q];
+                    }
+                }
+                __syncthreads();  // bins consumed before the next chunk
             }
+            if (atom_bin)  // the block's share of the detector's atoms
+                for (int64_t k = sg.begin + B0 + tid; k < sg.end; k += blocks * MERGE_BINS)
+#pragma unroll
+                    for (int j = 0; j < MERGE_PER; j++)
+                        if (k + j * MERGE_WG < sg.end)
+                            atom_bin[k + j * MERGE_WG] =
+                                m.out_off + (int64_t)((ts[k + j * MERGE_WG] - m.t_min) / TA);
+            __syncthreads();  // s_rng is rewritten by the next detector
         }
 #pragma unroll
-        for (int c = 0; c < NC; c++) out[c * ostride + m.out_off + b] = v[c];
-    }
-}
-
-// atom_bin[k] = out_off + (ts[k] - t_min) / TA for every atom of every segment;
-// segment s of template t is blockIdx.y-strided, atoms over x.
-struct MergeSeg {
-    int64_t begin, end, out_off;
-    uint32_t t_min, pad;
-};
-
-__global__ __launch_bounds__(256) void atom_bin_kernel(const MergeSeg *__restrict__ ms,
-                                                       int64_t S, const uint32_t *__restrict__ ts,
-                                                       uint32_t TA, int64_t *__restrict__ atom_bin) {
-    for (int64_t s = blockIdx.y; s < S; s += gridDim.y) {
-        const MergeSeg g = ms[s];
-        for (int64_t k = g.begin + (int64_t)blockIdx.x * 256 + threadIdx.x; k < g.end;
-             k += (int64_t)gridDim.x * 256)
-            atom_bin[k] = g.out_off + (int64_t)((ts[k] - g.t_min) / TA);
+        for (int j = 0; j < MERGE_PER; j++) {
+            const int b = j * MERGE_WG + tid;
+            if (b < nb) {
+#pragma unroll
+                for (int c = 0; c < NC; c++) out[c * ostride + m.out_off + B0 + b] = v[j][c];
+            }
+        }
     }
 }
 
@@ -3189,11 +3235,10 @@ struct tcw_handle {
     tcw_plan noalloc;  // tcw_map_noalloc: buffers are views into the static scratch
     tcw_stats *h_stats = nullptr;  // pinned, written by the last kernel
     tcw_stats *d_stats = nullptr;  // its device address
-    DevBuf d_mtab, d_mseg, d_msegs;  // tcw_merge_batch tables
+    DevBuf d_mtab, d_msegs;  // tcw_merge_batch tables
     ~tcw_handle() {
         if (h_stats) (void)hipHostFree(h_stats);
         d_mtab.release();
-        d_mseg.release();
         d_msegs.release();
     }
 };
@@ -4004,6 +4049,100 @@ int tcw_plan_destroy(tcw_plan *p) {
 
 namespace {
 
+// The tables of a batched merge.
+struct MergeTables {
+    int64_t T = 0, total = 0, maxN = 0, max_end = 0;
+    uint32_t TAtom = 0;
+    std::vector<MergeTmpl> tmpl;
+    std::vector<SegDev> segs;
+};
+
+int merge_tables(const tcw_batch_desc *d, MergeTables &tab, int64_t *m_off, uint32_t *t_data) {
+    if (d->T <= 0) return fail(TCW_ERR_INVALID, "no templates");
+    if (d->TAtom < 2) return fail(TCW_ERR_INVALID, "TAtom must be at least 2 seconds.");
+    tab.T = d->T;
+    tab.TAtom = d->TAtom;
+    tab.tmpl.resize((size_t)d->T);
+    int64_t off = 0;
+    for (int64_t t = 0; t < d->T; t++) {
+        const int64_t s0 = d->seg_begin[t], s1 = d->seg_begin[t + 1];
+        if (s1 <= s0 || s1 - s0 > TCW_MAX_DETECTORS)
+            return fail(TCW_ERR_INVALID, "template " + std::to_string(t) + ": needs 1.." +
+                                             std::to_string(TCW_MAX_DETECTORS) +
+                                             " detector segments");
+        uint32_t tmin = 0xffffffffu, tmax = 0;
+        for (int64_t s = s0; s < s1; s++) {
+            if (d->seg_off[s + 1] <= d->seg_off[s])
+                return fail(TCW_ERR_INVALID, "template " + std::to_string(t) + ": empty detector");
+            if (d->seg_tlast[s] < d->seg_tfirst[s])
+                return fail(TCW_ERR_INVALID, "template " + std::to_string(t) +
+                                                 ": timestamps not in ascending order");
+            tmin = std::min(tmin, d->seg_tfirst[s]);
+            tmax = std::max(tmax, d->seg_tlast[s]);
+        }
+        const int64_t N = (int64_t)((tmax - tmin) / d->TAtom) + 1;
+        tab.tmpl[(size_t)t] = MergeTmpl{(int64_t)tab.segs.size(),
+                                        (int64_t)tab.segs.size() + (s1 - s0), off, (uint32_t)N, tmin};
+        for (int64_t s = s0; s < s1; s++) {
+            tab.segs.push_back(SegDev{d->seg_off[s], d->seg_off[s + 1]});
+            tab.max_end = std::max(tab.max_end, d->seg_off[s + 1]);
+        }
+        m_off[t] = off;
+        t_data[t] = tmin;
+        off += N;
+        tab.maxN = std::max(tab.maxN, N);
+    }
+    m_off[d->T] = tab.total = off;
+    return TCW_OK;
+}
+
+int merge_check(const MergeTables &tab, int64_t col_stride, int64_t merged_stride) {
+    if (merged_stride < tab.total)
+        return fail(TCW_ERR_INVALID, "merged_stride " + std::to_string(merged_stride) +
+                                         " < merged bins " + std::to_string(tab.total));
+    if (col_stride < tab.max_end)
+        return fail(TCW_ERR_INVALID, "col_stride smaller than the atom count");
+    return TCW_OK;
+}
+
+int merge_upload(const MergeTables &tab, DevBuf &d_tab, DevBuf &d_segs) {
+    int rc;
+    if ((rc = d_tab.ensure(tab.tmpl.size() * sizeof(MergeTmpl))) ||
+        (rc = d_segs.ensure(tab.segs.size() * sizeof(SegDev))))
+        return rc;
+    TCW_HIP_TRY(hipMemcpy(d_tab.p, tab.tmpl.data(), tab.tmpl.size() * sizeof(MergeTmpl),
+                          hipMemcpyHostToDevice));
+    TCW_HIP_TRY(hipMemcpy(d_segs.p, tab.segs.data(), tab.segs.size() * sizeof(SegDev),
+                          hipMemcpyHostToDevice));
+    return TCW_OK;
+}
+
+int merge_launch(const MergeTables &tab, const DevBuf &d_tab, const DevBuf &d_segs,
+                 const uint32_t *ts, const float *cols, int64_t col_stride, float *merged,
+                 int64_t merged_stride, int64_t *atom_bin, hipStream_t st) {
+    const unsigned gy = (unsigned)std::min<int64_t>(tab.T, 65535);
+    hipLaunchKernelGGL(merge_kernel, dim3((unsigned)((tab.maxN + MERGE_BINS - 1) / MERGE_BINS), gy),
+                       dim3(MERGE_WG), 0, st, (const MergeTmpl *)d_tab.p, (const SegDev *)d_segs.p,
+                       tab.T, ts, cols, col_stride, tab.TAtom, merged, merged_stride, atom_bin);
+    TCW_HIP_TRY(hipGetLastError());
+    return TCW_OK;
+}
+
+}  // namespace
+
+// The tables of a merge that is run many times, on the device.
+struct tcw_merge_plan {
+    int device = 0;
+    MergeTables tab;  // sizes only
+    DevBuf d_tab, d_segs;
+    ~tcw_merge_plan() {
+        d_tab.release();
+        d_segs.release();
+    }
+};
+
+namespace {
+
 // One template as a batch of one (tcw_map and tcw_map_noalloc): checks the
 // atoms and plans `p` on `st` (descriptor uploads queued on `st`).
 int plan_single(tcw_handle *h, tcw_plan &p, const tcw_atoms *atoms, const tcw_window *win,
@@ -4124,82 +4263,61 @@ int tcw_map_noalloc(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win
                       stats_dev, st);
 }
 
+int tcw_merge_plan_create(tcw_handle *h, const tcw_batch_desc *d, tcw_merge_plan **out,
+                          int64_t *m_off, uint32_t *t_data) {
+    if (!h || !d || !out || !m_off || !t_data)
+        return fail(TCW_ERR_INVALID, "tcw_merge_plan_create: null argument");
+    MergeTables tab;
+    int rc = merge_tables(d, tab, m_off, t_data);
+    if (rc) return rc;
+    if ((rc = set_device(h->device))) return rc;
+    auto *p = new tcw_merge_plan;
+    p->device = h->device;
+    rc = merge_upload(tab, p->d_tab, p->d_segs);
+    if (rc) {
+        delete p;
+        return rc;
+    }
+    tab.tmpl.clear();
+    tab.segs.clear();
+    p->tab = tab;
+    *out = p;
+    return TCW_OK;
+}
+
+int tcw_merge_plan_destroy(tcw_merge_plan *p) {
+    if (p) (void)set_device(p->device);
+    delete p;
+    return TCW_OK;
+}
+
+int tcw_merge_run(tcw_merge_plan *p, const uint32_t *ts, const float *cols, int64_t col_stride,
+                  float *merged, int64_t merged_stride, int64_t *atom_bin, void *stream) {
+    if (!p || !ts || !cols || !merged)
+        return fail(TCW_ERR_INVALID, "tcw_merge_run: null argument");
+    int rc = merge_check(p->tab, col_stride, merged_stride);
+    if (rc || (rc = set_device(p->device))) return rc;
+    return merge_launch(p->tab, p->d_tab, p->d_segs, ts, cols, col_stride, merged, merged_stride,
+                        atom_bin, (hipStream_t)stream);
+}
+
 int tcw_merge_batch(tcw_handle *h, const tcw_batch_desc *d, const uint32_t *ts,
                     const float *cols, int64_t col_stride, float *merged, int64_t merged_stride,
                     int64_t *m_off, uint32_t *t_data, int64_t *atom_bin, void *stream) {
     if (!h || !d || !m_off || !t_data) return fail(TCW_ERR_INVALID, "tcw_merge_batch: null argument");
-    if (d->T <= 0) return fail(TCW_ERR_INVALID, "no templates");
-    if (d->TAtom < 2) return fail(TCW_ERR_INVALID, "TAtom must be at least 2 seconds.");
-    std::vector<MergeTmpl> tab((size_t)d->T);
-    std::vector<SegDev> segs;
-    std::vector<MergeSeg> mseg;
-    int64_t off = 0, maxN = 0;
-    for (int64_t t = 0; t < d->T; t++) {
-        const int64_t s0 = d->seg_begin[t], s1 = d->seg_begin[t + 1];
-        if (s1 <= s0 || s1 - s0 > TCW_MAX_DETECTORS)
-            return fail(TCW_ERR_INVALID, "template " + std::to_string(t) + ": needs 1.." +
-                                             std::to_string(TCW_MAX_DETECTORS) +
-                                             " detector segments");
-        uint32_t tmin = 0xffffffffu, tmax = 0;
-        for (int64_t s = s0; s < s1; s++) {
-            if (d->seg_off[s + 1] <= d->seg_off[s])
-                return fail(TCW_ERR_INVALID, "template " + std::to_string(t) + ": empty detector");
-            if (d->seg_tlast[s] < d->seg_tfirst[s])
-                return fail(TCW_ERR_INVALID, "template " + std::to_string(t) +
-                                                 ": timestamps not in ascending order");
-            tmin = std::min(tmin, d->seg_tfirst[s]);
-            tmax = std::max(tmax, d->seg_tlast[s]);
-        }
-        const int64_t N = (int64_t)((tmax - tmin) / d->TAtom) + 1;
-        tab[(size_t)t] = MergeTmpl{(int64_t)segs.size(), (int64_t)segs.size() + (s1 - s0), off,
-                                   (uint32_t)N, tmin};
-        for (int64_t s = s0; s < s1; s++) {
-            segs.push_back(SegDev{d->seg_off[s], d->seg_off[s + 1]});
-            mseg.push_back(MergeSeg{d->seg_off[s], d->seg_off[s + 1], off, tmin, 0});
-        }
-        m_off[t] = off;
-        t_data[t] = tmin;
-        off += N;
-        maxN = std::max(maxN, N);
-    }
-    m_off[d->T] = off;
+    MergeTables tab;
+    int rc = merge_tables(d, tab, m_off, t_data);
+    if (rc) return rc;
     if (!merged) return TCW_OK;
     if (!ts || !cols) return fail(TCW_ERR_INVALID, "tcw_merge_batch: null atoms");
-    if (merged_stride < off)
-        return fail(TCW_ERR_INVALID, "merged_stride " + std::to_string(merged_stride) +
-                                         " < merged bins " + std::to_string(off));
-    int64_t max_end = 0;
-    for (const auto &g : segs) max_end = std::max(max_end, g.end);
-    if (col_stride < max_end) return fail(TCW_ERR_INVALID, "col_stride smaller than the atom count");
-    int rc = set_device(h->device);
-    if (rc) return rc;
-    if ((rc = h->d_mtab.ensure(tab.size() * sizeof(MergeTmpl))) ||
-        (rc = h->d_msegs.ensure(segs.size() * sizeof(SegDev))) ||
-        (rc = h->d_mseg.ensure(mseg.size() * sizeof(MergeSeg))))
-        return rc;
+    if ((rc = merge_check(tab, col_stride, merged_stride)) || (rc = set_device(h->device))) return rc;
     hipStream_t st = (hipStream_t)stream;
     // the previous call's kernels may still read the tables
     TCW_HIP_TRY(hipStreamSynchronize(st));
-    TCW_HIP_TRY(hipMemcpy(h->d_mtab.p, tab.data(), tab.size() * sizeof(MergeTmpl),
-                          hipMemcpyHostToDevice));
-    TCW_HIP_TRY(hipMemcpy(h->d_msegs.p, segs.data(), segs.size() * sizeof(SegDev),
-                          hipMemcpyHostToDevice));
-    TCW_HIP_TRY(hipMemcpy(h->d_mseg.p, mseg.data(), mseg.size() * sizeof(MergeSeg),
-                          hipMemcpyHostToDevice));
-    const unsigned gy = (unsigned)std::min<int64_t>(d->T, 65535);
-    hipLaunchKernelGGL(merge_kernel, dim3((unsigned)((maxN + 255) / 256), gy), dim3(256), 0, st,
-                       (const MergeTmpl *)h->d_mtab.p, (const SegDev *)h->d_msegs.p, d->T, ts,
-                       cols, col_stride, d->TAtom, merged, merged_stride);
-    if (atom_bin) {
-        int64_t maxS = 0;
-        for (const auto &g : mseg) maxS = std::max(maxS, g.end - g.begin);
-        const unsigned sy = (unsigned)std::min<size_t>(mseg.size(), 65535);
-        const unsigned sx = (unsigned)std::min<int64_t>((maxS + 255) / 256, 1024);
-        hipLaunchKernelGGL(atom_bin_kernel, dim3(sx, sy), dim3(256), 0, st,
-                           (const MergeSeg *)h->d_mseg.p, (int64_t)mseg.size(), ts, d->TAtom,
-                           atom_bin);
-    }
-    TCW_HIP_TRY(hipGetLastError());
+    if ((rc = merge_upload(tab, h->d_mtab, h->d_msegs)) ||
+        (rc = merge_launch(tab, h->d_mtab, h->d_msegs, ts, cols, col_stride, merged, merged_stride,
+                           atom_bin, st)))
+        return rc;
     TCW_HIP_TRY(hipStreamSynchronize(st));
     return TCW_OK;
 }

@@ -120,15 +120,27 @@ class MergedAtoms:
         self.desc.windows = None
         self.m_off = np.zeros(self.T + 1, dtype=np.int64)
         self.t_data = np.zeros(self.T, dtype=np.uint32)
-        _hiplib.check(self.lib.tcw_merge_batch(
-            self.handle, ctypes.byref(self.desc), None, None, 0, None, 0,
-            self.m_off.ctypes.data, self.t_data.ctypes.data, None, None), "tcw_merge_batch")
+        plan = ctypes.c_void_p()
+        _hiplib.check(self.lib.tcw_merge_plan_create(
+            self.handle, ctypes.byref(self.desc), ctypes.byref(plan), self.m_off.ctypes.data,
+            self.t_data.ctypes.data), "tcw_merge_plan_create")
+        self.plan = plan
         self.total_bins = int(self.m_off[-1])
         self.N = np.diff(self.m_off)
         self.atom_bin = torch.empty(self.n_atoms, dtype=torch.int64, device=device)
         self.cols = None
         if cols_raw is not None:
             self.cols = self.merge(cols_raw)
+            # merged once here, used on any stream afterwards
+            torch.cuda.current_stream(device).synchronize()
+
+    def __del__(self):
+        try:
+            if getattr(self, "plan", None):
+                self.lib.tcw_merge_plan_destroy(self.plan)
+                self.plan = None
+        except Exception:
+            pass
 
     @classmethod
     def from_batch(cls, batch):
@@ -149,11 +161,9 @@ class MergedAtoms:
             raise ValueError(f"expected {self.n_atoms} atoms, got {cols_raw.shape[1]}")
         cols_raw = cols_raw.contiguous()
         out = torch.empty((7, self.total_bins), dtype=torch.float32, device=self.device)
-        _hiplib.check(self.lib.tcw_merge_batch(
-            self.handle, ctypes.byref(self.desc), _ptr(self.ts_d), _ptr(cols_raw),
-            cols_raw.shape[1], _ptr(out), self.total_bins, self.m_off.ctypes.data,
-            self.t_data.ctypes.data, _ptr(self.atom_bin), _stream(torch, self.device)),
-            "tcw_merge_batch")
+        _hiplib.check(self.lib.tcw_merge_run(
+            self.plan, _ptr(self.ts_d), _ptr(cols_raw), cols_raw.shape[1], _ptr(out),
+            self.total_bins, _ptr(self.atom_bin), _stream(torch, self.device)), "tcw_merge_run")
         return out
 
     def _merge_backward(self, grad_merged):
