@@ -140,69 +140,120 @@ struct ItemPart {
 // stage: binned merge + FP64 prefix (rect) / float32 atom table (exp)
 // ----------------------------------------------------------------------------
 
-constexpr int SR_WG = 256;                        // 4 wave64
-constexpr int SR_BINS = 4;                        // consecutive bins per thread per round
-constexpr int SR_ROUND = SR_WG * SR_BINS;         // 1024 bins per round
-constexpr int SR_CHUNK = 1024;                    // atoms staged in LDS per pass
-constexpr int SR_PASS_LANES = 32;                 // lanes per output pass
-constexpr int SR_PASS_BINS = SR_PASS_LANES * SR_BINS;  // 128 bins per wave per pass
+constexpr int SR_BINS = 4;           // consecutive bins per thread per round
+constexpr int SR_PASS_LANES = 32;    // lanes per output pass
+constexpr int SR_PASS = SR_PASS_LANES * SR_BINS * NC;  // doubles per wave and output pass
+// Threads of a template's workgroup: one round for the shorter templates
+// (128: N <= 512, 256: N <= 1024).  Longer ones take several rounds of 256
+// threads, or, if they are few, of 1024: a CU holds one such workgroup, whose
+// waves share the template's rounds, but all of them wait for each other at
+// every barrier.  Measured, N = 1000..4000 and 1000..8000, 256 | 1024 threads:
+// 128 templates 57 | 40 us, 288 62 | 45, 512 105 | 92, 768 122 | 124, 1024
+// 133 | 154; the line lies where the two meet.
+constexpr int SR_CLASSES = 3;
+constexpr int SR_THREADS[SR_CLASSES] = {128, 256, 256};
+constexpr int SR_WIDE_THREADS = 1024;
+constexpr int64_t SR_WIDE_TMPLS = 640;
+static_assert(SR_THREADS[2] == SR_THREADS[1], "one kernel");
+constexpr int stage_class(uint32_t N) {
+    return N <= SR_THREADS[0] * SR_BINS ? 0 : N <= SR_THREADS[1] * SR_BINS ? 1 : 2;
+}
+
+// DPP controls of a wave scan: shifts within the 16-lane rows, and the last
+// lane of a row (of the lower half) to the next row (the upper half)
+constexpr int DPP_ROW_SHR = 0x110;
+constexpr int DPP_ROW_BCAST15 = 0x142;
+constexpr int DPP_ROW_BCAST31 = 0x143;
+
+// the DPP source's value, 0.0 on lanes without one or in rows outside ROWS
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_d(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, ROWS, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// inclusive scan over the 64 lanes, in log depth, without LDS
+__device__ __forceinline__ double wave_scan(double x) {
+    x += dpp_d<DPP_ROW_SHR + 1>(x);
+    x += dpp_d<DPP_ROW_SHR + 2>(x);
+    x += dpp_d<DPP_ROW_SHR + 4>(x);
+    x += dpp_d<DPP_ROW_SHR + 8>(x);
+    x += dpp_d<DPP_ROW_BCAST15, 0xa>(x);
+    return x + dpp_d<DPP_ROW_BCAST31, 0xc>(x);
+}
+
+// x / TAtom and x % TAtom: the product with the reciprocal is at most one short
+__device__ __forceinline__ uint32_t div_TA(uint32_t x, const TmplDev &td, uint32_t &rem) {
+    uint32_t q = __umulhi(x, td.TA_rcp);
+    rem = x - q * td.TAtom;
+    const bool more = rem >= td.TAtom;
+    rem -= more ? td.TAtom : 0;
+    return q + more;
+}
+
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef d2 d2_u __attribute__((aligned(8)));  // the table starts at any double
 
 // Rectangular-window templates: the exclusive prefix P[b] = sum of merged
-// bins < b per column, [N+1][7] doubles.  One workgroup per template, rounds
-// of 1024 bins, 4 consecutive bins per thread.
-//  - merge: per detector, the workgroup copies the round's atoms into LDS in
-//    chunks of 1024 with coalesced loads (a cursor per detector carries the
-//    first atom of the next round); each thread finds its first bin's atoms
-//    by binary search in LDS and sums its bins.  A bin's merged value is the
-//    float32 sum over detectors X = 0,1,... (in that order) of the detector's
-//    atoms in the bin (in atom order), from 0 -- the additions of
-//    lalpulsar's binned merge, in its order, so merged atoms are
+// bins < b per column, [N+1][7] doubles.  One workgroup of NT threads per
+// template, rounds of 4 NT bins, 4 consecutive bins per thread.
+//  - merge: per detector, the bins of up to 4 NT timestamps are formed
+//    (coalesced loads), and the first atom of every bin is marked where the bin
+//    changes; each thread then reads its bins' atoms from the columns.  A
+//    bin's merged value is the float32 sum over detectors X = 0,1,... (in that
+//    order) of the detector's atoms in the bin (in atom order), from 0 -- the
+//    additions of lalpulsar's binned merge, in its order, so merged atoms are
 //    bit-identical;
-//  - scan (FP64): thread totals, a Kogge-Stone scan within the wave, the 4
-//    wave totals and the carry of earlier rounds in LDS.  A prefix value
-//    carries ~20 roundings of 2^-53 relative to the largest partial sum;
+//  - scan (FP64): thread totals, a scan within the wave in log depth, the wave
+//    totals and the carry of earlier rounds in LDS.  A prefix value carries
+//    ~20 roundings of 2^-53 relative to the largest partial sum;
 //  - output: the LDS buffer is reused to transpose the prefix values, 32 lanes
 //    of each wave per pass, so every global store is a contiguous run of the
 //    [N+1][7] table (a thread's own 4 bins span 224 bytes).
-__global__ __launch_bounds__(SR_WG) void stage_kernel(
-    const TmplDev *__restrict__ tds, const SegDev *__restrict__ segs,
-    const uint32_t *__restrict__ ts, const float *__restrict__ cols, int64_t cstride,
-    double *__restrict__ prefix, int *__restrict__ flags) {
-    // one block per template, before any map kernel: set its flags (exp
-    // templates: none)
-    const TmplDev td = tds[blockIdx.x];
-    if (td.mode != MODE_RECT_FAST && td.mode != MODE_RECT_GENERIC) {  // block-uniform
-        if (threadIdx.x == 0) flags[blockIdx.x] = 0;
-        return;
-    }
-    // staging: ts [SR_CHUNK] uint32, then NC float planes [SR_CHUNK];
-    // output: per wave SR_PASS_BINS x NC doubles
-    __shared__ double s_buf[SR_CHUNK * (NC + 1) / 2];
-    static_assert(4 * SR_PASS_BINS * NC <= SR_CHUNK * (NC + 1) / 2, "output buffer");
-    uint32_t *s_ts = reinterpret_cast<uint32_t *>(s_buf);
-    float *s_x = reinterpret_cast<float *>(s_buf) + SR_CHUNK;
-    __shared__ double s_off[NC][SR_WG / 64];  // wave totals, then wave offsets
-    __shared__ double s_carry[NC];            // sum of all earlier rounds
-    __shared__ int64_t s_ka;
-    __shared__ int s_flag;
-    if (threadIdx.x == 0) s_flag = 0;  // a barrier follows in the first round
+// Bound: the waves' own instructions (about 1100 a round, half of them the
+// output passes) on the few CUs that a batch of long templates fills, with the
+// round's chain (two dependent loads, the barriers, the scan) exposed; stores
+// and loads left out save 1 and 9 of 40 us.  The binary searches of a thread's
+// first bins, a scan through LDS and 8-byte LDS words took: 1024 templates of
+// N = 1000..8000 147 us (now 133), 128 of N = 1000..4000 and two detectors 49
+// (40), 1024 of 500 and two detectors 23.4 (20.6).
+template <int NT>
+__global__ __launch_bounds__(NT) void stage_kernel(
+    const TmplDev *__restrict__ tds, const int32_t *__restrict__ tmpls,
+    const SegDev *__restrict__ segs, const uint32_t *__restrict__ ts,
+    const float *__restrict__ cols, int64_t cstride, double *__restrict__ prefix,
+    int *__restrict__ flags) {
+    constexpr int NW = NT / 64;
+    constexpr int ROUND = NT * SR_BINS;
+    // per chunk of ROUND atoms: their bins, and the bins' first atoms; then the
+    // output passes' transpose buffers
+    __shared__ __align__(16) double s_buf[NW * SR_PASS];
+    static_assert(NW * SR_PASS * 2 >= 2 * ROUND, "bins and first atoms share the buffer");
+    int *s_bin = reinterpret_cast<int *>(s_buf);
+    int *s_first = s_bin + ROUND;
+    __shared__ double s_tot[NW][NC + 1];  // wave totals
+    __shared__ int64_t s_cur[TCW_MAX_DETECTORS];  // a detector's first atom not yet merged
+    __shared__ int s_cnt, s_flag;
 
-    const uint32_t N = td.N;
-    const uint64_t TA = td.TAtom;
+    const int t = tmpls[blockIdx.x];
+    const TmplDev td = tds[t];
+    const int N = (int)td.N;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nseg = (int)(td.seg_end - td.seg_begin);
     double *__restrict__ P = prefix + td.prefix_off;
-    // thread X < nseg keeps detector X's cursor: its first atom not yet merged
-    int64_t cur = tid < nseg ? segs[td.seg_begin + tid].begin : 0;
-    if (tid < NC) s_carry[tid] = 0.0;
+    if (tid == 0) s_flag = 0;
+    if (tid < nseg) s_cur[tid] = segs[td.seg_begin + tid].begin;
+    double carry[NC];  // sum of all earlier rounds
+#pragma unroll
+    for (int c = 0; c < NC; c++) carry[c] = 0.0;
+    __syncthreads();
 
-    for (uint32_t base = 0; base < N; base += SR_ROUND) {
-        const uint32_t bend = min(N, base + (uint32_t)SR_ROUND);
-        const uint32_t b0 = base + (uint32_t)tid * SR_BINS;
-        const uint64_t t_lo = (uint64_t)td.t_min + (uint64_t)b0 * TA;
-        const uint64_t tb_hi = (uint64_t)td.t_min + (uint64_t)bend * TA;  // later rounds' atoms
+    for (int base = 0; base < N; base += ROUND) {
+        const int nb = min(ROUND, N - base);  // bins of this round
         float v[SR_BINS][NC];
 #pragma unroll
         for (int j = 0; j < SR_BINS; j++)
@@ -210,54 +261,63 @@ __global__ __launch_bounds__(SR_WG) void stage_kernel(
             for (int c = 0; c < NC; c++) v[j][c] = 0.0f;
         for (int X = 0; X < nseg; X++) {
             const int64_t seg_end = segs[td.seg_begin + X].end;
-            if (tid == X) s_ka = cur;
-            __syncthreads();
-            int64_t c0 = s_ka;
-            __syncthreads();  // s_ka is rewritten for the next detector
-            int64_t next = seg_end;
+            int64_t c0 = s_cur[X];
             while (c0 < seg_end) {  // block-uniform
-                const int na = (int)min((int64_t)SR_CHUNK, seg_end - c0);
-                for (int i = tid; i < na; i += SR_WG) {
-                    s_ts[i] = ts[c0 + i];
+                const int na = (int)min((int64_t)ROUND, seg_end - c0);
+                int bin[SR_BINS];
 #pragma unroll
-                    for (int c = 0; c < NC; c++) s_x[c * SR_CHUNK + i] = cols[c * cstride + c0 + i];
+                for (int u = 0; u < SR_BINS; u++) {
+                    const int i = u * NT + tid;
+                    const uint32_t x = i < na ? ts[c0 + i] : 0;
+                    uint32_t rem;
+                    // -1: before the first bin (in none); nb: in a later round
+                    const int b = (int)min(div_TA(x - td.t_min, td, rem), 0x7fffffffu) - base;
+                    bin[u] = i >= na ? nb : x < td.t_min ? -1 : min(b, nb);
+                    s_bin[i] = bin[u];
+                    s_first[i] = -1;
+                }
+                if (tid == 0) s_cnt = na;
+                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < SR_BINS; u++) {
+                    const int i = u * NT + tid;
+                    const int before = i > 0 ? s_bin[i - 1] : -1;
+                    if (bin[u] != before || i == 0) {
+                        if (bin[u] >= 0 && bin[u] < nb) s_first[bin[u]] = i;
+                        if (bin[u] == nb && i < na) s_cnt = i;
+                    }
                 }
                 __syncthreads();
-                if (b0 < bend) {
-                    int lo = 0, hi = na;  // first staged atom with ts >= t_lo
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if ((uint64_t)s_ts[mid] < t_lo)
-                            lo = mid + 1;
-                        else
-                            hi = mid;
-                    }
-                    int k = lo;
+                const int cnt = s_cnt;
+                int k[SR_BINS];
+                const float *__restrict__ col = cols + c0;
+                // (a 32-bit offset from a uniform address: no 64-bit sums)
+                auto at = [&](int c, int k) {
+                    return *reinterpret_cast<const float *>(
+                        reinterpret_cast<const char *>(col + c * cstride) + (uint32_t)k * 4u);
+                };
 #pragma unroll
-                    for (int j = 0; j < SR_BINS; j++) {
-                        const uint64_t t_hi = t_lo + (uint64_t)(j + 1) * TA;
-                        for (; k < na && (uint64_t)s_ts[k] < t_hi; k++) {
+                for (int j = 0; j < SR_BINS; j++) k[j] = s_first[tid * SR_BINS + j];
+                float y[SR_BINS][NC];  // the bins' first atoms, all loads in flight
 #pragma unroll
-                            for (int c = 0; c < NC; c++) v[j][c] += s_x[c * SR_CHUNK + k];
-                        }
+                for (int j = 0; j < SR_BINS; j++)
+#pragma unroll
+                    for (int c = 0; c < NC; c++) y[j][c] = at(c, max(k[j], 0));
+#pragma unroll
+                for (int j = 0; j < SR_BINS; j++) {
+                    if (k[j] < 0) continue;
+#pragma unroll
+                    for (int c = 0; c < NC; c++) v[j][c] += y[j][c];
+                    for (int q = k[j] + 1; q < cnt && s_bin[q] == tid * SR_BINS + j; q++) {
+#pragma unroll
+                        for (int c = 0; c < NC; c++) v[j][c] += at(c, q);
                     }
                 }
-                int lo = 0, hi = na;  // first staged atom of a later round (same on all threads)
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if ((uint64_t)s_ts[mid] < tb_hi)
-                        lo = mid + 1;
-                    else
-                        hi = mid;
-                }
-                __syncthreads();  // staged atoms consumed before the next chunk
-                if (lo < na) {
-                    next = c0 + lo;
-                    break;
-                }
-                c0 += na;
+                __syncthreads();  // bins consumed before the next chunk
+                c0 += cnt;
+                if (cnt < na) break;
             }
-            if (tid == X) cur = next;
+            if (tid == 0) s_cur[X] = c0;  // read again after the next round's barriers
         }
         bool odd = false;  // what FLAG_NO_BOUND is for (NaN compares false)
 #pragma unroll
@@ -265,68 +325,73 @@ __global__ __launch_bounds__(SR_WG) void stage_kernel(
             odd |= !(v[j][0] >= 0.0f) | !(v[j][1] >= 0.0f) | !(fabsf(v[j][2]) < INFINITY);
         if (odd) s_flag = FLAG_NO_BOUND;
         // inclusive scan of the thread totals within the wave (bins >= N hold 0)
-        double x[NC];
+        double ex[NC];
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            double t = 0.0;
+            double sum = 0.0;
 #pragma unroll
-            for (int j = 0; j < SR_BINS; j++) t += (double)v[j][c];
-            x[c] = t;
-        }
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const double y = __shfl_up(x[c], d);
-                if (lane >= d) x[c] += y;
-            }
-        }
-        if (lane == 63) {
-#pragma unroll
-            for (int c = 0; c < NC; c++) s_off[c][wave] = x[c];
+            for (int j = 0; j < SR_BINS; j++) sum += (double)v[j][c];
+            const double x = wave_scan(sum);
+            if (lane == 63) s_tot[wave][c] = x;
+            ex[c] = __shfl_up(x, 1);
+            if (lane == 0) ex[c] = 0.0;
         }
         __syncthreads();
-        if (tid < NC) {  // exclusive scan of the wave totals, seeded by the carry
-            double run = s_carry[tid];
-            for (int w = 0; w < SR_WG / 64; w++) {
-                const double t = s_off[tid][w];
-                s_off[tid][w] = run;
-                run += t;
-            }
-            s_carry[tid] = run;
-        }
-        __syncthreads();
-        double ex[NC];  // exclusive prefix at the thread's first bin
+        // exclusive prefix at the thread's first bin: the carry, the earlier
+        // waves' totals in order, the earlier lanes
+#pragma unroll 4
+        for (int w = 0; w < wave; w++)
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            double e = __shfl_up(x[c], 1);
-            if (lane == 0) e = 0.0;
-            ex[c] = s_off[c][wave] + e;
-        }
-        double *out = s_buf + wave * (SR_PASS_BINS * NC);
+            for (int c = 0; c < NC; c++) carry[c] += s_tot[w][c];
+#pragma unroll
+        for (int c = 0; c < NC; c++) ex[c] += carry[c];
+#pragma unroll 4
+        for (int w = wave; w < NW; w++)
+#pragma unroll
+            for (int c = 0; c < NC; c++) carry[c] += s_tot[w][c];
+        // the thread's 4 bins are 28 consecutive doubles of the table: through
+        // LDS in 16-byte words, so that a store covers 1 KB of it in one run
+        d2 *out = reinterpret_cast<d2 *>(s_buf + wave * SR_PASS);
 #pragma unroll 1
         for (int pass = 0; pass < 64 / SR_PASS_LANES; pass++) {
-            if (lane / SR_PASS_LANES == pass && b0 < bend) {
-                const int q = lane % SR_PASS_LANES;
+            const int wb = wave * (64 * SR_BINS) + pass * (SR_PASS_LANES * SR_BINS);
+            const int cnt = min(SR_PASS_LANES * SR_BINS, nb - wb) * NC;
+            if (cnt <= 0) break;  // wave-uniform
+            if (lane / SR_PASS_LANES == pass) {
+                double r[SR_BINS * NC];
 #pragma unroll
                 for (int c = 0; c < NC; c++) {
-                    double r = ex[c];
+                    r[c] = ex[c];
 #pragma unroll
-                    for (int j = 0; j < SR_BINS; j++) {
-                        out[(q * SR_BINS + j) * NC + c] = r;
-                        r += (double)v[j][c];
-                    }
+                    for (int j = 1; j < SR_BINS; j++)
+                        r[j * NC + c] = r[(j - 1) * NC + c] + (double)v[j - 1][c];
                 }
+                d2 *row = out + (lane % SR_PASS_LANES) * (SR_BINS * NC / 2);
+#pragma unroll
+                for (int q = 0; q < SR_BINS * NC / 2; q++) row[q] = d2{r[2 * q], r[2 * q + 1]};
             }
-            __syncthreads();
-            const int64_t wb = (int64_t)base + wave * (64 * SR_BINS) + pass * SR_PASS_BINS;
-            const int cnt = (int)max((int64_t)0, min((int64_t)SR_PASS_BINS, (int64_t)bend - wb));
-            for (int i = lane; i < cnt * NC; i += 64) P[wb * NC + i] = out[i];
-            __syncthreads();  // copied out before the next pass (or round) rewrites
+            // the buffer is the wave's own: order its LDS accesses, no barrier
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            double *dst = P + (int64_t)(base + wb) * NC;
+#pragma unroll
+            for (int q = 0; q < SR_PASS / 2; q += 64) {
+                const int i = q + lane;
+                if (2 * i + 1 < cnt)
+                    *reinterpret_cast<d2_u *>(dst + 2 * i) = out[i];
+                else if (2 * i < cnt)
+                    dst[2 * i] = out[i][0];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
+        __syncthreads();  // the buffer holds bins again in the next round
     }
-    if (tid < NC) P[(int64_t)N * NC + tid] = s_carry[tid];
-    if (tid == 0) flags[blockIdx.x] = s_flag;
+    if (tid == 0) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) P[(int64_t)N * NC + c] = carry[c];
+        flags[t] = s_flag;
+    }
 }
 
 // Bins of a template's atom table: the recurrence path reads none at or
@@ -1237,15 +1302,6 @@ constexpr int64_t STEP_ITEMS = 1024;
 // maps below at 20, 28, 36 and 52 KB: 112, 95, 94 and 100 us).
 constexpr int STEP_LDS_AIM = 36 << 10;
 constexpr int STEP_LDS_MOST = 76 << 10;
-
-// x / TAtom and x % TAtom: the product with the reciprocal is at most one short
-__device__ __forceinline__ uint32_t div_TA(uint32_t x, const TmplDev &td, uint32_t &rem) {
-    uint32_t q = __umulhi(x, td.TA_rcp);
-    rem = x - q * td.TAtom;
-    const bool more = rem >= td.TAtom;
-    rem -= more ? td.TAtom : 0;
-    return q + more;
-}
 
 struct StepShape {
     int entries;  // staged prefix entries of an item at most
@@ -2764,14 +2820,6 @@ constexpr int FIN_AHEAD = 12;
 
 // FP64 values across the wave without LDS, as wave_sum and wave_max do for
 // floats: every lane ends with the same bits.
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-    const long long u = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-
 template <typename Op>
 __device__ __forceinline__ double wave_reduce_d(double v, Op op) {
     v = op(v, dpp_d<DPP_QUAD_XOR1>(v));
@@ -3146,6 +3194,10 @@ struct tcw_plan {
     std::vector<ItemDev> col_items;  // MODE_EXP_FAST (t, -, column block)
     std::vector<ItemDev> init_items;  // exp_init waves (t, part, column block), heaviest first
     std::vector<int32_t> exp_tmpls;  // templates needing the atom table
+    // templates needing the prefix table, per stage_kernel class, longest first
+    std::vector<int32_t> rect_tmpls[SR_CLASSES];
+    // exp_tmpls, then the classes of rect_tmpls (one buffer: a single map fills no more of it)
+    std::vector<int32_t> tmpl_list;
     int64_t exp_max_N = 0;
     bool exp_init_needed = false;  // some exp template has a non-empty direct sum
     bool exp_scan_wave = false;    // the wave-per-column chunk scan (few, long columns)
@@ -3160,7 +3212,7 @@ struct tcw_plan {
     int64_t walk_tmpls = 0, direct_tmpls = 0;   // MODE_EXP_DIRECT templates of either kernel
     int64_t step_tmpls = 0, generic_tmpls = 0;  // MODE_RECT_GENERIC templates of either kernel
     DevBuf d_tmpl, d_segs, d_items, d_prefix, d_merged, d_ipart, d_rowpart, d_colpart,
-        d_flags, d_seg_items, d_col_items, d_etab, d_exp_tmpls, d_init_items;
+        d_flags, d_seg_items, d_col_items, d_etab, d_tmpl_list, d_init_items;
     hipGraphExec_t graph = nullptr;
     hipStream_t cap_stream = nullptr;  // private stream the graph is captured on
     // exp_init_kernel runs here beside exp_seg_kernel (they are independent)
@@ -3187,6 +3239,7 @@ struct tcw_plan {
         col_items.clear();
         init_items.clear();
         exp_tmpls.clear();
+        for (auto &r : rect_tmpls) r.clear();
         exp_max_N = 0;
         exp_init_needed = false;
         exp_scan_wave = false;
@@ -3219,7 +3272,7 @@ struct tcw_plan {
         d_col_items.release();
         d_init_items.release();
         d_etab.release();
-        d_exp_tmpls.release();
+        d_tmpl_list.release();
         d_ts.release();
         d_cols.release();
     }
@@ -3344,11 +3397,6 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     int64_t N_t0, N_tau;
     int rc = effective_window(N, TAtom, t_min, win_in, w, N_t0, N_tau);
     if (rc) return rc;
-    if (seg_end - seg_begin > SR_WG)  // the merge keeps one cursor per detector and thread
-        return tcwc::fail(TCW_ERR_INVALID, "template " + std::to_string(t) + " has " +
-                                           std::to_string(seg_end - seg_begin) +
-                                           " detector segments; at most " +
-                                           std::to_string(SR_WG) + " are supported.");
     TmplDev td;
     std::memset(&td, 0, sizeof(td));
     td.seg_begin = seg_begin;
@@ -3509,6 +3557,7 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
             p.direct_tmpls++;
         }
     } else {
+        p.rect_tmpls[stage_class(N)].push_back((int32_t)t);
         td.prefix_off = p.prefix_doubles;
         p.prefix_doubles += ((int64_t)N + 1) * NC;
     }
@@ -3556,7 +3605,7 @@ void plan_buffers(tcw_plan &p, F f) {
     f(p.d_col_items, sizeof(ItemDev) * std::max<size_t>(p.col_items.size(), 1));
     f(p.d_init_items, sizeof(ItemDev) * std::max<size_t>(p.init_items.size(), 1));
     f(p.d_etab, sizeof(double) * std::max<int64_t>(p.etab_doubles, 1));
-    f(p.d_exp_tmpls, sizeof(int32_t) * std::max<size_t>(p.exp_tmpls.size(), 1));
+    f(p.d_tmpl_list, sizeof(int32_t) * std::max<size_t>(p.tmpl_list.size(), 1));
 }
 
 // After all templates: lay out items mode by mode, fix item_begin (the items
@@ -3580,6 +3629,13 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
         }
     }
     p.mode_begin[MODE_COUNT] = (int64_t)p.items.size();
+    p.tmpl_list = p.exp_tmpls;
+    for (auto &r : p.rect_tmpls) {
+        // the longest templates first: the last workgroups to start are short
+        std::stable_sort(r.begin(), r.end(),
+                         [&](int32_t x, int32_t y) { return p.tmpl[x].N > p.tmpl[y].N; });
+        p.tmpl_list.insert(p.tmpl_list.end(), r.begin(), r.end());
+    }
     struct Up {
         DevBuf *buf;
         const void *src;
@@ -3592,7 +3648,7 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
         {&p.d_seg_items, p.seg_items.data(), sizeof(ItemDev) * p.seg_items.size()},
         {&p.d_col_items, p.col_items.data(), sizeof(ItemDev) * p.col_items.size()},
         {&p.d_init_items, p.init_items.data(), sizeof(ItemDev) * p.init_items.size()},
-        {&p.d_exp_tmpls, p.exp_tmpls.data(), sizeof(int32_t) * p.exp_tmpls.size()},
+        {&p.d_tmpl_list, p.tmpl_list.data(), sizeof(int32_t) * p.tmpl_list.size()},
     };
     if (p.host_ts) {
         ups.push_back({&p.d_ts, p.host_ts, sizeof(uint32_t) * (size_t)p.n_host_atoms});
@@ -3757,12 +3813,19 @@ int launch_all(tcw_plan &p, const uint32_t *ts, const float *cols, int64_t cstri
     const bool strict = p.flags & TCW_FLAG_LAL_STRICT;
     auto *flags = (int *)p.d_flags.p;
     if (ev) TCW_HIP_TRY(hipEventRecord(ev[0], st));
-    // (stage_exp_kernel clears the single-atom flags of the exp templates, so
-    // a batch of exp templates only launches no stage_kernel)
-    if ((int64_t)p.exp_tmpls.size() < p.T)
-        hipLaunchKernelGGL(stage_kernel, dim3((unsigned)p.T), dim3(SR_WG), 0, st,
-                           (const TmplDev *)p.d_tmpl.p, (const SegDev *)p.d_segs.p, ts, cols,
+    const int32_t *rect = (const int32_t *)p.d_tmpl_list.p + p.exp_tmpls.size();
+    for (int k = 0; k < SR_CLASSES; k++) {
+        const unsigned n = (unsigned)p.rect_tmpls[k].size();
+        if (n == 0) continue;
+        const bool wide = k == SR_CLASSES - 1 && n <= SR_WIDE_TMPLS;
+        auto *kern = wide     ? stage_kernel<SR_WIDE_THREADS>
+                     : k == 0 ? stage_kernel<SR_THREADS[0]>
+                              : stage_kernel<SR_THREADS[1]>;
+        hipLaunchKernelGGL(kern, dim3(n), dim3(wide ? SR_WIDE_THREADS : SR_THREADS[k]), 0, st,
+                           (const TmplDev *)p.d_tmpl.p, rect, (const SegDev *)p.d_segs.p, ts, cols,
                            cstride, (double *)p.d_prefix.p, flags);
+        rect += n;
+    }
     if (!p.exp_tmpls.empty()) {
         const int64_t n_exp = (int64_t)p.exp_tmpls.size();
         const int64_t wide_blocks = (p.exp_max_N + 1023) / 1024;
@@ -3770,11 +3833,11 @@ int launch_all(tcw_plan &p, const uint32_t *ts, const float *cols, int64_t cstri
         if (n_exp > 0 && wide_blocks * n_exp < SX_NARROW_BELOW)
             hipLaunchKernelGGL(stage_exp_kernel<1>, dim3((unsigned)((p.exp_max_N + 255) / 256), gy),
                                dim3(256), 0, st, (const TmplDev *)p.d_tmpl.p,
-                               (const int32_t *)p.d_exp_tmpls.p, n_exp, (const SegDev *)p.d_segs.p,
+                               (const int32_t *)p.d_tmpl_list.p, n_exp, (const SegDev *)p.d_segs.p,
                                ts, cols, cstride, (float *)p.d_merged.p, flags);
         else if (n_exp > 0)
             hipLaunchKernelGGL(stage_exp_kernel<4>, dim3((unsigned)wide_blocks, gy), dim3(256), 0,
-                               st, (const TmplDev *)p.d_tmpl.p, (const int32_t *)p.d_exp_tmpls.p,
+                               st, (const TmplDev *)p.d_tmpl.p, (const int32_t *)p.d_tmpl_list.p,
                                n_exp, (const SegDev *)p.d_segs.p, ts, cols, cstride,
                                (float *)p.d_merged.p, flags);
     }
