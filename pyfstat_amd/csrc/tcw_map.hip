@@ -74,12 +74,12 @@ constexpr int RB_DEFAULT[MODE_COUNT] = {192, 16, 16, 128};
 // at a time (256 templates of 48 x 48 to 240 x 240: maps 22 us, 26 at 1024
 // items, 29 at 512; 1024 templates of 125 x 125: 35 us, 37 at 1024, 38 at 4096).
 constexpr int64_t SMALL_BATCH_ITEMS = 2048;
-// exp_walk_kernel items aimed at when rows are not tuned: two a CU, which is
-// how many fit at a time; fewer rows repeat the direct sum, more leave CUs idle
-// (256 templates of 125 x 125 cells: 130 us at 64 rows, 165 at 32, 152 at 128;
-// 64 of 500 x 500: 575 us at 128 rows, 739 at 64, 604 at 256; 4 of 500 x 500:
-// 200 us at 16 rows, 228 at 32).
-constexpr int64_t WALK_ITEMS = 512;
+// exp_walk_kernel items aimed at when rows are not tuned: one a CU; fewer rows
+// repeat the direct sum, more leave CUs idle.  Rows by 32, so that eight waves
+// get four each at least.  Measured (maps, us, at 32 | 64 | 128 | 256 rows):
+// 32 templates of 125 x 125 cells 30 | 37 | 47 | 47; 4 of 500 x 500 89 | 63 | 74 |
+// 132; 64 of 500 x 500 1004 | 583 | 373 | 352.
+constexpr int64_t WALK_ITEMS = 256;
 constexpr int WALK_MAX_ROWS = 256;
 constexpr int EXP_SMALL_BATCH_ROWS = 64;    // exp rows when untuned and under 256 column blocks
 
@@ -1593,32 +1593,42 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
 // rho^(hi' + 1 - lo') is one of four values per lane, as that exponent is
 // Q - 1 .. Q + 2.  A cell costs O(dt0 / TAtom) instead of O(3 tau / TAtom).
 //
-// An item of RB rows x 256 columns starts with the direct sum at its top row
-// and walks down.  A group of 64 columns has two waves, or four or eight in
-// items of at most 128 or 64 columns: they share the direct sum's atoms (staged
-// in LDS chunk by chunk), then all walk and take turns at evaluating four rows.
-// Entering and leaving atoms come from LDS where the item's ranges of them fit.
+// An item is RB rows x 64 columns, one column a lane, and its rows are shared
+// out to eight waves from the top down.  The waves share the direct sum at the
+// item's top row by atoms (staged in LDS chunk by chunk); then each sums what
+// enters and leaves between its own top row and the next wave's (two Horner
+// sums, the recurrence over many rows at once), which gives every wave the sum
+// at its top row; then each walks its rows.  Entering and leaving atoms come
+// from LDS where the item's ranges of them fit.
 //
 // What the direct sum gives exactly and a sliding sum would not: a window
 // whose bins are all zero has E = 0 (the kind column counts bins with data),
 // and from the first infinite or NaN atom on, the item's rows are summed
 // directly, as are all rows where the steps are longer than the windows.
 //
-// Bound: latency -- the direct sum at the top (16 to 21 instructions and 16 LDS
-// cycles an atom and wave, two waves a SIMD) and ~0.9 us a row step.  32
-// templates of 125 x 125 cells and 1000 bins: 700 us with a direct sum for
-// every cell, 52 us so (four waves a workgroup instead of eight: 74; the atoms
-// through scalar loads instead of LDS: 172).
+// Bound: latency of the item's phases (one or two workgroups a CU), and for long
+// windows the direct sum (16 to 21 instructions an atom and wave).  125 x 125
+// cells and 1000 bins: 32 templates 700 us with a direct sum for every cell, 52
+// with items of 256 columns whose waves all walked every row, 30 so (13 of them
+// the direct sum, 3 the steps between the waves' rows); 256 templates 139, now
+// 71.  500 x 500 cells and 4000 bins: 64 templates 577, now 352; one 200, now 57.
 constexpr int WALK_WAVES = 8;
 constexpr int WALK_WG = 64 * WALK_WAVES;
+constexpr int WALK_TILE = 64;        // columns of an item
 constexpr int WALK_TAIL_CAP = 1024;  // leaving atoms staged in LDS (32 KB)
 constexpr int WALK_HEAD_CAP = 256;   // entering atoms staged in LDS (8 KB)
-constexpr int WALK_CHUNK = 512;      // atoms of the direct sum staged at a time (16 KB)
+constexpr int WALK_CHUNK = 1024;     // atoms of the direct sum staged at a time (32 KB)
 static_assert(WALK_WAVES * MERGED_STRIDE * 64 * 2 <= WALK_TAIL_CAP * MERGED_STRIDE &&
                   WALK_CHUNK <= WALK_TAIL_CAP,
               "the direct sum's chunk and parts share the leaving atoms' LDS");
+// a wave's change of E to the next wave's top row: 7 sums, the kinds, and the
+// power of rho that E takes
+constexpr int WALK_STEP = NC + 2;
+constexpr int walk_rows(int rb) { return (rb + 3) / 4 * 4; }
 constexpr int walk_lds(int rb) {
-    return ((WALK_TAIL_CAP + WALK_HEAD_CAP) * MERGED_STRIDE + 4 * rb * 2) * (int)sizeof(float);
+    return ((WALK_TAIL_CAP + WALK_HEAD_CAP) * MERGED_STRIDE + walk_rows(rb) * 2) *
+               (int)sizeof(float) +
+           (WALK_WAVES - 1) * WALK_STEP * 64 * (int)sizeof(double);
 }
 
 struct WalkCol {  // a lane's column, 3 tau = TAtom Q + R
@@ -1672,7 +1682,7 @@ __device__ __forceinline__ bool walk_stage(float *dst, const float *__restrict__
 template <bool MASK>
 __device__ __forceinline__ void walk_horner(const float *x, int count, int L, const WalkCol &wc,
                                             double (&E)[NC], float &kinds) {
-#pragma unroll 4
+#pragma unroll 2  // (4: more than 128 VGPRs)
     for (int l = count - 1; l >= 0; l--) {
         const float *v = x + l * MERGED_STRIDE;
         double r0 = wc.rho[0], r1 = wc.rho[1];
@@ -1722,73 +1732,69 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
     const float *__restrict__ X = merged + td.merged_off;
     float *__restrict__ Ft = Fout + td.F_off;
     const int RB = td.rb_rows;
-    const int row0 = it.rb * RB, col0 = it.cb * TILE_COLS;
+    const int row0 = it.rb * RB, col0 = it.cb * WALK_TILE;
     const int N_tau = (int)td.N_tau;
     const int nrows = min(RB, (int)td.N_t0 - row0);
     const int N = (int)td.N;
     const uint32_t TA = td.TAtom;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int groups = (min(TILE_COLS, N_tau - col0) + 63) / 64;
-    const int W = WALK_WAVES / (groups == 3 ? 4 : groups);  // waves of a group
-    const int g = wave / W, w = wave % W;
-    const bool active = g < groups;  // (three groups: the others only keep the barriers)
-    const int n = col0 + g * 64 + lane;
-    const bool valid = active && n < N_tau;
+    const int n = col0 + lane;
+    const bool valid = n < N_tau;
     float *tail = lds;
     double *comb = reinterpret_cast<double *>(lds);
     float *head = tail + WALK_TAIL_CAP * MERGED_STRIDE;
-    float *sh_rowM = head + WALK_HEAD_CAP * MERGED_STRIDE;  // [4][RB]
-    float *sh_rowS = sh_rowM + 4 * RB;
-    for (int k = threadIdx.x; k < 4 * RB; k += WALK_WG) {
+    double *step = reinterpret_cast<double *>(head + WALK_HEAD_CAP * MERGED_STRIDE);
+    float *sh_rowM = reinterpret_cast<float *>(step + (WALK_WAVES - 1) * WALK_STEP * 64);
+    float *sh_rowS = sh_rowM + walk_rows(RB);
+    for (int k = threadIdx.x; k < walk_rows(RB); k += WALK_WG) {
         sh_rowM[k] = -INFINITY;
         sh_rowS[k] = 0.0f;
     }
+    // the wave's rows within the item, top .. bot: whole groups of four
+    const int groups = (nrows + 3) / 4, per = (groups + WALK_WAVES - 1) / WALK_WAVES;
+    auto top_of = [&](int k) { return min(nrows, 4 * (groups - k * per)) - 1; };  // < 0: no rows
+    const int top = top_of(wave), next = top_of(wave + 1), bot = max(next + 1, 0);
 
-    auto column = [&](int nn) {
-        WalkCol wc;
-        const uint32_t tau = td.tau + (uint32_t)nn * td.dtau;
+    WalkCol wc;
+    {
+        const uint32_t tau = td.tau + (uint32_t)min(n, N_tau - 1) * td.dtau;
         wc.ratau = (double)TA / (double)tau;
         wc.Q = (int)(3u * tau / TA);
         wc.R = 3u * tau % TA;
-        return wc;
-    };
-    WalkCol wc = column(min(n, N_tau - 1));
+    }
     wc.rho[1] = exp(-wc.ratau);
     wc.rho[0] = wc.rho[1] * wc.rho[1];
     wc.lead[0] = exp(-(double)(wc.Q - 1) * wc.ratau);
 #pragma unroll
     for (int k = 1; k < 4; k++) wc.lead[k] = wc.lead[k - 1] * wc.rho[1];
-    const WalkCol wfirst = column(col0), wlast = column(min(col0 + TILE_COLS, N_tau) - 1);
+    // the last lane's window is the longest, the first one's the shortest
+    const int Q0 = __builtin_amdgcn_readlane(wc.Q, 0), Q63 = __builtin_amdgcn_readlane(wc.Q, 63);
 
     const int dq = (int)(td.dt0 / TA);
     const uint32_t dphi = td.dt0 % TA;
-    auto row_at = [&](int m) {
-        const uint32_t T = td.t0 - td.t_min + (uint32_t)m * td.dt0;
+    auto row_at = [&](int rl) {
+        const uint32_t T = td.t0 - td.t_min + (uint32_t)(row0 + rl) * td.dt0;
         return WalkRow{(int)(T / TA), T % TA};
     };
-    WalkRow row = row_at(row0 + nrows - 1);
-    const WalkRow bottom = row_at(row0);
-    int hi = row.hi(wc, TA);
-    // the last lane's window is the longest, the first one's the shortest
-    const int Q63 = __builtin_amdgcn_readlane(wc.Q, 63);
+    const WalkRow first = row_at(nrows - 1), bottom = row_at(0);
     double E[NC];
     float kinds = 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; c++) E[c] = 0.0;
     bool odd = false;  // an infinity or NaN in reach of the block (block-uniform)
-    {   // the direct sum at the top row, chunk by chunk over the block's longest
-        // window: the waves of a group take equal shares of each chunk
-        const int lo = row.lo();
-        const int L = active ? hi - lo + 1 : 0;
+    {   // the direct sum at the item's top row, chunk by chunk over its longest
+        // window: the waves take equal shares of each chunk
+        const int lo = first.lo();
+        const int L = first.hi(wc, TA) - lo + 1;
         const int Lmin = __builtin_amdgcn_readlane(L, 0), Lmax = __builtin_amdgcn_readlane(L, 63);
-        const int Lblk = min(row.hi(wlast, TA) - lo + 1, N - lo);
+        const int Lblk = min(Lmax, N - lo);
         for (int c0 = 0; c0 < Lblk; c0 += WALK_CHUNK) {  // block-uniform
             const int nc = min(WALK_CHUNK, Lblk - c0);
             odd |= __syncthreads_or(walk_stage<WALK_CHUNK>(
                 tail, X + (int64_t)(lo + c0) * MERGED_STRIDE, nc));
-            const int share = (nc + W - 1) / W;
-            const int s0 = w * share, cnt = min(min(share, nc - s0), Lmax - c0 - s0);
+            const int share = (nc + WALK_WAVES - 1) / WALK_WAVES;
+            const int s0 = wave * share, cnt = min(share, nc - s0);
             if (cnt > 0 && !odd) {  // uniform
                 double H[NC];
                 float kh = 0.0f;
@@ -1812,7 +1818,7 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
             __syncthreads();
         }
     }
-    if (W > 1) {  // add the group's parts, in one order on all of its waves
+    {   // add the parts, in one order on all waves
         double *mine = comb + wave * MERGED_STRIDE * 64 + lane;
 #pragma unroll
         for (int c = 0; c < NC; c++) mine[c * 64] = E[c];
@@ -1821,28 +1827,36 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
 #pragma unroll
         for (int c = 0; c < NC; c++) E[c] = 0.0;
         kinds = 0.0f;
-        for (int k = 0; k < W; k++) {
-            const double *part = comb + (g * W + k) * MERGED_STRIDE * 64 + lane;
+#pragma unroll 2
+        for (int k = 0; k < WALK_WAVES; k++) {
+            const double *part = comb + k * MERGED_STRIDE * 64 + lane;
 #pragma unroll
             for (int c = 0; c < NC; c++) E[c] += part[c * 64];
             kinds += (float)part[NC * 64];
         }
         __syncthreads();  // comb is staged over
     }
-    // atoms that leave and enter in the item's row steps: block-uniform ranges below N
-    const int tail_lo = bottom.q + wfirst.Q;  // hi' + 1 at least
-    const int tail_n = min(N, row.q + wlast.Q + 2) - tail_lo;
+    // atoms that leave and enter between the item's rows: block-uniform ranges below N
+    const int tail_lo = bottom.q + Q0;  // hi' + 1 at least
+    const int tail_n = min(N, first.q + Q63 + 2) - tail_lo;
     const int head_lo = bottom.lo();
-    const int head_n = min(N, row.lo()) - head_lo;
+    const int head_n = min(N, first.lo()) - head_lo;
     const bool in_lds = tail_n < WALK_TAIL_CAP && head_n <= WALK_HEAD_CAP;
+    bool head_odd = false;
     if (in_lds) {
         // slot 0 holds zeros, for the lanes with no atom to take out
         if (threadIdx.x < MERGED_STRIDE) tail[threadIdx.x] = 0.0f;
         walk_stage<WALK_TAIL_CAP>(tail + MERGED_STRIDE, X + (int64_t)tail_lo * MERGED_STRIDE,
                                   tail_n);
-        walk_stage<WALK_HEAD_CAP>(head, X + (int64_t)head_lo * MERGED_STRIDE, head_n);
+        head_odd = walk_stage<WALK_HEAD_CAP>(head, X + (int64_t)head_lo * MERGED_STRIDE, head_n);
+    } else {
+        for (int k = threadIdx.x; k < head_n; k += WALK_WG)
+            head_odd |= X[(int64_t)(head_lo + k) * MERGED_STRIDE + NC] == BIN_ODD;
     }
-    __syncthreads();
+    odd |= __syncthreads_or(head_odd);
+    // sum every row directly: where an atom is not finite, or the steps are
+    // longer than the windows
+    const bool direct = odd || dq >= Q63;
     auto load = [&](float (&x)[MERGED_STRIDE], const float *sh, int64_t at, bool some) {
         if (in_lds) {
 #pragma unroll
@@ -1852,36 +1866,82 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
             for (int c = 0; c < MERGED_STRIDE; c++) x[c] = some ? X[at * MERGED_STRIDE + c] : 0.0f;
         }
     };
+    // sum += rho^(l - lo2) x_l for the entering atoms l = lo2 .. lo - 1
+    auto enter = [&](int lo, int lo2, double (&sum)[NC], float &k) {
+        for (int l = min(lo, N) - 1; l >= lo2; l--) {
+            float x[MERGED_STRIDE];
+            load(x, head + (l - head_lo) * MERGED_STRIDE, l, true);
+            k += x[NC];
+#pragma unroll
+            for (int c = 0; c < NC; c++) sum[c] = fma(wc.rho[c < 3 ? 0 : 1], sum[c], (double)x[c]);
+        }
+    };
+
+    WalkRow row = row_at(max(top, 0));
+    int hi = row.hi(wc, TA);
+    if (!direct) {  // block-uniform
+        if (next >= 0) {
+            const WalkRow to = row_at(next);
+            const int lo = row.lo(), lo2 = to.lo(), hi2 = to.hi(wc, TA), last = min(hi, N - 1);
+            double D[NC], O[NC];
+            float kd = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NC; c++) D[c] = O[c] = 0.0;
+            enter(lo, lo2, D, kd);
+            for (int i = hi2 + row.q - to.q + 2; i > hi2; i--) {  // (the same count on every lane)
+                const bool out = i <= last;
+                float x[MERGED_STRIDE];
+                load(x, tail + (out ? i - tail_lo + 1 : 0) * MERGED_STRIDE, i, out);
+                kd -= x[NC];
+#pragma unroll
+                for (int c = 0; c < NC; c++) O[c] = fma(wc.rho[c < 3 ? 0 : 1], O[c], (double)x[c]);
+            }
+            const double w1 = exp(-(double)(hi2 + 1 - lo2) * wc.ratau), w2 = w1 * w1;
+            double *mine = step + wave * WALK_STEP * 64 + lane;
+#pragma unroll
+            for (int c = 0; c < NC; c++) mine[c * 64] = fma(c < 3 ? -w2 : -w1, O[c], D[c]);
+            mine[NC * 64] = (double)kd;
+            mine[(NC + 1) * 64] = exp(-(double)(lo - lo2) * wc.ratau);
+        }
+        __syncthreads();
+        if (top >= 0) {
+#pragma unroll 2
+            for (int k = 0; k < wave; k++) {
+                const double *part = step + k * WALK_STEP * 64 + lane;
+                const double m1 = part[(NC + 1) * 64], m2 = m1 * m1;
+                kinds += (float)part[NC * 64];
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const double e = fma(c < 3 ? m2 : m1, E[c], part[c * 64]);
+                    E[c] = kinds == 0.0f ? 0.0 : e;
+                }
+            }
+        }
+    } else if (top >= 0) {
+        walk_row_sum(X, N, wc, row.lo(), hi - row.lo() + 1, row.q + Q63 + 2 - row.lo(), E, kinds);
+    }
 
     Reducer<BTSG, 1> red;
     red.init();
     bool single = false;
-    // sum every row directly: where an atom is not finite, or the steps are
-    // longer than the windows
-    bool direct = odd || dq >= Q63;
-    if (odd && active)
-        walk_row_sum(X, N, wc, row.lo(), hi - row.lo() + 1, row.q + Q63 + 2 - row.lo(), E, kinds);
     const int colidx[1] = {n};
-    for (int k4 = active ? (nrows - 1) / 4 : -1; k4 >= 0; k4--) {
-        const bool mine = k4 % W == w;  // uniform
+    for (int r4 = top >= 0 ? top / 4 * 4 : -1; r4 >= bot; r4 -= 4) {
         float F4[4][1];
 #pragma unroll
         for (int j = 3; j >= 0; j--) {
-            const int m = row0 + 4 * k4 + j;
+            const int m = row0 + r4 + j;
             F4[j][0] = -INFINITY;
-            if (4 * k4 + j >= nrows) continue;  // uniform
-            if (mine) {
-                const float f = cell_F(E[0], E[1], E[2], E[3], E[4], E[5], E[6]);
-                if (valid) {
-                    Ft[(int64_t)m * N_tau + n] = f;
-                    F4[j][0] = f;
-                }
-                if (STRICT) {
-                    const int i0 = min(row.q + (row.phi + TA / 2 >= TA), N - 1);
-                    single |= valid && min(hi, N - 1) == i0;
-                }
+            if (r4 + j >= nrows) continue;  // uniform
+            const float f = cell_F(E[0], E[1], E[2], E[3], E[4], E[5], E[6]);
+            if (valid) {
+                Ft[(int64_t)m * N_tau + n] = f;
+                F4[j][0] = f;
             }
-            if (m == row0) continue;
+            if (STRICT) {
+                const int i0 = min(row.q + (row.phi + TA / 2 >= TA), N - 1);
+                single |= valid && min(hi, N - 1) == i0;
+            }
+            if (r4 + j == bot) continue;
             // to row m - 1
             const int lo = row.lo();
             row.q -= dq;
@@ -1891,20 +1951,10 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
             }
             row.phi -= dphi;
             const int lo2 = row.lo(), hi2 = row.hi(wc, TA);
-            if (!direct) {
-                for (int l = min(lo, N) - 1; l >= lo2; l--) {
-                    float x[MERGED_STRIDE];
-                    load(x, head + (l - head_lo) * MERGED_STRIDE, l, true);
-                    direct |= __any(x[NC] == BIN_ODD);  // (the same on every lane)
-                    kinds += x[NC];
-#pragma unroll
-                    for (int c = 0; c < NC; c++)
-                        E[c] = fma(wc.rho[c < 3 ? 0 : 1], E[c], (double)x[c]);
-                }
-            }
             if (direct) {  // uniform
                 walk_row_sum(X, N, wc, lo2, hi2 - lo2 + 1, row.q + Q63 + 2 - lo2, E, kinds);
             } else {
+                enter(lo, lo2, E, kinds);
                 const int lead = row.end(wc, TA) + (row.phi == 0);
                 const double wa = lead & 1 ? wc.lead[1] : wc.lead[0];
                 const double wb = lead & 1 ? wc.lead[3] : wc.lead[2];
@@ -1929,12 +1979,10 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
             }
             hi = hi2;
         }
-        if (mine)
-            red.add(F4, row0 + 4 * k4, colidx, N_tau, lane, 4 * k4, sh_rowM + g * RB,
-                    sh_rowS + g * RB);
+        red.add(F4, row0 + r4, colidx, N_tau, lane, r4, sh_rowM, sh_rowS);
     }
     if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
-    // combine: a column belongs to the waves of its group, a row to one wave of each group
+    // combine: a column belongs to all waves, a row to one
     wave_argmax(red.best, red.bidx);
     float stot = 0.0f;
     if (BTSG) stot = wave_sum(red.total());
@@ -1949,20 +1997,15 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
     float M = sh_M[0];
     for (int k = 1; k < WALK_WAVES; k++) M = fmaxf(M, sh_M[k]);
     if (BTSG) {
-        if (valid && w == 0) {
+        if (valid && wave == 0) {
             float S = 0.0f;
-            for (int k = 0; k < W; k++)
-                if (sh_M[wave + k] != -INFINITY)
-                    S += sh_col[wave + k][lane] * exp2_diff(sh_M[wave + k], M);
+            for (int k = 0; k < WALK_WAVES; k++)
+                if (sh_M[k] != -INFINITY) S += sh_col[k][lane] * exp2_diff(sh_M[k], M);
             colpart[td.colpart_off + (int64_t)it.rb * N_tau + n] = S;
         }
-        for (int rl = threadIdx.x; rl < nrows; rl += WALK_WG) {
-            float S = 0.0f;
-            for (int k = 0; k < groups; k++)
-                if (sh_rowM[k * RB + rl] != -INFINITY)
-                    S += sh_rowS[k * RB + rl] * exp2_diff(sh_rowM[k * RB + rl], M);
-            rowpart[td.rowpart_off + (int64_t)it.cb * td.N_t0 + row0 + rl] = S;
-        }
+        for (int rl = threadIdx.x; rl < nrows; rl += WALK_WG)
+            rowpart[td.rowpart_off + (int64_t)it.cb * td.N_t0 + row0 + rl] =
+                sh_rowM[rl] != -INFINITY ? sh_rowS[rl] * exp2_diff(sh_rowM[rl], M) : 0.0f;
     }
     if (threadIdx.x == 0) {
         float bv = sh_best[0];
@@ -3231,6 +3274,10 @@ struct tcw_plan {
     // when set, device buffers are views into this memory (tcw_map_noalloc)
     char *arena = nullptr;
     size_t arena_bytes = 0;
+    bool arena_short = false;  // the last plan needed more than arena_bytes
+    // the layout with the least scratch: long row blocks, and the per-cell
+    // kernels (16 rows x 256 columns) off the grid
+    bool compact = false;
     void reset() {
         tmpl.clear();
         segs.clear();
@@ -3430,7 +3477,7 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         // pass of rows by 32-bit byte offsets)
         // off the grid: the sliding sum with any steps
         td.walk = !(p.flags & TCW_FLAG_GENERIC) && w.t0 >= t_min && end < (1ull << 32) &&
-                  w.tau >= TAtom;
+                  w.tau >= TAtom && !p.compact;
         if (!(p.flags & TCW_FLAG_GENERIC) && on_grid && end < (1ull << 32) &&
             N_tau <= (int64_t)1 << 20) {
             mode = MODE_EXP_FAST;
@@ -3457,12 +3504,15 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
             td.a = (int32_t)(w.dt0 / TAtom);
             td.q0 = (int32_t)(((uint64_t)w.t0 - t_min + half) / TAtom);
             td.q00 = (int32_t)(((uint64_t)w.t0 + w.tau - t_min + half) / TAtom);
+        } else if (p.compact) {
+            td.walk = 0;
         }
     }
     td.mode = mode;
     const int req = p.rows_req[mode];  // the plan's tuned rows, 0 = built-in choice
     int rb = req > 0 ? req : RB_DEFAULT[mode];
-    if ((mode == MODE_RECT_FAST || (mode == MODE_RECT_GENERIC && td.walk)) && req <= 0) {
+    if ((mode == MODE_RECT_FAST || (mode == MODE_RECT_GENERIC && td.walk)) && req <= 0 &&
+        !p.compact) {
         // few or small maps (the single-map call): fewer rows per item, so
         // that the batch's items cover the CUs (about SMALL_BATCH_ITEMS of them
         // if the templates are alike)
@@ -3475,9 +3525,9 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     if (mode == MODE_EXP_DIRECT && td.walk && req <= 0) {
         // enough items for the chip, and otherwise long ones: each starts with
         // a direct sum
-        const double ncb = (double)((N_tau + TILE_COLS - 1) / TILE_COLS);
+        const double ncb = (double)((N_tau + WALK_TILE - 1) / WALK_TILE);
         const double want = (double)N_t0 * ncb * (double)p.T / (double)WALK_ITEMS;
-        rb = std::min(WALK_MAX_ROWS, std::max(16, ((int)std::min(want, 1e6) + 15) / 16 * 16));
+        rb = std::min(WALK_MAX_ROWS, std::max(32, ((int)std::min(want, 1e6) + 31) / 32 * 32));
     }
     if (mode == MODE_EXP_FAST && req <= 0) {
         const int64_t pairs = p.T * ((N_tau + TILE_COLS - 1) / TILE_COLS);
@@ -3495,7 +3545,7 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         rb = (int)std::min<int64_t>(rb, (N_t0 + 15) / 16 * 16);
     td.rb_rows = rb;
     td.n_rowblk = (uint32_t)((N_t0 + rb - 1) / rb);
-    td.tile = TILE_COLS;
+    td.tile = mode == MODE_EXP_DIRECT && td.walk ? WALK_TILE : TILE_COLS;
     if (mode == MODE_RECT_GENERIC && td.walk) {
         auto bytes = [&](int tile) {
             return step_bytes(step_shape(rb, tile, td.N_tau, td.dt0, td.dtau, TAtom));
@@ -3682,7 +3732,8 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
             if (off + a <= p.arena_bytes) b.set_view(p.arena + off, a);
             off += a;
         });
-        if (off > p.arena_bytes)
+        p.arena_short = off > p.arena_bytes;
+        if (p.arena_short)
             return fail(TCW_ERR_INVALID, "this map needs " + std::to_string(off) +
                                              " bytes of scratch; the static scratch holds " +
                                              std::to_string(p.arena_bytes) + " bytes");
@@ -4318,12 +4369,19 @@ int tcw_map_noalloc(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win
     hipStream_t st = (hipStream_t)stream;
     // the plan's buffers become views into the scratch (plan_finish), or the
     // call fails before anything is queued when the map needs more
-    rc = plan_single(h, h->noalloc, atoms, win, flags, st, "tcw_map_noalloc");
+    tcw_plan &p = h->noalloc;
+    p.compact = p.arena_short = false;
+    rc = plan_single(h, p, atoms, win, flags, st, "tcw_map_noalloc");
+    if (rc && p.arena_short) {
+        // off the grid the fast kernels' partials take up to a quarter more a
+        // cell (64 columns an item): the map may still fit in the general ones'
+        p.compact = true;
+        rc = plan_single(h, p, atoms, win, flags, st, "tcw_map_noalloc");
+    }
     if (rc) return rc;
     // every scratch byte a kernel reads is written earlier in the same call
     // (the stage kernel also clears the single-atom flag), so nothing is cleared
-    return launch_all(h->noalloc, atoms->ts, atoms->cols, atoms->col_stride, F_mn_dev,
-                      stats_dev, st);
+    return launch_all(p, atoms->ts, atoms->cols, atoms->col_stride, F_mn_dev, stats_dev, st);
 }
 
 int tcw_merge_plan_create(tcw_handle *h, const tcw_batch_desc *d, tcw_merge_plan **out,
