@@ -2534,109 +2534,57 @@ __global__ __launch_bounds__(INIT_WG) void exp_init_kernel(const TmplDev *__rest
     }
 }
 
-// Per tau column: E at every chunk top.  Work items (t, -, cb); one wave per
-// column, 4 columns per workgroup.  With f_s(x) = mult x + Y(s) (mult = the
-// weight factor of one chunk of rows), the chunk tops are V(n_seg-1) = the
-// direct sum and V(s-1) = f_s(V(s)), a first-order linear recurrence with a
-// constant coefficient: lane l of a 64-chunk tile holds Y(s_hi - l) and a
-// log-depth (Kogge-Stone) scan, x_l += mult^d x_{l-d} for d = 1 .. 32, gives
-// V(s_hi - l) = mult^l V(s_hi) + x_{l-1}; tiles run from the top chunk down,
-// each carrying V(s_hi - 64) = mult^64 V(s_hi) + x_63.  Slot s holds Y(s) on
-// entry and V(s) on exit (slot 0 has no Y).
-constexpr int SCAN_COLS = WG / 64;  // columns per workgroup
-
-__global__ __launch_bounds__(WG) void exp_scan_kernel(const TmplDev *__restrict__ tds,
-                                                      const ItemDev *__restrict__ items,
-                                                      double *__restrict__ etab) {
-    const ItemDev it = items[blockIdx.x / (TILE_COLS / SCAN_COLS)];
-    const TmplDev td = tds[it.t];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int n = it.cb * TILE_COLS + (int)(blockIdx.x % (TILE_COLS / SCAN_COLS)) * SCAN_COLS + wave;
-    if (n >= (int)td.N_tau) return;  // wave-uniform
-    const double tau = (double)td.tau + (double)n * (double)td.dtau;
-    const double xstep = (double)td.TAtom * (double)td.a * (double)td.rb_rows / tau;
-    // mult[k]^d for the scan steps d = 1, 2, ..., 32 (k = 0: A, B, C; k = 1: Fa, Fb)
-    double pw[2][6];
-    pw[1][0] = exp(-xstep);
-    pw[0][0] = pw[1][0] * pw[1][0];
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-#pragma unroll
-        for (int d = 1; d < 6; d++) pw[k][d] = pw[k][d - 1] * pw[k][d - 1];
-    // mult^l for this lane, and mult^64
-    double ml[2], m64[2];
-    ml[1] = exp(-xstep * (double)lane);
-    ml[0] = ml[1] * ml[1];
-    m64[0] = pw[0][5] * pw[0][5];
-    m64[1] = pw[1][5] * pw[1][5];
-    double carry[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) {  // top chunk: the direct sum's parts
-        carry[c] = 0.0;
-        if (!td.init_empty)
-            for (int pp = 0; pp < INIT_PARTS; pp++)
-                carry[c] += expf_etab(etab, td, td.n_seg + pp, c)[n];
-    }
-    for (int s_hi = td.n_seg - 1; s_hi >= 0; s_hi -= 64) {
-        const int sl = s_hi - lane;
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int k = c < 3 ? 0 : 1;
-            double *slot = expf_etab(etab, td, max(sl, 0), c) + n;
-            double x = sl >= 1 ? *slot : 0.0;
-#pragma unroll
-            for (int d = 0; d < 6; d++) {
-                const double y = __shfl_up(x, 1 << d);
-                if (lane >= (1 << d)) x = fma(pw[k][d], y, x);
-            }
-            double sx = __shfl_up(x, 1);
-            if (lane == 0) sx = 0.0;
-            if (sl >= 0) *slot = fma(ml[k], carry[c], sx);
-            const double x63 = __shfl(x, 63);
-            carry[c] = fma(m64[k], carry[c], x63);
-        }
-    }
-}
-
-// The same scan, sequential along the chunks: one thread per tau column (its
-// loads and stores coalesce across the columns).  For batches of many
-// templates with few chunks each, where one wave per column would leave most
-// lanes idle.
+// Per tau column: E at every chunk top.  Work items (t, -, cb).  With mult the
+// weight factor of one chunk of rows, the chunk tops are V(n_seg-1) = the
+// direct sum and V(s-1) = mult V(s) + Y(s).  Slot s holds Y(s) on entry and
+// V(s) on exit (slot 0 has no Y).  A thread per (column, sum): its loads and
+// stores coalesce over the columns, and SCAN_AHEAD slots are loaded together,
+// since the loads' latency, not the recurrence, is the bound.
+// One map of 2000 x 2000 cells (62 chunks): 13.4 us with a wave per column and a
+// lane per chunk (log depth, but every lane on its own cache line), now 7.2
+// (8.0 with 16 slots ahead, 9.4 with 8); 32 of 1000 x 1000: the three
+// recurrence kernels 415, now 301.
 constexpr int SCAN_WG = 64;
 constexpr int SCAN_SPLIT = TILE_COLS / SCAN_WG;
+constexpr int SCAN_AHEAD = 32;
 
-__global__ __launch_bounds__(SCAN_WG) void exp_scan_seq_kernel(const TmplDev *__restrict__ tds,
-                                                               const ItemDev *__restrict__ items,
-                                                               double *__restrict__ etab) {
-    const ItemDev it = items[blockIdx.x / SCAN_SPLIT];
+__global__ __launch_bounds__(SCAN_WG) void exp_scan_kernel(const TmplDev *__restrict__ tds,
+                                                           const ItemDev *__restrict__ items,
+                                                           double *__restrict__ etab) {
+    const ItemDev it = items[blockIdx.x / (SCAN_SPLIT * NC)];
     const TmplDev td = tds[it.t];
-    const int n = it.cb * TILE_COLS + (int)(blockIdx.x % SCAN_SPLIT) * SCAN_WG + threadIdx.x;
+    const int part = (int)(blockIdx.x % (SCAN_SPLIT * NC));
+    const int c = part / SCAN_SPLIT;
+    const int n = it.cb * TILE_COLS + part % SCAN_SPLIT * SCAN_WG + (int)threadIdx.x;
     if (n >= (int)td.N_tau) return;
     const double tau = (double)td.tau + (double)n * (double)td.dtau;
     const double steps = (double)td.a * td.rb_rows;
     const double m1 = exp(-(double)td.TAtom * steps / tau);
-    const double mult[2] = {m1 * m1, m1};
-    double E[NC];
+    const double mult = c < 3 ? m1 * m1 : m1;
+    double E = 0.0;
+    if (!td.init_empty) {  // top chunk: the direct sum's parts
+        double y[INIT_PARTS];
 #pragma unroll
-    for (int c = 0; c < NC; c++) {  // top chunk: the direct sum's parts
-        E[c] = 0.0;
-        if (!td.init_empty)
-            for (int pp = 0; pp < INIT_PARTS; pp++) E[c] += expf_etab(etab, td, td.n_seg + pp, c)[n];
+        for (int pp = 0; pp < INIT_PARTS; pp++) y[pp] = expf_etab(etab, td, td.n_seg + pp, c)[n];
+#pragma unroll
+        for (int pp = 0; pp < INIT_PARTS; pp++) E += y[pp];
     }
-    for (int s = td.n_seg - 1; s >= 1; s--) {
+    double *slot0 = expf_etab(etab, td, 0, c) + n;
+    const int64_t stride = (int64_t)NC * td.N_tau;
+    for (int s = td.n_seg - 1; s >= 1; s -= SCAN_AHEAD) {
+        double Y[SCAN_AHEAD];
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            double *slot = expf_etab(etab, td, s, c) + n;
-            const double Y = *slot;
-            *slot = E[c];
-            E[c] = fma(mult[c < 3 ? 0 : 1], E[c], Y);
-        }
+        for (int u = 0; u < SCAN_AHEAD; u++)  // (slot 1 again past the end)
+            Y[u] = slot0[max(s - u, 1) * stride];
+#pragma unroll
+        for (int u = 0; u < SCAN_AHEAD; u++)
+            if (s - u >= 1) {  // uniform
+                slot0[(s - u) * stride] = E;
+                E = fma(mult, E, Y[u]);
+            }
     }
-#pragma unroll
-    for (int c = 0; c < NC; c++) expf_etab(etab, td, 0, c)[n] = E[c];
+    slot0[0] = E;
 }
-
 
 // Rows st .. sb of a chunk (one pass) in groups of 4 (the pass's rows are a
 // multiple of 4), reduced together.  Rows past the map (m > m_hi, only in a
@@ -3243,7 +3191,6 @@ struct tcw_plan {
     std::vector<int32_t> tmpl_list;
     int64_t exp_max_N = 0;
     bool exp_init_needed = false;  // some exp template has a non-empty direct sum
-    bool exp_scan_wave = false;    // the wave-per-column chunk scan (few, long columns)
     int64_t mode_begin[MODE_COUNT + 1] = {0, 0, 0, 0, 0};
     int64_t prefix_doubles = 0, merged_floats = 0, rowpart_n = 0, colpart_n = 0;
     int64_t etab_doubles = 0;
@@ -3289,7 +3236,6 @@ struct tcw_plan {
         for (auto &r : rect_tmpls) r.clear();
         exp_max_N = 0;
         exp_init_needed = false;
-        exp_scan_wave = false;
         prefix_doubles = merged_floats = rowpart_n = colpart_n = F_total = 0;
         etab_doubles = 0;
         max_lds_bytes = 0;
@@ -3579,11 +3525,6 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
                         p.init_items.push_back(ItemDev{(int32_t)t, part, (int32_t)cbk,
                                                        init_work(td, cbk, part)});
             }
-            // few (template, column block) pairs, each with many chunks: a
-            // wave per column scans the chunks in log depth; otherwise a
-            // thread per column walks them (coalesced, no idle lanes)
-            if (p.T * (int64_t)td.n_colblk < DIRECT_INIT_MIN_BLOCKS && nseg >= 16)
-                p.exp_scan_wave = true;
             td.etab_off = p.etab_doubles;
             p.etab_doubles += (nseg + INIT_PARTS) * NC * N_tau;
             for (int64_t sg = 1; sg < nseg; sg++)
@@ -3916,16 +3857,10 @@ int launch_all(tcw_plan &p, const uint32_t *ts, const float *cols, int64_t cstri
         TCW_HIP_TRY(hipEventRecord(p.ev_join, p.side));
         TCW_HIP_TRY(hipStreamWaitEvent(st, p.ev_join, 0));
     }
-    if (!p.col_items.empty() && !p.exp_scan_wave)
-        hipLaunchKernelGGL(exp_scan_seq_kernel, dim3((unsigned)(p.col_items.size() * SCAN_SPLIT)),
+    if (!p.col_items.empty())
+        hipLaunchKernelGGL(exp_scan_kernel, dim3((unsigned)(p.col_items.size() * SCAN_SPLIT * NC)),
                            dim3(SCAN_WG), 0, st, (const TmplDev *)p.d_tmpl.p,
                            (const ItemDev *)p.d_col_items.p, (double *)p.d_etab.p);
-    if (!p.col_items.empty() && p.exp_scan_wave)
-        hipLaunchKernelGGL(exp_scan_kernel,
-                           dim3((unsigned)(p.col_items.size() * (TILE_COLS / SCAN_COLS))),
-                           dim3(WG), 0, st,
-                           (const TmplDev *)p.d_tmpl.p, (const ItemDev *)p.d_col_items.p,
-                           (double *)p.d_etab.p);
     if (ev) TCW_HIP_TRY(hipEventRecord(ev[1], st));
     if (btsg) {
         if (strict)
