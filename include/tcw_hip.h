@@ -135,8 +135,9 @@ int tcw_map_host(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win,
  * the reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The same
  * kernels as tcw_map, with every intermediate buffer carved from the static
- * scratch of h's device (looked up once by tcw_create); a map off the atom
- * grid whose partials only fit in the per-cell kernels' layout takes those.
+ * scratch of h's device (looked up once by tcw_create); a map whose partials or
+ * chunk tables only fit in a plainer layout (off the atom grid the per-cell
+ * kernels) takes that one, which alone decides what the scratch accepts.
  * stats_dev: DEVICE tcw_stats, written by the last kernel; the call does not
  * wait for the device (read stats_dev after synchronising `stream`; under
  * TCW_FLAG_LAL_STRICT check stats_dev->single_atom yourself).

@@ -81,7 +81,21 @@ constexpr int64_t SMALL_BATCH_ITEMS = 2048;
 // 132; 64 of 500 x 500 1004 | 583 | 373 | 352.
 constexpr int64_t WALK_ITEMS = 256;
 constexpr int WALK_MAX_ROWS = 256;
-constexpr int EXP_SMALL_BATCH_ROWS = 64;    // exp rows when untuned and under 256 column blocks
+// Exp rows on the atom grid when untuned and under DIRECT_INIT_MIN_BLOCKS column
+// blocks: about EXP_SMALL_CHUNKS chunks over all columns, those above the map
+// included (they are walked too): shorter ones leave more to the scan and to
+// finalize, longer ones leave CUs idle.  Measured (pass, us, at 16 | 32 | 64 |
+// 128 | 256 rows): one map of 2000 x 2000 cells 137 | 100 | 82 | 84 | 124; one of
+// 150 x 150 39 | 43 | 51 | 69 | 84; 8 of 300 x 150 46 | 45 | 54 | 71 | 113; 128 of
+// 300 x 150 172 | 124 | 116 | 107 | 123; 32 of 1000 x 1000 876 | 542 | 411 | 363 |
+// 354.
+constexpr int64_t EXP_SMALL_CHUNKS = 512;
+constexpr int EXP_SMALL_MIN_ROWS = 16, EXP_SMALL_MAX_ROWS = 256;
+// Rows of the layout that bounds tcw_map_noalloc's maps (tcw_plan::compact):
+// rect items of 16 to 128 rows, about 512 of them, exp chunks of 64 under
+// DIRECT_INIT_MIN_BLOCKS column blocks.
+constexpr int COMPACT_RECT_ROWS = 128, COMPACT_EXP_ROWS = 64;
+constexpr int64_t COMPACT_RECT_ITEMS = 512;
 
 struct TmplDev {
     int64_t seg_begin, seg_end;  // detector segments of this template
@@ -3222,9 +3236,11 @@ struct tcw_plan {
     char *arena = nullptr;
     size_t arena_bytes = 0;
     bool arena_short = false;  // the last plan needed more than arena_bytes
-    // the layout with the least scratch: long row blocks, and the per-cell
-    // kernels (16 rows x 256 columns) off the grid
+    // the layout that decides what the arena accepts, so that a faster one
+    // neither refuses nor accepts other maps: COMPACT_* rows and, off the grid,
+    // the per-cell kernels
     bool compact = false;
+    bool dry = false;  // stop once the scratch is sized
     void reset() {
         tmpl.clear();
         segs.clear();
@@ -3457,15 +3473,18 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     td.mode = mode;
     const int req = p.rows_req[mode];  // the plan's tuned rows, 0 = built-in choice
     int rb = req > 0 ? req : RB_DEFAULT[mode];
-    if ((mode == MODE_RECT_FAST || (mode == MODE_RECT_GENERIC && td.walk)) && req <= 0 &&
-        !p.compact) {
+    if ((mode == MODE_RECT_FAST || (mode == MODE_RECT_GENERIC && td.walk)) && req <= 0) {
         // few or small maps (the single-map call): fewer rows per item, so
         // that the batch's items cover the CUs (about SMALL_BATCH_ITEMS of them
         // if the templates are alike)
-        const int most = mode == MODE_RECT_FAST ? RB_DEFAULT[mode] : STEP_RB;
+        const int most = p.compact                ? COMPACT_RECT_ROWS
+                         : mode == MODE_RECT_FAST ? RB_DEFAULT[mode]
+                                                  : STEP_RB;
         const double ncb = (double)((N_tau + TILE_COLS - 1) / TILE_COLS);
         const double want = (double)N_t0 * ncb * (double)p.T /
-                            (double)(mode == MODE_RECT_FAST ? SMALL_BATCH_ITEMS : STEP_ITEMS);
+                            (double)(p.compact                ? COMPACT_RECT_ITEMS
+                                     : mode == MODE_RECT_FAST ? SMALL_BATCH_ITEMS
+                                                              : STEP_ITEMS);
         rb = want >= most ? most : std::max(16, ((int)std::ceil(want) + 15) / 16 * 16);
     }
     if (mode == MODE_EXP_DIRECT && td.walk && req <= 0) {
@@ -3478,7 +3497,11 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     if (mode == MODE_EXP_FAST && req <= 0) {
         const int64_t pairs = p.T * ((N_tau + TILE_COLS - 1) / TILE_COLS);
         if (pairs < DIRECT_INIT_MIN_BLOCKS) {
-            rb = EXP_SMALL_BATCH_ROWS;  // few column blocks: shorter chunks, more of them
+            const int64_t span = ((int64_t)td.H - td.k00 + td.a - 1) / std::max(td.a, 1);
+            const int64_t want = pairs * std::max<int64_t>(span, N_t0) / EXP_SMALL_CHUNKS;
+            rb = (int)std::min<int64_t>(EXP_SMALL_MAX_ROWS,
+                                        std::max<int64_t>(EXP_SMALL_MIN_ROWS, (want + 15) / 16 * 16));
+            if (p.compact) rb = COMPACT_EXP_ROWS;
         } else {
             // about EXP_TARGET_ITEMS work items: one chunk per column when the
             // batch has that many column blocks
@@ -3678,6 +3701,7 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
             return fail(TCW_ERR_INVALID, "this map needs " + std::to_string(off) +
                                              " bytes of scratch; the static scratch holds " +
                                              std::to_string(p.arena_bytes) + " bytes");
+        if (p.dry) return TCW_OK;
     } else {
         plan_buffers(p, [&](DevBuf &b, size_t bytes) {
             if (!rc) rc = b.ensure(bytes);
@@ -4222,6 +4246,26 @@ int plan_single(tcw_handle *h, tcw_plan &p, const tcw_atoms *atoms, const tcw_wi
     return plan_build(p, h->device, &d, flags, nullptr, st, true);
 }
 
+// An upper bound of the compact layout's scratch lies below `room` (the bound is
+// a few times too high; it spares a map that is small anyway a second plan).
+bool surely_fits(const tcw_atoms *atoms, const tcw_window *win, size_t room) {
+    if (atoms->TAtom < 2 || atoms->t_max < atoms->t_min) return false;  // refused by the plan
+    const uint64_t N = (uint64_t)(atoms->t_max - atoms->t_min) / atoms->TAtom + 1;
+    tcw_window w;
+    int64_t N_t0, N_tau;
+    if (effective_window((uint32_t)N, atoms->TAtom, atoms->t_min, *win, w, N_t0, N_tau))
+        return false;
+    const double n_t0 = (double)N_t0, n_tau = (double)N_tau, n = (double)N;
+    const double rowblks = n_t0 / 16 + 1, colblks = n_tau / TILE_COLS + 1;
+    const double segs = (n + n_t0) / 16 + 3;  // exp chunks of 16 rows, one atom apart
+    const double bytes = 65536 + 56 * (n + 1) + 4 * MERGED_STRIDE * (n + 4096) +
+                         rowblks * colblks * (sizeof(ItemDev) + sizeof(ItemPart)) +
+                         4 * (colblks * n_t0 + rowblks * n_tau) +
+                         sizeof(ItemDev) * colblks * (segs + 1 + INIT_PARTS) +
+                         8 * NC * n_tau * (segs + INIT_PARTS);
+    return bytes < (double)room;
+}
+
 // A map on its way to the host goes through pinned memory up to this size (the
 // map's copy then shares the call's one wait); larger ones are copied
 // afterwards, straight to the caller's memory.
@@ -4305,11 +4349,15 @@ int tcw_map_noalloc(tcw_handle *h, const tcw_atoms *atoms, const tcw_window *win
     // the plan's buffers become views into the scratch (plan_finish), or the
     // call fails before anything is queued when the map needs more
     tcw_plan &p = h->noalloc;
-    p.compact = p.arena_short = false;
+    p.arena_short = false;
+    p.compact = p.dry = !surely_fits(atoms, win, p.arena_bytes);
+    if (p.dry) {
+        if ((rc = plan_single(h, p, atoms, win, flags, st, "tcw_map_noalloc"))) return rc;
+        p.compact = p.dry = false;
+    }
     rc = plan_single(h, p, atoms, win, flags, st, "tcw_map_noalloc");
     if (rc && p.arena_short) {
-        // off the grid the fast kernels' partials take up to a quarter more a
-        // cell (64 columns an item): the map may still fit in the general ones'
+        // narrower items or shorter chunks take more scratch than the compact layout
         p.compact = true;
         rc = plan_single(h, p, atoms, win, flags, st, "tcw_map_noalloc");
     }
