@@ -46,6 +46,7 @@ constexpr int SFT_TILE = 64;  // SFTs per workgroup
 constexpr int DTERMS_MAX = 64;
 constexpr int RUN = 8;  // bins per rational run: |prod (delta + c)| <= 65^8 fits float
 constexpr unsigned DEMOD_GRID_Y = 65535;
+constexpr int64_t MANY_TILES = 4000;  // workgroups from which 64 templates a tile pay
 
 // Taylor coefficients, evaluated at compile time from pi:
 //   sin(w x) = sum_k sin_coef(w, k) x^(2k+1),  cos(w x) = sum_k cos_coef(w, k) x^(2k)
@@ -332,9 +333,21 @@ int demod_launch(tcw_handle *h, const tcw_sft_set *sfts, int64_t n_sky, const do
     if (rc) return rc;
     const int64_t bx = (sfts->n_sft + SFT_TILE - 1) / SFT_TILE;
     if (bx > INT32_MAX) return fail(TCW_ERR_INVALID, "tcw_demod_atoms: too many SFTs");
-    // template slots per tile: 64 for a bank of templates, fewer lanes of one
-    // SFT when there are only a few templates
-    const int tt = n_tmpl >= 32 ? 64 : n_tmpl >= 4 ? 8 : 1;
+    // template slots per tile.  Few templates: fewer lanes of one SFT.  A bank:
+    // 64 where the launch then still has many workgroups a CU (the lanes read
+    // the same bins, and a wave writes whole rows), fewer, down to 8, where it
+    // would leave CUs idle or end in an uneven last round.  Measured (us at 64 |
+    // 32 | 16 | 8 slots; templates x SFTs): 4096 x 8000 208 | 213 | 228 | 259; 4096 x
+    // 4000 116 | 114 | 119 | 132; 2048 x 4000 68 | 63 | 66 | 73; 1024 x 4000 40 | 36 |
+    // 36 | 39; 512 x 4000 23 | 21.5 | 20 | 21; 256 x 4000 16 | 12.5 | 11 | 11.5; 512 x
+    // 1000 16 | 12 | 10 | 9; 256 x 1000 14 | 10 | 8 | 8.
+    auto tiles = [&](int slots) { return bx * ((n_tmpl + slots - 1) / slots) * n_sky; };
+    const int tt = n_tmpl < 4                        ? 1
+                   : n_tmpl < 32                     ? 8
+                   : tiles(64) >= MANY_TILES         ? 64
+                   : tiles(32) >= MANY_TILES * 3 / 4 ? 32
+                   : tiles(16) >= MANY_TILES / 4     ? 16
+                                                     : 8;
     const unsigned gy = (unsigned)std::min<int64_t>((n_tmpl + tt - 1) / tt, DEMOD_GRID_Y);
     const dim3 grid((unsigned)bx, gy, (unsigned)n_sky);
     const auto *bins = (const float2 *)sfts->bins;
@@ -347,6 +360,10 @@ int demod_launch(tcw_handle *h, const tcw_sft_set *sfts, int64_t n_sky, const do
     // dterms 8 (lalpulsar's default) unrolled at compile time
     if (tt == 64) {
         if (dterms == 8) TCW_DEMOD_LAUNCH(64, 8); else TCW_DEMOD_LAUNCH(64, 0);
+    } else if (tt == 32) {
+        if (dterms == 8) TCW_DEMOD_LAUNCH(32, 8); else TCW_DEMOD_LAUNCH(32, 0);
+    } else if (tt == 16) {
+        if (dterms == 8) TCW_DEMOD_LAUNCH(16, 8); else TCW_DEMOD_LAUNCH(16, 0);
     } else if (tt == 8) {
         if (dterms == 8) TCW_DEMOD_LAUNCH(8, 8); else TCW_DEMOD_LAUNCH(8, 0);
     } else {
