@@ -161,7 +161,8 @@ constexpr int SR_PASS = SR_PASS_LANES * SR_BINS * NC;  // doubles per wave and o
 // (128: N <= 512, 256: N <= 1024).  Longer ones take several rounds of 256
 // threads, or, if they are few, of 1024: a CU holds one such workgroup, whose
 // waves share the template's rounds, but all of them wait for each other at
-// every barrier.  Measured, N = 1000..4000 and 1000..8000, 256 | 1024 threads:
+// every barrier.  Measured (before timestamps were loaded ahead, which takes 3 to
+// 10 us off either), N = 1000..4000 and 1000..8000, 256 | 1024 threads:
 // 128 templates 57 | 40 us, 288 62 | 45, 512 105 | 92, 768 122 | 124, 1024
 // 133 | 154; the line lies where the two meet.
 constexpr int SR_CLASSES = 3;
@@ -231,8 +232,10 @@ typedef d2 d2_u __attribute__((aligned(8)));  // the table starts at any double
 // round's chain (two dependent loads, the barriers, the scan) exposed; stores
 // and loads left out save 1 and 9 of 40 us.  The binary searches of a thread's
 // first bins, a scan through LDS and 8-byte LDS words took: 1024 templates of
-// N = 1000..8000 147 us (now 133), 128 of N = 1000..4000 and two detectors 49
-// (40), 1024 of 500 and two detectors 23.4 (20.6).
+// N = 1000..8000 147 us, 128 of N = 1000..4000 and two detectors 49, 1024 of 500
+// and two detectors 23.4; without them 136, 40 and 20.6; with the next
+// detector's timestamps loaded ahead and the segments read once 125, 37 and 18.6
+// (ahead across rounds too: the same).
 template <int NT>
 __global__ __launch_bounds__(NT) void stage_kernel(
     const TmplDev *__restrict__ tds, const int32_t *__restrict__ tmpls,
@@ -248,7 +251,8 @@ __global__ __launch_bounds__(NT) void stage_kernel(
     int *s_bin = reinterpret_cast<int *>(s_buf);
     int *s_first = s_bin + ROUND;
     __shared__ double s_tot[NW][NC + 1];  // wave totals
-    __shared__ int64_t s_cur[TCW_MAX_DETECTORS];  // a detector's first atom not yet merged
+    // a detector's first atom not yet merged, and its end
+    __shared__ int64_t s_cur[TCW_MAX_DETECTORS], s_end[TCW_MAX_DETECTORS];
     __shared__ int s_cnt, s_flag;
 
     const int t = tmpls[blockIdx.x];
@@ -260,7 +264,11 @@ __global__ __launch_bounds__(NT) void stage_kernel(
     const int nseg = (int)(td.seg_end - td.seg_begin);
     double *__restrict__ P = prefix + td.prefix_off;
     if (tid == 0) s_flag = 0;
-    if (tid < nseg) s_cur[tid] = segs[td.seg_begin + tid].begin;
+    if (tid < nseg) {
+        const SegDev sg = segs[td.seg_begin + tid];
+        s_cur[tid] = sg.begin;
+        s_end[tid] = sg.end;
+    }
     double carry[NC];  // sum of all earlier rounds
 #pragma unroll
     for (int c = 0; c < NC; c++) carry[c] = 0.0;
@@ -273,16 +281,29 @@ __global__ __launch_bounds__(NT) void stage_kernel(
         for (int j = 0; j < SR_BINS; j++)
 #pragma unroll
             for (int c = 0; c < NC; c++) v[j][c] = 0.0f;
+        // a chunk's timestamps; the first chunk's of the next detector are loaded
+        // while this one is merged
+        uint32_t tx[SR_BINS];
+        auto fetch = [&](int64_t c0, int64_t seg_end) {
+#pragma unroll
+            for (int u = 0; u < SR_BINS; u++) {
+                const int64_t i = c0 + u * NT + tid;
+                tx[u] = i < seg_end ? ts[i] : 0;
+            }
+        };
+        fetch(s_cur[0], s_end[0]);
         for (int X = 0; X < nseg; X++) {
-            const int64_t seg_end = segs[td.seg_begin + X].end;
+            const int64_t seg_end = s_end[X];
             int64_t c0 = s_cur[X];
+            bool have = true;  // tx holds the chunk at c0 (block-uniform)
             while (c0 < seg_end) {  // block-uniform
                 const int na = (int)min((int64_t)ROUND, seg_end - c0);
+                if (!have) fetch(c0, seg_end);
                 int bin[SR_BINS];
 #pragma unroll
                 for (int u = 0; u < SR_BINS; u++) {
                     const int i = u * NT + tid;
-                    const uint32_t x = i < na ? ts[c0 + i] : 0;
+                    const uint32_t x = tx[u];
                     uint32_t rem;
                     // -1: before the first bin (in none); nb: in a later round
                     const int b = (int)min(div_TA(x - td.t_min, td, rem), 0x7fffffffu) - base;
@@ -291,6 +312,8 @@ __global__ __launch_bounds__(NT) void stage_kernel(
                     s_first[i] = -1;
                 }
                 if (tid == 0) s_cnt = na;
+                have = false;
+                if (X + 1 < nseg) fetch(s_cur[X + 1], s_end[X + 1]);
                 __syncthreads();
 #pragma unroll
                 for (int u = 0; u < SR_BINS; u++) {
@@ -331,6 +354,7 @@ __global__ __launch_bounds__(NT) void stage_kernel(
                 c0 += cnt;
                 if (cnt < na) break;
             }
+            if (have && X + 1 < nseg) fetch(s_cur[X + 1], s_end[X + 1]);  // none of X's left
             if (tid == 0) s_cur[X] = c0;  // read again after the next round's barriers
         }
         bool odd = false;  // what FLAG_NO_BOUND is for (NaN compares false)
