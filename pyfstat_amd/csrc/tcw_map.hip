@@ -2434,12 +2434,17 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // p sums its share of the block's l range into slot n_seg + p; the scan adds
 // the parts.  Each lane sums INIT_GROUPS columns (its lane, + 64, + 128, +
 // 192 of the block), so every atom, read from LDS as a broadcast, feeds up to
-// 4 x 9 FMA/MUL instructions.  The wave stages its atoms in LDS in chunks of
-// INIT_CHUNK with coalesced loads, the next chunk in flight in registers
-// while the current one is summed.  The l range runs in segments that end
-// where a column group's longest window ends (groups whose windows have all
-// ended drop out); within 63 Ls atoms of that end the lanes of the group
-// mask their weights.
+// 4 x 7 FMAs of Horner sums that run from the far end of the share, where the
+// windows are longest, to its near end.  The wave stages its atoms in LDS in
+// chunks of INIT_CHUNK with coalesced loads, the next chunk in flight in
+// registers while the current one is summed.  The l range runs in segments
+// that start where a column group's longest window ends (before that the
+// group has nothing to sum); within 63 Ls atoms of that end the lanes of the
+// group start one by one.
+// Bound: FP64 issue (7 FMAs an atom and column) at 55% of it, the heaviest
+// waves' shares.  256 templates of 512 columns, windows of 6 to 1540 atoms:
+// 65 us with weights advanced beside forward sums (9 instructions an atom and
+// column), now 55 (unrolled by 4 instead of 2: 90, spills).
 constexpr int INIT_WG = 64;
 constexpr int INIT_GROUPS = TILE_COLS / INIT_WG;
 constexpr int INIT_CHUNK = 64;                                // atoms per LDS chunk (4 KB)
@@ -2447,34 +2452,27 @@ constexpr int INIT_PER = INIT_CHUNK * MERGED_STRIDE / INIT_WG;  // doubles per l
 
 struct InitState {
     double E[INIT_GROUPS][NC];
-    double w[INIT_GROUPS][2];
     double rho[INIT_GROUPS][2];
-    int64_t lr[INIT_GROUPS];  // this lane's window end, per group
-    int64_t lo[INIT_GROUPS];  // the group's shortest window (uniform)
+    int lr[INIT_GROUPS];  // this lane's window end, per group
 };
 
 template <bool MASK>
-__device__ __forceinline__ void init_add(InitState &S, int i, int64_t l, const double *x) {
-    double wa = S.w[i][0], wb = S.w[i][1];
-    if (MASK) {
-        const bool in = l < S.lr[i];
-        wa = in ? wa : 0.0;
-        wb = in ? wb : 0.0;
-    }
+__device__ __forceinline__ void init_add(InitState &S, int i, int l, const double *x) {
+    if (!MASK || l < S.lr[i]) {
 #pragma unroll
-    for (int c = 0; c < NC; c++) S.E[i][c] = fma(c < 3 ? wa : wb, x[c], S.E[i][c]);
-    S.w[i][0] *= S.rho[i][0];
-    S.w[i][1] *= S.rho[i][1];
+        for (int c = 0; c < NC; c++) S.E[i][c] = fma(S.rho[i][c < 3 ? 0 : 1], S.E[i][c], x[c]);
+    }
 }
 
-// atoms [a, b) of the chunk starting at atom c0, for the column groups I0 ..
-// INIT_GROUPS - 1; group I0 masks its lanes' weights when MASK0, the later
-// groups never need to (their shortest window reaches past b)
+// atoms [a, b) of the chunk starting at atom c0, from b - 1 down, for the column
+// groups I0 .. INIT_GROUPS - 1; the lanes of group I0 start at their windows'
+// ends when MASK0, the later groups never need to (their shortest window
+// reaches past b)
 template <int I0, bool MASK0>
-__device__ __forceinline__ void init_segment(InitState &S, const double *buf, int64_t c0,
-                                             int64_t a, int64_t b) {
+__device__ __forceinline__ void init_segment(InitState &S, const double *buf, int c0, int a,
+                                             int b) {
 #pragma unroll 2
-    for (int64_t l = a; l < b; l++) {
+    for (int l = b - 1; l >= a; l--) {
         double x[NC];
         const double *p = buf + (l - c0) * MERGED_STRIDE;  // broadcast
 #pragma unroll
@@ -2485,7 +2483,7 @@ __device__ __forceinline__ void init_segment(InitState &S, const double *buf, in
     }
 }
 
-__global__ __launch_bounds__(INIT_WG) void exp_init_kernel(const TmplDev *__restrict__ tds,
+__global__ __launch_bounds__(INIT_WG, 4) void exp_init_kernel(const TmplDev *__restrict__ tds,
                                                            const ItemDev *__restrict__ items,
                                                            const float *__restrict__ merged,
                                                            double *__restrict__ etab) {
@@ -2498,13 +2496,15 @@ __global__ __launch_bounds__(INIT_WG) void exp_init_kernel(const TmplDev *__rest
     const int lane = (int)threadIdx.x;
     const int64_t k0 = (int64_t)td.k00 + (int64_t)td.a * ((int64_t)td.n_seg * td.rb_rows - 1);
     const int64_t room = (int64_t)td.H - k0;
-    auto clip = [&](int64_t L) { return max(min(L, room), (int64_t)0); };
+    // (H is an int32)
+    auto clip = [&](int64_t L) { return (int)max(min(L, room), (int64_t)0); };
     // longest window of the block (L grows with n), clipped at H: uniform
-    const int64_t lr_blk = clip((int64_t)td.L0 + (int64_t)td.Ls * col_last);
-    const int64_t q = (lr_blk + INIT_PARTS - 1) / INIT_PARTS;
-    const int64_t l0 = part * q, l1 = min(lr_blk, l0 + q);
+    const int lr_blk = clip((int64_t)td.L0 + (int64_t)td.Ls * col_last);
+    const int q = (lr_blk + INIT_PARTS - 1) / INIT_PARTS;
+    const int l0 = min(part * q, lr_blk), l1 = min(lr_blk, l0 + q);
     InitState S;
-    int64_t hi[INIT_GROUPS];  // each group's longest window (uniform)
+    double w[INIT_GROUPS];  // rho^l0
+    int lo0 = 0, hi[INIT_GROUPS];  // group 0's shortest window, each one's longest (uniform)
 #pragma unroll
     for (int i = 0; i < INIT_GROUPS; i++) {
 #pragma unroll
@@ -2514,44 +2514,43 @@ __global__ __launch_bounds__(INIT_WG) void exp_init_kernel(const TmplDev *__rest
         const int n = min(g0 + lane, col_last);  // lanes past the map follow the last column
         const bool any = g0 <= col_last;
         S.lr[i] = any ? clip((int64_t)td.L0 + (int64_t)td.Ls * n) : 0;
-        S.lo[i] = any ? clip((int64_t)td.L0 + (int64_t)td.Ls * g0) : 0;
-        hi[i] = any ? clip((int64_t)td.L0 + (int64_t)td.Ls * glast) : 0;
+        if (i == 0) lo0 = any ? clip((int64_t)td.L0 + (int64_t)td.Ls * g0) : 0;
+        hi[i] = any ? clip((int64_t)td.L0 + (int64_t)td.Ls * glast) : hi[max(i, 1) - 1];
         const double tau = (double)td.tau + (double)n * (double)td.dtau;
         const double r1 = exp(-(double)td.TAtom / tau);
         S.rho[i][0] = r1 * r1;
         S.rho[i][1] = r1;
-        const double w1 = exp(-(double)l0 * (double)td.TAtom / tau);  // rho^l0
-        S.w[i][0] = w1 * w1;
-        S.w[i][1] = w1;
+        w[i] = exp(-(double)l0 * (double)td.TAtom / tau);
     }
     // Windows grow with the column: group i's shortest window (lo) is at
     // least group i-1's longest (hi).  Atoms below lo[0] lie inside every
     // window; segment I0 = [hi[I0-1], hi[I0]) needs group I0 masked and no
     // group before it.
-    const int64_t seg_end[5] = {S.lo[0], hi[0], hi[1], hi[2], hi[3]};
+    const int seg_begin[5] = {0, lo0, hi[0], hi[1], hi[2]};
     // rows k0 + l, l < l1 <= room, lie below H
     const float *__restrict__ X = merged + td.merged_off + k0 * MERGED_STRIDE;
     float r[INIT_PER];  // exact: the table holds float32 sums
-    auto fetch = [&](int64_t c0) {
-        const int64_t nq = min((int64_t)INIT_CHUNK, l1 - c0) * MERGED_STRIDE;
+    auto fetch = [&](int c1) {  // atoms [max(l0, c1 - INIT_CHUNK), c1)
+        const int c0 = max(l0, c1 - INIT_CHUNK);
+        const int nq = (c1 - c0) * MERGED_STRIDE;
 #pragma unroll
         for (int k = 0; k < INIT_PER; k++) {
-            const int64_t qd = (int64_t)k * INIT_WG + lane;
-            r[k] = qd < nq ? X[c0 * MERGED_STRIDE + qd] : 0.0f;
+            const int qd = k * INIT_WG + lane;
+            r[k] = qd < nq ? X[(int64_t)c0 * MERGED_STRIDE + qd] : 0.0f;
         }
     };
-    if (l0 < l1) fetch(l0);
-    for (int64_t c0 = l0; c0 < l1; c0 += INIT_CHUNK) {
-        const int64_t c1 = min(l1, c0 + INIT_CHUNK);
+    if (l0 < l1) fetch(l1);
+    for (int c1 = l1; c1 > l0; c1 -= INIT_CHUNK) {
+        const int c0 = max(l0, c1 - INIT_CHUNK);
         __syncthreads();  // the previous chunk is consumed
 #pragma unroll
         for (int k = 0; k < INIT_PER; k++) buf[k * INIT_WG + lane] = (double)r[k];
         __syncthreads();
-        if (c1 < l1) fetch(c1);  // in flight while this chunk is summed
-        int64_t sa = c0;
+        if (c0 > l0) fetch(c0);  // in flight while this chunk is summed
+        int sb = c1;
 #pragma unroll
-        for (int sgm = 0; sgm < 5; sgm++) {
-            const int64_t sb = min(c1, max(sa, seg_end[sgm]));
+        for (int sgm = 4; sgm >= 0; sgm--) {
+            const int sa = max(c0, min(sb, seg_begin[sgm]));
             if (sa < sb) {  // uniform
                 if (sgm == 0) init_segment<0, false>(S, buf, c0, sa, sb);
                 if (sgm == 1) init_segment<0, true>(S, buf, c0, sa, sb);
@@ -2559,7 +2558,7 @@ __global__ __launch_bounds__(INIT_WG) void exp_init_kernel(const TmplDev *__rest
                 if (sgm == 3) init_segment<2, true>(S, buf, c0, sa, sb);
                 if (sgm == 4) init_segment<3, true>(S, buf, c0, sa, sb);
             }
-            sa = sb;
+            sb = sa;
         }
     }
 #pragma unroll
@@ -2567,7 +2566,9 @@ __global__ __launch_bounds__(INIT_WG) void exp_init_kernel(const TmplDev *__rest
         const int n = col0 + INIT_WG * i + lane;
         if (n <= col_last) {
 #pragma unroll
-            for (int c = 0; c < NC; c++) expf_etab(etab, td, td.n_seg + part, c)[n] = S.E[i][c];
+            for (int c = 0; c < NC; c++)
+                expf_etab(etab, td, td.n_seg + part, c)[n] =
+                    (c < 3 ? w[i] * w[i] : w[i]) * S.E[i][c];
         }
     }
 }
