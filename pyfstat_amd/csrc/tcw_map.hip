@@ -442,8 +442,8 @@ __host__ __device__ __forceinline__ uint32_t exp_table_bins(const TmplDev &td) {
 // [exp_table_bins][8] (7 columns + padding), the same float32 detector-order
 // sums as stage_kernel (the kernels that read it widen them to FP64, exactly).
 // A workgroup owns 256 * SXB consecutive bins of one template: per detector,
-// a block-wide search bounds the block's atoms, which are copied
-// into LDS in chunks with coalesced loads; each thread then sums its SXB bins
+// the block's atoms are bounded (bound_two: 9.9 us for 32 templates of 1000 bins
+// with a block-wide search per detector, now 8.2) and copied into LDS in chunks with coalesced loads; each thread then sums its SXB bins
 // from LDS (atoms in order, detectors in order).  Grid: (bin blocks, exp
 // templates), y-strided.  SXB = 4 (1024-bin blocks) for batches, 1 (256-bin
 // blocks) when 1024-bin blocks would give fewer than SX_NARROW_BELOW
@@ -455,45 +455,38 @@ constexpr int SX_CHUNK = 1024;  // atoms staged per pass
 // consecutive lanes on consecutive floats
 constexpr int SX_ROW = MERGED_STRIDE + 1;
 
-// For sorted ts[lo0, hi0): the first index with ts >= key0 into s_r[0][0]
-// and with ts >= key1 into s_r[1][0] (hi0 if none).  The two halves of a
-// 256-thread block search one key each, 128-way: each round samples 128
-// evenly spaced timestamps of the remaining range (one load per thread, all
-// in flight together) and keeps the gap where the key falls, so a range of
-// n atoms takes about log_128(n) rounds of loads instead of log_2(n)
-// dependent ones.  Every thread of the block calls it; the results are valid
-// on return.
-__device__ __forceinline__ void block_lower_bound2(const uint32_t *__restrict__ ts, int64_t lo0,
-                                                   int64_t hi0, uint64_t key0, uint64_t key1,
-                                                   int64_t (&s_r)[2][2], int (&s_c)[4]) {
-    const int tid = threadIdx.x, half = tid >> 7, t = tid & 127, wave = tid >> 6;
-    const uint64_t key = half ? key1 : key0;
-    if (tid < 2) {
-        s_r[tid][0] = lo0;
-        s_r[tid][1] = hi0;
+// For sorted ts[lo, hi): the first index with ts >= key (hi if none), by one
+// wave: a round samples 64 evenly spaced timestamps (one load a lane) and keeps
+// the gap where the key falls, so n atoms take about log_64(n) loads in turn.
+__device__ __forceinline__ int64_t wave_lower_bound(const uint32_t *__restrict__ ts, int64_t lo,
+                                                    int64_t hi, uint64_t key, int lane) {
+    while (hi > lo) {
+        const int64_t n = hi - lo;
+        const int64_t sd = n <= 64 ? 1 : (n + 63) / 64;
+        const bool pred = lane * sd < n && (uint64_t)ts[lo + lane * sd] < key;
+        const int64_t c = __popcll(__ballot(pred));  // samples below the key
+        if (c == 0) return lo;
+        hi = min(lo + c * sd, hi);  // the answer is in (sample c-1, sample c]
+        lo += (c - 1) * sd + 1;
+    }
+    return lo;
+}
+
+// The first atoms with ts >= key0 and >= key1 of detector segments s and s + 1
+// (if below s_end) into r[0], r[1] and r[2], r[3]: each wave of a 256-thread
+// block searches one of the four.  The caller synchronises before the next call.
+__device__ __forceinline__ void bound_two(const uint32_t *__restrict__ ts,
+                                          const SegDev *__restrict__ segs, int64_t s,
+                                          int64_t s_end, uint64_t key0, uint64_t key1,
+                                          int64_t (&r)[4]) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (s + (wave >> 1) < s_end) {
+        const SegDev sg = segs[s + (wave >> 1)];
+        const int lane = threadIdx.x & 63;
+        const int64_t k = wave_lower_bound(ts, sg.begin, sg.end, wave & 1 ? key1 : key0, lane);
+        if (lane == 0) r[wave] = k;
     }
     __syncthreads();
-    // the answer lies in [lo, hi]; n = hi - lo timestamps are left to test
-    while (s_r[0][1] > s_r[0][0] || s_r[1][1] > s_r[1][0]) {  // block-uniform
-        const int64_t lo = s_r[half][0], hi = s_r[half][1];
-        const int64_t n = hi - lo;
-        const int64_t sd = n <= 128 ? 1 : (n + 127) / 128;
-        const bool pred = n > 0 && t * sd < n && (uint64_t)ts[lo + t * sd] < key;
-        const uint64_t b = __ballot(pred);
-        if ((tid & 63) == 0) s_c[wave] = __popcll(b);
-        __syncthreads();
-        if (t == 0 && n > 0) {
-            // c samples lie below the key: the answer is in (sample c-1, sample c]
-            const int c = s_c[2 * half] + s_c[2 * half + 1];
-            if (c == 0) {
-                s_r[half][1] = lo;
-            } else {
-                s_r[half][0] = lo + (int64_t)(c - 1) * sd + 1;
-                s_r[half][1] = min(lo + (int64_t)c * sd, hi);
-            }
-        }
-        __syncthreads();
-    }
 }
 
 template <int SXB>
@@ -508,8 +501,7 @@ __global__ __launch_bounds__(256) void stage_exp_kernel(
     __shared__ float s_raw[SX_RAW];
     uint32_t *s_ts = reinterpret_cast<uint32_t *>(s_raw);
     float(*s_x)[SX_CHUNK] = reinterpret_cast<float(*)[SX_CHUNK]>(s_raw + SX_CHUNK);
-    __shared__ int64_t s_rng[2][2];
-    __shared__ int s_cnt[4];
+    __shared__ int64_t s_rng[4];
     const int tid = threadIdx.x;
     for (int64_t e = blockIdx.y; e < n_exp; e += gridDim.y) {
         // before any map kernel: clear the template's single-atom flag
@@ -531,11 +523,10 @@ __global__ __launch_bounds__(256) void stage_exp_kernel(
 #pragma unroll
             for (int c = 0; c < NC; c++) v[j][c] = 0.0f;
         for (int64_t X = td.seg_begin; X < td.seg_end; X++) {
-            const SegDev sg = segs[X];
-            // first atom with ts >= tb_lo, resp. >= tb_hi
-            block_lower_bound2(ts, sg.begin, sg.end, tb_lo, tb_hi, s_rng, s_cnt);
-            const int64_t ka = s_rng[0][0], kb = s_rng[1][0];
-            __syncthreads();  // s_rng is rewritten by the next detector
+            const int two = (int)(X - td.seg_begin) & 1;  // bounded two at a time
+            if (two == 0) bound_two(ts, segs, X, td.seg_end, tb_lo, tb_hi, s_rng);
+            const int64_t ka = s_rng[2 * two], kb = s_rng[2 * two + 1];
+            __syncthreads();  // s_rng is rewritten for the next two
             for (int64_t c0 = ka; c0 < kb; c0 += SX_CHUNK) {
                 const int na = (int)min((int64_t)SX_CHUNK, kb - c0);
                 for (int i = tid; i < na; i += 256) {
@@ -3056,8 +3047,8 @@ struct MergeTmpl {
     uint32_t N, t_min;
 };
 
-// A workgroup owns MERGE_BINS consecutive bins of one template.  Per detector a
-// block-wide search bounds the block's atoms; chunk by chunk their bins are
+// A workgroup owns MERGE_BINS consecutive bins of one template.  Per detector
+// the block's atoms are bounded; chunk by chunk their bins are
 // formed, the first atom of every bin is marked where the bin changes, and each
 // thread sums the atoms of its bins, MERGE_WG apart, so that the lanes' reads of
 // the columns and the stores are nearly and exactly consecutive.  Float32 sums,
@@ -3067,7 +3058,7 @@ struct MergeTmpl {
 // written by the blocks in equal shares of the atoms.
 // Bound: HBM bytes -- 32 an atom in, 28 a bin and 8 an atom out.  512 templates
 // of 2 x 1844 atoms: 33 us with a binary search of the timestamps per bin and
-// 7 for the atoms' bins in a kernel of its own, 25 together so (4.2 TB/s).
+// 7 for the atoms' bins in a kernel of its own, 24 together so (4.3 TB/s).
 constexpr int MERGE_WG = 256;
 constexpr int MERGE_PER = 4;                      // bins and atoms of a thread
 constexpr int MERGE_BINS = MERGE_WG * MERGE_PER;  // bins per block, atoms per chunk
@@ -3077,8 +3068,7 @@ __global__ __launch_bounds__(MERGE_WG) void merge_kernel(
     const uint32_t *__restrict__ ts, const float *__restrict__ cols, int64_t cstride,
     uint32_t TA, float *__restrict__ out, int64_t ostride, int64_t *__restrict__ atom_bin) {
     __shared__ int s_bin[MERGE_BINS], s_first[MERGE_BINS];
-    __shared__ int64_t s_rng[2][2];
-    __shared__ int s_cnt[4];
+    __shared__ int64_t s_rng[4];
     const int tid = threadIdx.x;
     for (int64_t t = blockIdx.y; t < T; t += gridDim.y) {
         const MergeTmpl m = mt[t];
@@ -3095,8 +3085,9 @@ __global__ __launch_bounds__(MERGE_WG) void merge_kernel(
             for (int c = 0; c < NC; c++) v[j][c] = 0.0f;
         for (int64_t s = m.seg_begin; s < m.seg_end; s++) {
             const SegDev sg = segs[s];
-            block_lower_bound2(ts, sg.begin, sg.end, t_lo, t_hi, s_rng, s_cnt);
-            const int64_t ka = s_rng[0][0], kb = s_rng[1][0];
+            const int two = (int)(s - m.seg_begin) & 1;  // bounded two at a time
+            if (two == 0) bound_two(ts, segs, s, m.seg_end, t_lo, t_hi, s_rng);
+            const int64_t ka = s_rng[2 * two], kb = s_rng[2 * two + 1];
             for (int64_t c0 = ka; c0 < kb; c0 += MERGE_BINS) {  // block-uniform
                 const int na = (int)min((int64_t)MERGE_BINS, kb - c0);
                 int bin[MERGE_PER];
