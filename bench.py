@@ -68,7 +68,7 @@ REFINE_WARM_S = 0.5
 # and WRITE_SIZE (scaled by a 1 GiB copy in the same run) for the default-size
 # workloads; the commands and raw counters are in the named summaries.
 PROFILED_TRAFFIC = {
-    "rect_batched": (1.017e9 + 25.43e9, "profiles/rect_fast_kernel.rect_batched.md"),
+    "rect_batched": (1.255e9 + 25.77e9, "profiles/rect_fast_kernel.rect_batched.md"),
     "exp_shared": (0.156e9 + 0.540e9, "profiles/exp_fast_kernel.exp_shared.md"),
     "demod_atoms": (0.0207e9 + 0.9440e9, "profiles/demod_atoms_kernel.demod_atoms.md"),
 }
@@ -76,13 +76,13 @@ FP64_VALU_PEAK_TFLOPS = 78.6
 # What bounds the map kernel instead of HBM (rocprofv3 counters of the same
 # kernel, summarised in the profile files named here).
 LIMITER = {
-    "rect_batched": "VALU issue: 43 VALU instructions per cell (24 FP64 add/mul/FMA; part of "
-                    "the rest is lanes past N_tau in each template's last 256-column block, 8.6% "
-                    "of the lane-cells here), the VALU issuing every SIMD cycle at the "
-                    "~1.76 GHz the card holds under this load; "
+    "rect_batched": "VALU issue: 36 VALU instructions per cell (21 FP64 add/mul/FMA; lanes past "
+                    "N_tau in each template's last column block are 3.5% of the lane-cells "
+                    "here), the VALU issuing every SIMD cycle at the 1.6-1.8 GHz the card "
+                    "holds under this load; "
                     "profiles/rect_fast_kernel.rect_batched.md",
     "exp_shared": "latency at two waves per SIMD (one row chunk per column: 2048 waves): "
-                  "~56 VALU instructions per cell at ~59% VALU busy, FP64 dependency chains and "
+                  "~56 VALU instructions per cell at ~60% VALU busy, FP64 dependency chains and "
                   "LDS broadcasts of the entering atoms; profiles/exp_fast_kernel.exp_shared.md",
 }
 

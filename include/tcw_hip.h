@@ -180,9 +180,9 @@ int tcw_batch_plan(tcw_handle *h, const tcw_batch_desc *desc, uint32_t flags,
 
 /* tcw_batch_plan with the rows (t0) per work item chosen per kernel mode:
  * rows_by_mode (host [4], may be NULL = all 0) for modes 0 (rect, regular
- * grid), 1 (rect, generic), 2 (exp, direct) and 3 (exp on the atom grid);
+ * grid), 1 (rect, any steps), 2 (exp, any steps) and 3 (exp on the atom grid);
  * each 0 (the library's choice for the batch) or a multiple of 16 in
- * [16, 512] ([16, 128] for mode 3).  The setting belongs to this plan only.
+ * [16, 512] ([16, 1024] for mode 3).  The setting belongs to this plan only.
  * What the autotuner varies; no counterpart in the reference. */
 int tcw_batch_plan_rows(tcw_handle *h, const tcw_batch_desc *desc, uint32_t flags,
                         const int32_t *rows_by_mode, tcw_plan **out, int64_t *F_off);

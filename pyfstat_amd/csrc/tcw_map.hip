@@ -49,7 +49,8 @@ namespace {
 
 constexpr int NC = TCW_NCOL;
 constexpr int WG = 256;           // threads per workgroup (4 wave64)
-constexpr int TILE_COLS = 256;    // tau columns per work item (rect_step_kernel: 256, 128 or 64)
+constexpr int TILE_COLS = 256;    // tau columns per work item (rect_step_kernel: 256, 128 or
+                                  // 64; exp_walk_kernel: 64)
 constexpr int MERGED_STRIDE = 8;  // floats per atom in the atom table (7 columns + kind)
 // the kind column: 0 for a bin of zeros, 1 for one with data, BIN_ODD for one
 // with an infinity or NaN (more than any count of bins with data)
