@@ -596,12 +596,17 @@ __device__ __forceinline__ double cell_D(double A, double B, double C) {
 // The map is float32: the quotient of the FP64 numerator and determinant
 // (each rounded to float) through v_rcp_f32 is within ~3e-7 relative, and
 // v_rcp_f64 issues at ~1/3.5 the rate of an FP64 FMA.
-__device__ __forceinline__ float cell_quot(double A, double B, double C, double far, double fai,
-                                           double fbr, double fbi, float &Df) {
+__device__ __forceinline__ double cell_num(double A, double B, double C, double far, double fai,
+                                           double fbr, double fbi) {
     const double p = fma(far, far, fai * fai);
     const double q = fma(fbr, fbr, fbi * fbi);
     const double r = fma(far, fbr, fai * fbi);
-    const double num = fma(B, p, fma(A, q, (-2.0 * C) * r));
+    return fma(B, p, fma(A, q, (-2.0 * C) * r));
+}
+
+__device__ __forceinline__ float cell_quot(double A, double B, double C, double far, double fai,
+                                           double fbr, double fbi, float &Df) {
+    const double num = cell_num(A, B, C, far, fai, fbr, fbi);
     Df = (float)cell_D(A, B, C);
     return (float)num * __builtin_amdgcn_rcpf(Df);
 }
@@ -1614,14 +1619,17 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
 //   lo = q + [phi > 0],   hi = q + Q - 1 + [s >= h] + [s >= TAtom + h],
 // s = phi + R, h = TAtom - TAtom / 2 (atoms at or past N count as zero), with
 // weights w rho^(i - lo), rho = e^(-TAtom/tau).  F does not change with a
-// common factor of the weights, so w is left out, and
+// common factor of the weights, so w is left out of the sums, and
 //   E(m) = sum_{i = lo}^{hi} rho^(i - lo) x_i   (rho^2 for a^2, b^2, ab)
 // goes from row to row by the atoms that enter (the same on every lane) and
 // those that leave (dt0 / TAtom or one more, by lane):
 //   E(m-1) = rho^(lo - lo') E(m) + sum_{i = lo'}^{lo-1} rho^(i-lo') x_i
 //            - sum_{i = hi'+1}^{hi} rho^(i-lo') x_i;
 // rho^(hi' + 1 - lo') is one of four values per lane, as that exponent is
-// Q - 1 .. Q + 2.  A cell costs O(dt0 / TAtom) instead of O(3 tau / TAtom).
+// Q - 1 .. Q + 2.  (The numerator and the determinant take their factor w^4
+// before they are rounded to float, as they have it in the direct sum, so that F
+// is the same float and nearly equal maxima keep their order; 30 instead of 28.5
+// us.)  A cell costs O(dt0 / TAtom) instead of O(3 tau / TAtom).
 //
 // An item is RB rows x 64 columns, one column a lane, and its rows are shared
 // out to eight waves from the top down.  The waves share the direct sum at the
@@ -1665,6 +1673,7 @@ struct WalkCol {  // a lane's column, 3 tau = TAtom Q + R
     double rho[2];   // rho^2, rho
     double lead[4];  // rho^(Q - 1 + k)
     double ratau;    // TAtom / tau
+    double w4[3];    // w^4 of the row, and its change to the next row without and with a wrap
     int Q;
     uint32_t R;
 };
@@ -1798,11 +1807,14 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
     wc.lead[0] = exp(-(double)(wc.Q - 1) * wc.ratau);
 #pragma unroll
     for (int k = 1; k < 4; k++) wc.lead[k] = wc.lead[k - 1] * wc.rho[1];
+    // w = e^(-psi/tau): the row's first atom lies psi after its start
+    const uint32_t dphi = td.dt0 % TA;
+    wc.w4[1] = exp(-4.0 * (double)dphi * wc.ratau / (double)TA);
+    wc.w4[2] = exp(4.0 * (double)(TA - dphi) * wc.ratau / (double)TA);
     // the last lane's window is the longest, the first one's the shortest
     const int Q0 = __builtin_amdgcn_readlane(wc.Q, 0), Q63 = __builtin_amdgcn_readlane(wc.Q, 63);
 
     const int dq = (int)(td.dt0 / TA);
-    const uint32_t dphi = td.dt0 % TA;
     auto row_at = [&](int rl) {
         const uint32_t T = td.t0 - td.t_min + (uint32_t)(row0 + rl) * td.dt0;
         return WalkRow{(int)(T / TA), T % TA};
@@ -1909,6 +1921,8 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
 
     WalkRow row = row_at(max(top, 0));
     int hi = row.hi(wc, TA);
+    uint32_t psi = row.phi > 0 ? TA - row.phi : 0;
+    wc.w4[0] = exp(-4.0 * (double)psi * wc.ratau / (double)TA);
     if (!direct) {  // block-uniform
         if (next >= 0) {
             const WalkRow to = row_at(next);
@@ -1962,7 +1976,10 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
             const int m = row0 + r4 + j;
             F4[j][0] = -INFINITY;
             if (r4 + j >= nrows) continue;  // uniform
-            const float f = cell_F(E[0], E[1], E[2], E[3], E[4], E[5], E[6]);
+            const double num = cell_num(E[0], E[1], E[2], E[3], E[4], E[5], E[6]);
+            const double D = cell_D(E[0], E[1], E[2]);
+            const float q = (float)(wc.w4[0] * num) * __builtin_amdgcn_rcpf((float)(wc.w4[0] * D));
+            const float f = cell_ok(E[0], E[1], E[2]) ? q : 2.0f;
             if (valid) {
                 Ft[(int64_t)m * N_tau + n] = f;
                 F4[j][0] = f;
@@ -1980,6 +1997,10 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
                 row.q--;
             }
             row.phi -= dphi;
+            psi += dphi;
+            const bool wrap = psi >= TA;
+            psi -= wrap ? TA : 0;
+            wc.w4[0] *= wrap ? wc.w4[2] : wc.w4[1];
             const int lo2 = row.lo(), hi2 = row.hi(wc, TA);
             if (direct) {  // uniform
                 walk_row_sum(X, N, wc, lo2, hi2 - lo2 + 1, row.q + Q63 + 2 - lo2, E, kinds);
@@ -2056,8 +2077,18 @@ __global__ __launch_bounds__(WALK_WG) void exp_walk_kernel(
 // read once per wave through uniform loads; each lane carries its own tau.
 // The weights are advanced by rho = exp(-TAtom/tau) per atom (FP64, relative
 // error ~ k * 1e-16 after k atoms), the sums are FP64.
+// Bound: latency of the sums' chains, so the rows and groups of 64 columns of an
+// item are dealt to DIRECT_WAVES waves, which leave F in LDS, and four of them
+// then reduce whole rows; 64 VGPRs, two workgroups a CU.  Half-atom starts, maps
+// us with four waves an item | so: 12 templates of 31 x 23 cells 99 | 56, 32 of 125
+// x 125 793 | 369, 64 of 250 x 500 10300 | 7840 (eight waves 67, 511, 8030; the
+// unmasked loop unrolled by 2: 57, 396, 13090).
+constexpr int DIRECT_WAVES = 16;
+constexpr int DIRECT_ROWS = 16;
+constexpr int DIRECT_WG = 64 * DIRECT_WAVES;
+
 template <bool BTSG, bool STRICT>
-__global__ __launch_bounds__(WG) void exp_direct_kernel(
+__global__ __launch_bounds__(DIRECT_WG, 8) void exp_direct_kernel(
     const TmplDev *__restrict__ tds, const ItemDev *__restrict__ items, int64_t item0,
     const float *__restrict__ merged, float *__restrict__ Fout,
     ItemPart *__restrict__ ipart, float *__restrict__ rowpart,
@@ -2065,6 +2096,7 @@ __global__ __launch_bounds__(WG) void exp_direct_kernel(
     __shared__ float sh_rowM[MAX_RB];
     __shared__ float sh_rowS[MAX_RB];
     __shared__ FinShared sh_fin;
+    __shared__ float sh_F[DIRECT_ROWS][TILE_COLS];
     const int64_t item_id = item0 + block_slot();
     const ItemDev it = items[item_id];
     const TmplDev td = tds[it.t];
@@ -2085,19 +2117,23 @@ __global__ __launch_bounds__(WG) void exp_direct_kernel(
 #pragma unroll
     for (int c = 0; c < 4; c++) colidx[c] = col0 + c * 64 + lane;
 
-    for (int rl = wave; rl < RB; rl += 4) {
-        const int m = row0 + rl;
-        if (m >= N_t0) break;
-        const uint32_t t0m = td.t0 + (uint32_t)m * td.dt0;
-        const uint32_t i0 = idx_start(t0m, td.t_min, TA, td.N);
-        // first atom with t_i >= t0m (timestamps t_min + i*TA never wrap)
-        uint32_t ilo = 0;
-        if (t0m > td.t_min) ilo = (uint32_t)(((uint64_t)(t0m - td.t_min) + TA - 1) / TA);
-        const uint32_t lo = max(i0, ilo);
-        float F[1][4];
-        for (int c = 0; c < 4; c++) {
-            const bool valid = colidx[c] < N_tau;
-            const uint32_t n = valid ? (uint32_t)colidx[c] : 0u;
+    const int nrows = min(RB, N_t0 - row0);
+    const int groups = (min(TILE_COLS, N_tau - col0) + 63) / 64;  // of 64 columns
+    for (int r0 = 0; r0 < nrows; r0 += DIRECT_ROWS) {
+        const int rows = min(DIRECT_ROWS, nrows - r0);
+        // a wave sums one row of one group at a time
+        for (int pair = wave; pair < rows * groups; pair += DIRECT_WAVES) {
+            const int rl = pair / groups, c = pair % groups;
+            const int m = row0 + r0 + rl;
+            const uint32_t t0m = td.t0 + (uint32_t)m * td.dt0;
+            const uint32_t i0 = idx_start(t0m, td.t_min, TA, td.N);
+            // first atom with t_i >= t0m (timestamps t_min + i*TA never wrap)
+            uint32_t ilo = 0;
+            if (t0m > td.t_min) ilo = (uint32_t)(((uint64_t)(t0m - td.t_min) + TA - 1) / TA);
+            const uint32_t lo = max(i0, ilo);
+            const int col = col0 + c * 64 + lane;
+            const bool valid = col < N_tau;
+            const uint32_t n = (uint32_t)min(col, N_tau - 1);
             const uint32_t tau = td.tau + n * td.dtau;
             const uint32_t t1 = t0m + 3u * tau;
             const uint32_t i1 = idx_end_q((uint32_t)(t1 - td.t_min + TA / 2) / TA, td.N);
@@ -2112,35 +2148,57 @@ __global__ __launch_bounds__(WG) void exp_direct_kernel(
             const double rtau = 1.0 / (double)tau;
             const double rho = exp(-(double)TA * rtau);
             double w = exp(-(double)(td.t_min + lo * TA - t0m) * rtau);
-            // wave-uniform loop bounds: the longest lane decides
-            int64_t hi_w = hi;
+            // wave-uniform loop bounds: every lane up to the shortest window's end,
+            // then those whose window goes on (a zero weight would let an infinity
+            // or NaN past a lane's end in)
+            int64_t hi_w = hi, hi_0 = hi;
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1)
+            for (int o = 32; o > 0; o >>= 1) {
                 hi_w = max(hi_w, (int64_t)__shfl_xor((long long)hi_w, o));
-            for (int64_t i = lo; i <= hi_w; i++) {
-                const double wi = (i <= hi) ? w : 0.0;
-                const double w2 = wi * wi;
+                hi_0 = min(hi_0, (int64_t)__shfl_xor((long long)hi_0, o));
+            }
+            auto add = [&](int64_t i) {
                 const float *xi = X + i * MERGED_STRIDE;
+                const double w2 = w * w;
                 acc[0] = fma(xi[0], w2, acc[0]);
                 acc[1] = fma(xi[1], w2, acc[1]);
                 acc[2] = fma(xi[2], w2, acc[2]);
-                acc[3] = fma(xi[3], wi, acc[3]);
-                acc[4] = fma(xi[4], wi, acc[4]);
-                acc[5] = fma(xi[5], wi, acc[5]);
-                acc[6] = fma(xi[6], wi, acc[6]);
+                acc[3] = fma(xi[3], w, acc[3]);
+                acc[4] = fma(xi[4], w, acc[4]);
+                acc[5] = fma(xi[5], w, acc[5]);
+                acc[6] = fma(xi[6], w, acc[6]);
+            };
+            int64_t i = lo;
+#pragma unroll 1  // (unrolled, the loads' scalar registers spill)
+            for (; i <= hi_0; i++) {
+                add(i);
+                w *= rho;
+            }
+            for (; i <= hi_w; i++) {
+                if (i <= hi) add(i);
                 w *= rho;
             }
             const float f = cell_F(acc[0], acc[1], acc[2], acc[3], acc[4], acc[5], acc[6]);
-            if (valid) Ft[(int64_t)m * N_tau + colidx[c]] = f;
-            F[0][c] = valid ? f : -INFINITY;
+            if (valid) Ft[(int64_t)m * N_tau + col] = f;
+            sh_F[rl][c * 64 + lane] = valid ? f : -INFINITY;
         }
-        red.add(F, m, colidx, N_tau, lane, rl, sh_rowM, sh_rowS);
+        __syncthreads();
+        for (int rl = wave; wave < 4 && rl < rows; rl += 4) {
+            float F[1][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) F[0][c] = c < groups ? sh_F[rl][c * 64 + lane] : -INFINITY;
+            red.add(F, row0 + r0 + rl, colidx, N_tau, lane, r0 + rl, sh_rowM, sh_rowS);
+        }
+        __syncthreads();
     }
     if (STRICT && single) atomicOr(flags + it.t, FLAG_SINGLE_ATOM);
-    __syncthreads();
-    wave_argmax(red.best, red.bidx);
-    finish_item(red, wave, lane, td, it, item_id, min(RB, N_t0 - row0), ipart, rowpart,
-                colpart, sh_rowM, sh_rowS, sh_fin, [](int ln, int c) { return c * 64 + ln; });
+    if (wave < 4) {
+        wave_argmax(red.best, red.bidx);
+        finish_item(red, wave, lane, td, it, item_id, nrows, ipart, rowpart, colpart, sh_rowM,
+                    sh_rowS, sh_fin, [](int ln, int c) { return c * 64 + ln; });
+    } else {
+        __syncthreads();  // finish_item's
+    }
 }
 
 // ----------------------------------------------------------------------------
@@ -3454,9 +3512,12 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
                              w.dtau % TAtom == 0 && w.tau >= TAtom;
         // (rows of at most 2^20 cells: the map kernel's row stores address a
         // pass of rows by 32-bit byte offsets)
-        // off the grid: the sliding sum with any steps
+        // off the grid: the sliding sum with any steps.  (Starts that step by
+        // part of an atom repeat windows: the posterior's mode is then one of
+        // several equal rows, and which one the sums' rounding decides.  They
+        // keep the direct sum and with it their answers.)
         td.walk = !(p.flags & TCW_FLAG_GENERIC) && w.t0 >= t_min && end < (1ull << 32) &&
-                  w.tau >= TAtom && !p.compact;
+                  w.tau >= TAtom && !p.compact && (w.dt0 >= TAtom || N_t0 == 1);
         if (!(p.flags & TCW_FLAG_GENERIC) && on_grid && end < (1ull << 32) &&
             N_tau <= (int64_t)1 << 20) {
             mode = MODE_EXP_FAST;
@@ -3483,8 +3544,8 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
             td.a = (int32_t)(w.dt0 / TAtom);
             td.q0 = (int32_t)(((uint64_t)w.t0 - t_min + half) / TAtom);
             td.q00 = (int32_t)(((uint64_t)w.t0 + w.tau - t_min + half) / TAtom);
-        } else if (p.compact) {
-            td.walk = 0;
+        } else if (p.compact || (w.dt0 < TAtom && N_t0 > 1) || (w.dtau < TAtom && N_tau > 1)) {
+            td.walk = 0;  // (steps of part of an atom repeat rows or columns, as above)
         }
     }
     td.mode = mode;
@@ -3829,7 +3890,8 @@ void launch_maps(tcw_plan &p, float *F, hipStream_t st) {
                                p.max_lds_walk, st, tds, items, p.mode_begin[MODE_EXP_DIRECT],
                                merged, F, ipart, rowpart, colpart, flags);
         if (p.direct_tmpls > 0)
-            hipLaunchKernelGGL((exp_direct_kernel<BTSG, STRICT>), dim3((unsigned)n), dim3(WG), 0,
+            hipLaunchKernelGGL((exp_direct_kernel<BTSG, STRICT>), dim3((unsigned)n),
+                               dim3(DIRECT_WG), 0,
                                st, tds, items, p.mode_begin[MODE_EXP_DIRECT], merged, F, ipart,
                                rowpart, colpart, flags);
     }

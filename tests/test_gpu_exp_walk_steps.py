@@ -132,3 +132,34 @@ def test_single_atom_flag_matches_direct_sum(hip_ready):
     assert np.array_equal(one, two) and one.any() and not one.all()
     b.close()
     ref.close()
+
+
+@pytest.mark.parametrize("dt0", [TA // 2, TA // 4, 700, TA + 1, 2700])
+def test_equal_windows_keep_their_order(hip_ready, dt0):
+    """Starts that step by part of an atom repeat windows, whose F are equal but for
+    rounding: the maximum and the posterior's mode are the direct sum's, as are
+    all but a few F of larger steps."""
+    from pyfstat_amd.batched import BatchedTransientMaps
+
+    maps = []
+    for generic in (False, True):
+        ts, cols, off, wins, T = [], [], [0], [], 24
+        for k in range(T):
+            (t, c), = _atoms(250, 300 + k, "plain", 1)
+            ts.append(t)
+            cols.append(c)
+            off.append(off[-1] + t.size)
+            wins.append(transientWindowRange_t(
+                type=TRANSIENT_EXPONENTIAL, t0=synth.T_START, t0Band=99 * dt0, dt0=dt0,
+                tau=2 * TA, tauBand=22 * 4500, dtau=4500))
+        b = BatchedTransientMaps(np.concatenate(ts), np.concatenate(cols, 1), off,
+                                 np.arange(T + 1), wins, TA, BtSG=True, force_generic=generic)
+        b.run()
+        maps.append((b.F_host(), b.stats()))
+        b.close()
+    (F, st), (G, sg) = maps
+    # both round the same two FP64 numbers, 1e-13 apart, to float32: all but
+    # about 1e-6 of the cells are the same float
+    assert (F != G).mean() < 1e-4
+    for f in ("m_ML", "n_ML", "m_MP", "n_MP"):
+        np.testing.assert_array_equal(st[f], sg[f])
