@@ -32,6 +32,7 @@
 
 #include "tcw_common.h"
 #include "tcw_hip.h"
+#include "tcw_step.h"
 
 // Device memory of tcw_map_noalloc: the single-map plan's buffers (descriptors,
 // prefix or atom tables, reduction partials) are carved out of this array, so
@@ -1326,42 +1327,19 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 // 4000 bins, steps of 2 and 3 bins, 37e6 cells: maps 192 us with the generic
 // kernel (an integer division and an uncoalesced 56-byte read a cell), 90 us
 // so, 210 us with these indices but the table read in place.
-// rows per item at most and items aimed at, untuned
-// Rows per item at most and items aimed at, untuned (the maps below: 64 rows
+// Rows per item at most and items aimed at, untuned (the maps above: 64 rows
 // 100 us, 32 rows 110, 96 rows 115, all with 256 columns an item).
 constexpr int STEP_RB = 64;
 constexpr int64_t STEP_ITEMS = 1024;
-// Bytes of staged range per item.  The widest of 256, 128 and 64 columns whose
-// range stays below the first figure (four workgroups a CU or more), else 64
-// columns if that stays below the second, else 256 read from the table (the
-// maps below at 20, 28, 36 and 52 KB: 112, 95, 94 and 100 us).
-constexpr int STEP_LDS_AIM = 36 << 10;
-constexpr int STEP_LDS_MOST = 76 << 10;
+using tcwc::step_bytes;
+using tcwc::step_in_lds;
+using tcwc::step_range;
+using tcwc::step_shape;
+using tcwc::STEP_LDS_AIM;
+using tcwc::STEP_LDS_MOST;
+using tcwc::StepRange;
+using tcwc::StepShape;
 
-struct StepShape {
-    int entries;  // staged prefix entries of an item at most
-    int pad;
-};
-__host__ __device__ __forceinline__ StepShape step_shape(int rb, int tile, uint32_t N_tau,
-                                                         uint32_t dt0, uint32_t dtau,
-                                                         uint32_t TA) {
-    const uint32_t nc = N_tau < (uint32_t)tile ? N_tau : (uint32_t)tile;
-    const uint64_t span = ((uint64_t)(rb - 1) * dt0 + (uint64_t)(nc - 1) * dtau) / TA + 3;
-    StepShape sh;
-    sh.entries = span < (1u << 20) ? (int)span : 1 << 20;
-    const uint32_t b = dtau / TA;
-    sh.pad = 31;
-    if (b > 0 && b % 2 == 0 && dtau % TA == 0)
-        for (sh.pad = 0; 2u << sh.pad <= b; sh.pad++) {
-        }
-    return sh;
-}
-__host__ __device__ __forceinline__ int step_bytes(const StepShape &sh) {
-    return (sh.entries * NC + (sh.entries >> sh.pad) + 1) * (int)sizeof(double);
-}
-__host__ __device__ __forceinline__ bool step_in_lds(const StepShape &sh) {
-    return step_bytes(sh) <= STEP_LDS_MOST;
-}
 // dynamic LDS of an item: the rows' references and sums, and the staged range
 // (none if it does not fit) or the final reduction in its place
 __host__ __device__ __forceinline__ int step_lds(int rb, const StepShape &sh) {
@@ -1388,7 +1366,6 @@ __device__ __forceinline__ void rect_step_item(const TmplDev &td, const ItemDev 
     const uint32_t T0 = td.t0 + TA / 2 - td.t_min;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    auto clamp_j = [&](int j) { return min(max(j, 1), N); };
     int jb = 0;  // entry in LDS slot 0
     if (LDS) {
         const uint32_t Tr = T0 + (uint32_t)row0 * dt0;
@@ -1396,8 +1373,10 @@ __device__ __forceinline__ void rect_step_item(const TmplDev &td, const ItemDev 
         const uint32_t xf = td.tau + (uint32_t)col0 * dtau;
         const uint32_t xl = td.tau + (uint32_t)min(col0 + td.tile - 1, N_tau - 1) * dtau;
         uint32_t rem;
-        jb = clamp_j((int)(div_TA(Tr, td, rem) + div_TA(xf, td, rem)));
-        const int nw = (clamp_j((int)(div_TA(Tl, td, rem) + div_TA(xl, td, rem) + 1)) - jb + 1) * NC;
+        const StepRange range = step_range(Tr, xf, Tl, xl, N,
+                                           [&](uint32_t x) { return div_TA(x, td, rem); });
+        jb = range.first;
+        const int nw = range.count * NC;
         const double *__restrict__ src = P + (int64_t)jb * NC;
         for (int k0 = threadIdx.x; k0 < nw; k0 += 8 * WG) {
             double v[8];
