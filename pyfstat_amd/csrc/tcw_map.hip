@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -1016,7 +1017,11 @@ static_assert(rect_item_lds(16, 1) - 16 * 2 * sizeof(float) >= sizeof(FinShared)
 // shared test only when they are a few bins long, i.e. in a template's first
 // column block, whose items test cell by cell from the start.  Per 16 cells: 8
 // minima and ~8 FP64 operations in place of 80.
+// Determinants outside float's range: min(D) starts at FLT_MAX, below what was
+// rounded to infinity, and GUARD_ROUND is Q times half the spacing of the floats
+// next to zero, which is what rounding may have added to a D there.
 constexpr double GUARD_SLACK = 1.0 + 1e-5;
+constexpr double GUARD_ROUND = QCOND * 0.5 * 1.401298464324817e-45;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -1114,7 +1119,9 @@ __device__ __forceinline__ int rect_first_max(float &best, int bstep, const Tmpl
             return (row0 + rl0 + r) * N_tau + col0 + l * C + __builtin_amdgcn_readlane(first, l);
         }
     }
-    return 0x7fffffff;
+    // (not found again, should the two condition tests ever disagree: a cell of
+    // the step, inside the map)
+    return (row0 + rl0) * N_tau + col0 + __builtin_ctzll(held) * C;
 }
 
 // One work item.  FIRST: the template's first column block (cell-by-cell
@@ -1177,7 +1184,7 @@ __device__ __forceinline__ void rect_fast_item(const TmplDev &td, const ItemDev 
             for (int k = 0; k < NC; k++) Pi[r][k] = P[(int64_t)i0[r] * NC + k];
         }
         typename RowCells<C>::type F[4];
-        float Dmin = INFINITY;
+        float Dmin = FLT_MAX;
         double Tall = 0.0;
         // Diagonal by diagonal: its entry meets the starts of up to four rows.
         // The starts sit in scalar registers, so a lane holds one diagonal's 7
@@ -1217,7 +1224,8 @@ __device__ __forceinline__ void rect_fast_item(const TmplDev &td, const ItemDev 
             }
         }
         if constexpr (!FIRST) {
-            const bool ok_all = Tall * Tall * GUARD_SLACK < QCOND * (double)Dmin;
+            const bool ok_all =
+                fma(Tall * GUARD_SLACK, Tall, GUARD_ROUND) < QCOND * (double)Dmin;
             if (no_bound || !__all(ok_all)) {  // wave-uniform: cell by cell
                 // (an address the compiler cannot match with the one above: it
                 // would keep the differences of all cells alive, and spill)
