@@ -17,14 +17,16 @@ N_TAUS = (1, 64, 256, 257, 300, 385, 512)
 def _batch(kind, n_t0, generic):
     from pyfstat_amd.batched import BatchedTransientMaps
 
-    ts, cols = _atoms(700, 7, "plain")
+    # (tiny: all windows past the first column block end with the data, and a
+    # wave's lanes agree)
+    ts, cols = _atoms(250 if kind == "tiny" else 700, 7, "plain")
     cols = cols.astype(np.float64)
     cols[:3] *= 1e24  # determinants of 1e48 and more
     if kind == "degenerate":  # condition numbers near 4e5: F = 2 in every cell
         cols[1] = cols[0]
         cols[2] = cols[0] * (1.0 - 5e-6)
     elif kind == "tiny":  # determinants of a few units of the last float32 place there is
-        cols[:3] *= 6e-47
+        cols[:3] *= 2e-46
         cols[1] = cols[0]
         cols[2] = cols[0] * np.sqrt(1.0 - 4.0 / (1.0003 * 10001.0**2 / 1e4))
     elif kind == "some":  # until some way into the data
