@@ -195,6 +195,11 @@ int64_t tcw_plan_scratch_bytes(const tcw_plan *p);
  * counterpart in the reference. */
 int tcw_plan_items(const tcw_plan *p, int64_t *items);
 
+/* Templates per map kernel (templates[0..5]: rect regular grid, rect steps, rect
+ * per cell, exp on the atom grid, exp sliding sum, exp per cell); modes 1 and 2
+ * of the rows hold two kernels each.  No counterpart in the reference. */
+int tcw_plan_kernels(const tcw_plan *p, int64_t *templates);
+
 /* Run a planned batch on device-resident atoms.  ts/cols follow the plan's
  * segment layout (cols is [TCW_NCOL][col_stride]); F_out is the concatenated
  * float32 output (F_off layout); stats_dev is a device array of T tcw_stats.

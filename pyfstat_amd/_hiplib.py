@@ -32,6 +32,15 @@ MODE_RECT_GENERIC = 1
 MODE_EXP_DIRECT = 2
 MODE_EXP_FAST = 3
 MODE_COUNT = 4
+# the map kernels in the order of tcw_plan_kernels, and the mode of each
+KERNEL_MODES = {
+    "rect_fast": MODE_RECT_FAST,
+    "rect_step": MODE_RECT_GENERIC,
+    "rect_generic": MODE_RECT_GENERIC,
+    "exp_fast": MODE_EXP_FAST,
+    "exp_walk": MODE_EXP_DIRECT,
+    "exp_direct": MODE_EXP_DIRECT,
+}
 
 EXPORTED_SYMBOLS = (
     "tcw_version",
@@ -48,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "tcw_batch_plan_rows",
     "tcw_plan_scratch_bytes",
     "tcw_plan_items",
+    "tcw_plan_kernels",
     "tcw_batch_run",
     "tcw_batch_run_timed",
     "tcw_plan_destroy",
@@ -209,6 +219,8 @@ def load():
     lib.tcw_plan_scratch_bytes.argtypes = [vp]
     lib.tcw_plan_items.restype = ctypes.c_int
     lib.tcw_plan_items.argtypes = [vp, vp]
+    lib.tcw_plan_kernels.restype = ctypes.c_int
+    lib.tcw_plan_kernels.argtypes = [vp, vp]
     lib.tcw_batch_run.restype = ctypes.c_int
     lib.tcw_batch_run.argtypes = [vp, vp, vp, vp, ctypes.c_int64, vp, vp, ctypes.c_int, vp]
     lib.tcw_batch_run_timed.restype = ctypes.c_int

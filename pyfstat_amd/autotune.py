@@ -1,5 +1,6 @@
 """Autotuner for the batched map kernels: rows (t0) per work item per kernel
-mode, chosen by timing the step's kernels on the caller's own batch.
+mode, chosen by timing the step's kernels on the caller's own batch; the
+library's own choice is one of the candidates.
 
 A work item is up to ``rows`` t0 rows x 256 tau columns of one template.  More
 rows amortise the item's set-up (diagonal staging for the rect kernel, the
@@ -8,8 +9,8 @@ more items to spread over the 256 CUs and a smaller LDS footprint.  The best
 value depends on the batch's shapes, so it is measured: each candidate value
 is planned (``BatchedTransientMaps.set_rows`` + ``replan``, which pass it to
 ``tcw_batch_plan_rows``) and the step's kernels timed with HIP events
-(``run_timed``); the fastest is kept and cached per (device, mode, shape
-class).  The setting belongs to the tuned batch's plan: other batches and
+(``run_timed``); the fastest is kept and cached per (device, mode, kernels, shape
+and step class).  The setting belongs to the tuned batch's plan: other batches and
 single-map calls keep the library's own choice.
 
 The reference has no counterpart (its kernels use fixed 1-D launches,
@@ -24,12 +25,15 @@ import numpy as np
 
 from . import _hiplib
 
+# 0 is the library's choice, which takes other values than these for some
+# batches; the rest spans what it chooses between
 CANDIDATES = {
-    _hiplib.MODE_RECT_FAST: (16, 32, 64, 128, 192, 256, 384),
-    _hiplib.MODE_RECT_GENERIC: (16, 32, 64),
-    _hiplib.MODE_EXP_DIRECT: (16, 32, 64),
-    _hiplib.MODE_EXP_FAST: (64, 128, 256, 512, 1024),
+    _hiplib.MODE_RECT_FAST: (0, 16, 32, 64, 128, 192, 256, 384),
+    _hiplib.MODE_RECT_GENERIC: (0, 16, 32, 64, 128),
+    _hiplib.MODE_EXP_DIRECT: (0, 16, 32, 64, 128, 256),
+    _hiplib.MODE_EXP_FAST: (0, 16, 32, 64, 128, 256, 512, 1024),
 }
+
 
 def cache_path():
     env = os.environ.get("PYFSTAT_AMD_TUNE_CACHE")
@@ -64,13 +68,18 @@ def _bucket(x):
 
 
 def shape_class(b, mode, device_name=""):
-    """Cache key: device, mode, and log2 buckets of the template count and of
-    the templates' median t0 rows and tau columns (none of which depends on
-    the rows-per-item setting being tuned)."""
+    """Cache key: device, mode, the mode's kernels that the batch's templates
+    take, and log2 buckets of the template count and of the templates' median t0
+    rows, tau columns and steps in atoms (none of which depends on the
+    rows-per-item setting being tuned)."""
     shapes = np.array([b._shape(t) for t in range(b.T)], dtype=np.int64)
+    steps = np.array([(w.dt0, w.dtau) for w in b.windows], dtype=np.float64) / b.TAtom
+    templates = b.templates_per_kernel()
+    kernels = "+".join(k for k, m in _hiplib.KERNEL_MODES.items() if m == mode and templates[k])
     version = _hiplib.load().tcw_version().decode(errors="replace")
-    return (f"{version}|{device_name}|mode{mode}|T{_bucket(b.T)}"
-            f"|rows{_bucket(np.median(shapes[:, 0]))}|cols{_bucket(np.median(shapes[:, 1]))}")
+    return (f"{version}|{device_name}|mode{mode}|{kernels}|T{_bucket(b.T)}"
+            f"|rows{_bucket(np.median(shapes[:, 0]))}|cols{_bucket(np.median(shapes[:, 1]))}"
+            f"|dt0{_bucket(np.median(steps[:, 0]))}|dtau{_bucket(np.median(steps[:, 1]))}")
 
 
 def set_rows(b, mode, rows):

@@ -147,6 +147,12 @@ class BatchedTransientMaps:
         _hiplib.check(self.lib.tcw_plan_items(self.plan, out.ctypes.data), "tcw_plan_items")
         return out
 
+    def templates_per_kernel(self):
+        """Templates of each map kernel, by name."""
+        out = np.zeros(len(_hiplib.KERNEL_MODES), dtype=np.int64)
+        _hiplib.check(self.lib.tcw_plan_kernels(self.plan, out.ctypes.data), "tcw_plan_kernels")
+        return dict(zip(_hiplib.KERNEL_MODES, out.tolist()))
+
     # ------------------------------------------------------------------
     @classmethod
     def from_device_atoms(cls, atoms, windows, **kw):

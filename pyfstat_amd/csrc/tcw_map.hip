@@ -4101,6 +4101,19 @@ int tcw_plan_items(const tcw_plan *p, int64_t *items) {
     return TCW_OK;
 }
 
+int tcw_plan_kernels(const tcw_plan *p, int64_t *templates) {
+    if (!p || !templates) return fail(TCW_ERR_INVALID, "tcw_plan_kernels: null argument");
+    int64_t n[MODE_COUNT] = {0, 0, 0, 0};
+    for (const TmplDev &td : p->tmpl) n[td.mode]++;
+    templates[0] = n[MODE_RECT_FAST];
+    templates[1] = p->step_tmpls;
+    templates[2] = p->generic_tmpls;
+    templates[3] = n[MODE_EXP_FAST];
+    templates[4] = p->walk_tmpls;
+    templates[5] = p->direct_tmpls;
+    return TCW_OK;
+}
+
 int tcw_batch_run(tcw_handle *h, tcw_plan *p, const uint32_t *ts, const float *cols,
                   int64_t col_stride, float *F_out, tcw_stats *stats_dev, int use_graph,
                   void *stream) {

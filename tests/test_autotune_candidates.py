@@ -4,17 +4,21 @@ import numpy as np
 import pytest
 
 from pyfstat_amd import _hiplib, autotune
+from pyfstat_amd.atoms import TRANSIENT_RECTANGULAR, transientWindowRange_t
 
 KERNELS = ("rect_fast", "rect_step", "rect_generic", "exp_direct", "exp_walk", "exp_fast")
 
 
 class FakeBatch:
     T = 8
+    TAtom = 1800
 
-    def __init__(self, kernels, best=0):
+    def __init__(self, kernels, dt0=2700, dtau=2700):
         self.kernels = kernels  # templates of each kernel
-        self.best = best
         self.rows = {}
+        self.windows = [transientWindowRange_t(type=TRANSIENT_RECTANGULAR, t0=0, t0Band=499 * dt0,
+                                               dt0=dt0, tau=3600, tauBand=499 * dtau, dtau=dtau)
+                        ] * self.T
 
     def _shape(self, t):
         return (500, 500)
@@ -55,5 +59,8 @@ def test_a_value_of_one_kernel_is_not_taken_for_another(mode, one, two):
     keys = [autotune.shape_class(FakeBatch(k), mode, "dev")
             for k in ({one: 8}, {two: 8}, {one: 4, two: 4})]
     assert len(set(keys)) == 3
+    # nor one of short steps for long ones
+    keys.append(autotune.shape_class(FakeBatch({one: 8}, dtau=20 * 1800), mode, "dev"))
+    assert keys[3] not in keys[:3]
     # the other modes' kernels do not matter
     assert keys[0] == autotune.shape_class(FakeBatch({one: 8, "rect_fast": 3}), mode, "dev")
