@@ -27,6 +27,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -3248,6 +3249,10 @@ struct HostStage {
         dev.release();
     }
 };
+// A batch plan's descriptors go in one pageable copy up to this size (planning 256
+// maps of 48 x 48 to 240 x 240 cells: seven allocations and copies 89 us, one of
+// each 50); beyond it the bytes count, and gathering them would double those.
+constexpr size_t PACKED_TABLES_MAX = 256u << 10;
 constexpr size_t stage_align(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 struct tcw_plan {
@@ -3294,6 +3299,7 @@ struct tcw_plan {
     const float *host_cols = nullptr;   // [7][n_host_atoms]
     int64_t n_host_atoms = 0;
     DevBuf d_ts, d_cols;                // views of the stage's device buffer
+    DevBuf d_tables;  // a batch plan's small descriptors: views of this one
     // when set, device buffers are views into this memory (tcw_map_noalloc)
     char *arena = nullptr;
     size_t arena_bytes = 0;
@@ -3346,6 +3352,7 @@ struct tcw_plan {
         d_tmpl_list.release();
         d_ts.release();
         d_cols.release();
+        d_tables.release();
     }
 };
 
@@ -3646,10 +3653,15 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
     p.rowpart_n += N_t0 * (int64_t)td.n_colblk;
     td.colpart_off = p.colpart_n;
     p.colpart_n += N_tau * (int64_t)td.n_rowblk;
-    // items of a template are contiguous in item-id space; item_begin fixed below
+    // items of a template are contiguous in item-id space; item_begin counts from
+    // the mode's first item until plan_finish
+    std::vector<ItemDev> &items = items_by_mode[mode];
+    td.item_begin = (int64_t)items.size();
+    items.resize(items.size() + (size_t)td.n_rowblk * td.n_colblk);
+    ItemDev *it = items.data() + td.item_begin;
     for (uint32_t rbk = 0; rbk < td.n_rowblk; rbk++)
         for (uint32_t cbk = 0; cbk < td.n_colblk; cbk++)
-            items_by_mode[mode].push_back(ItemDev{(int32_t)t, (int32_t)rbk, (int32_t)cbk, 0});
+            *it++ = ItemDev{(int32_t)t, (int32_t)rbk, (int32_t)cbk, 0};
     if (mode == MODE_RECT_GENERIC && td.walk) {
         p.max_lds_step = std::max(
             p.max_lds_step,
@@ -3700,14 +3712,13 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
     p.items.clear();
     for (int md = 0; md < MODE_COUNT; md++) {
         p.mode_begin[md] = (int64_t)p.items.size();
-        for (size_t k = 0; k < items_by_mode[md].size(); k++) {
-            const ItemDev &it = items_by_mode[md][k];
-            TmplDev &td = p.tmpl[it.t];
-            if (it.rb == 0 && it.cb == 0) td.item_begin = (int64_t)p.items.size();
-            p.items.push_back(it);
-        }
+        if (p.items.empty())  // most batches hold one mode
+            p.items.swap(items_by_mode[md]);
+        else
+            p.items.insert(p.items.end(), items_by_mode[md].begin(), items_by_mode[md].end());
     }
     p.mode_begin[MODE_COUNT] = (int64_t)p.items.size();
+    for (TmplDev &td : p.tmpl) td.item_begin += p.mode_begin[td.mode];
     p.tmpl_list = p.exp_tmpls;
     for (auto &r : p.rect_tmpls) {
         // the longest templates first: the last workgroups to start are short
@@ -3738,6 +3749,7 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
     size_t staged = 0;
     for (const Up &u : ups) staged += stage_align(std::max<size_t>(u.bytes, 1));
     const bool one_copy = p.stage && async && staged <= HOST_STAGE_MAX;
+    const bool packed = !p.arena && !async && staged <= PACKED_TABLES_MAX;
     int rc = TCW_OK;
     if (one_copy) {
         if ((rc = p.stage->ensure(staged))) return rc;
@@ -3749,6 +3761,17 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
             off += a;
         }
         TCW_HIP_TRY(hipMemcpyAsync(p.stage->dev.p, p.stage->pin, staged, hipMemcpyHostToDevice, st));
+    } else if (packed) {
+        if ((rc = p.d_tables.ensure(staged))) return rc;
+        const std::unique_ptr<char[]> host(new char[staged]);
+        size_t off = 0;
+        for (const Up &u : ups) {
+            const size_t a = stage_align(std::max<size_t>(u.bytes, 1));
+            if (u.bytes) std::memcpy(host.get() + off, u.src, u.bytes);
+            u.buf->set_view((char *)p.d_tables.p + off, a);
+            off += a;
+        }
+        TCW_HIP_TRY(hipMemcpy(p.d_tables.p, host.get(), staged, hipMemcpyHostToDevice));
     } else {
         for (const Up &u : ups)  // views of an earlier call
             if (u.buf->view) u.buf->release();
@@ -3773,7 +3796,7 @@ int plan_finish(tcw_plan &p, std::vector<ItemDev> (&items_by_mode)[MODE_COUNT],
         });
         if (rc) return rc;
     }
-    if (one_copy) return TCW_OK;
+    if (one_copy || packed) return TCW_OK;
     for (const Up &u : ups) {
         if (u.bytes == 0) continue;
         if ((rc = u.buf->ensure(u.bytes))) return rc;
