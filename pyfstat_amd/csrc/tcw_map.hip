@@ -3533,10 +3533,15 @@ int plan_template(tcw_plan &p, int64_t t, const tcw_window &win_in, uint32_t N,
         // offsets within their four rows)
         td.walk = !(p.flags & TCW_FLAG_GENERIC) && x_lo >= t_min && x_hi < (1ull << 32) &&
                   N_tau <= (int64_t)1 << 20;
-        if (td.walk && regular) {
+        // the kernel's start indices of a wave's four rows, up to three past the
+        // map, are 32 bits wide
+        const uint64_t q0 = ((uint64_t)w.t0 - t_min + half) / TAtom;
+        const bool starts_fit =
+            q0 + (uint64_t)(w.dt0 / TAtom) * (uint64_t)(N_t0 + 2) <= 0x7fffffffu;
+        if (td.walk && regular && starts_fit) {
             mode = MODE_RECT_FAST;
             td.a = (int32_t)(w.dt0 / TAtom);
-            td.q0 = (int32_t)(((uint64_t)w.t0 - t_min + half) / TAtom);
+            td.q0 = (int32_t)q0;
             td.q00 = (int32_t)(((uint64_t)w.t0 + w.tau - t_min + half) / TAtom);
         } else if (p.compact || (w.dt0 < TAtom && N_t0 > 1) || (w.dtau < TAtom && N_tau > 1)) {
             td.walk = 0;  // (steps of part of an atom repeat rows or columns, as above)
