@@ -150,7 +150,12 @@ class MergedAtoms:
 
     def merge(self, cols_raw):
         """Merged float32 [7, total_bins] of raw atoms [7, n_atoms]
-        (differentiable: the backward gathers each atom's bin gradient)."""
+        (differentiable: the backward gathers each atom's bin gradient).
+
+        Queued on the current stream without waiting for it, as torch's own
+        operations are: another stream that reads the result or ``atom_bin`` has
+        to wait for this one first (``stream.wait_stream``), and
+        ``cols_raw`` has to stay unchanged until the merge has run."""
         return _MergeFunction.apply(cols_raw, self)
 
     def _merge_forward(self, cols_raw):
