@@ -1189,7 +1189,7 @@ __device__ __forceinline__ void rect_fast_item(const TmplDev &td, const ItemDev 
         double Tall = 0.0;
         // Diagonal by diagonal: its entry meets the starts of up to four rows.
         // The starts sit in scalar registers, so a lane holds one diagonal's 7
-        // sums at a time (79 VGPRs, six waves a SIMD; row by row it holds C of
+        // sums at a time (87 VGPRs, five waves a SIMD; row by row it holds C of
         // them: 96-104, four or five waves).
 #pragma unroll
         for (int x = 0; x < C + 3; x++) {
@@ -1317,7 +1317,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 }
 
 // ----------------------------------------------------------------------------
-// rectangular window, any steps without wrap-around
+// rectangular window, steps of an atom or more, without wrap-around
 // ----------------------------------------------------------------------------
 //
 // Row m starts at t0 + m dt0 + TAtom/2 - t_min = TAtom q + phi, column n lasts
@@ -1333,7 +1333,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 //
 // Bound: VALU issue and latency together (63 instructions a cell, 24 of them
 // FP64; 69% of the cycles issue, at ~3 waves a SIMD).  128 templates of 1000 to
-// 4000 bins, steps of 2 and 3 bins, 37e6 cells: maps 192 us with the generic
+// 4000 bins, steps of 2 and 3 bins, 37e6 cells: maps 195 us with the generic
 // kernel (an integer division and an uncoalesced 56-byte read a cell), 90 us
 // so, 210 us with these indices but the table read in place.
 // Rows per item at most and items aimed at, untuned (the maps above: 64 rows
@@ -1600,7 +1600,8 @@ __global__ __launch_bounds__(WG) void rect_generic_kernel(
                 colpart, sh_rowM, sh_rowS, sh_fin, [](int ln, int c) { return c * 64 + ln; });
 }
 
-// Exponential window off the atom grid: the window sum slides with any steps.
+// Exponential window off the atom grid: the window sum slides with any starts an
+// atom or more apart, and any durations.
 //
 // Row m starts at T = t0 + m dt0 - t_min = TAtom q + phi, column n lasts 3 tau =
 // TAtom Q + R.  The cell's atoms (exp.cu:39-102) are lo(m) .. hi(m, n),
